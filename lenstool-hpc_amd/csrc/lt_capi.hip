@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "lenstool_hip/lt_capi.h"
+#include "lt_far.h"
 #include "lt_internal.h"
 #include "lt_kernels.h"
 
@@ -129,13 +130,15 @@ int default_px(int kind, int precision, int nhalos, long long npix)
 struct DevModel {
     HaloRec* recs = nullptr;
     HaloRec32* recs32 = nullptr;
+    FarRec* frecs = nullptr;
     Run* runs = nullptr;
     int nruns = 0;
+    FarStats far;  // of the model (of a batch's first sample) as it was created
 };
 
-// Launch the kernel that produces map `kind` from a device model.
+// Launch the kernel that produces map `kind` from a device model. `whole`: the grid that g is rows of.
 int launch_map(const DevModel& m, int kind, int mode, double* const outs[5], double r, double mult,
-               const GridDesc& g, int precision, int px, hipStream_t s, int nhalos)
+               const GridDesc& g, const GridDesc& whole, int precision, int px, hipStream_t s, int nhalos)
 {
     OutDesc o{};
     o.p0 = outs[0];
@@ -156,6 +159,19 @@ int launch_map(const DevModel& m, int kind, int mode, double* const outs[5], dou
     if (precision != LT_PREC_FP64 && precision != LT_PREC_FP32C)
         return fail(LT_ERR_INVALID, "precision must be LT_PREC_FP64 or LT_PREC_FP32C");
     hipError_t e;
+    // Large grids: the halo sums by tile expansions (lt_far.hip), in FP64 whatever precision is asked for
+    // (both cost less than the FP32C direct sum there, and the result is the FP64 map).
+    const FarShape shape = px == LT_PX_HALO_LANES ? FarShape::Direct : far_shape(m.far, kind, precision, whole, nullptr);
+    const bool tiled = shape != FarShape::Direct;
+    if (tiled) {
+        if (kind == LT_MAP_AMPLI && mode == 5) {  // kappa: the Hessian's trace alone
+            o.kind = LT_MAP_MASS;
+            o.mult = 1.0;
+        }
+        e = launch_far(m.recs, m.frecs, m.runs, m.nruns, nhalos, g, o, shape, s);
+        if (e != hipSuccess) return hip_fail(e, "kernel launch");
+        return LT_OK;
+    }
     switch (kind) {
     case LT_MAP_GRADIENT:
     case LT_MAP_DPL:
@@ -245,19 +261,27 @@ int host_map(int kind, int mode, Use use, double* const host_out[5], const lt_gr
     const size_t rec_bytes = recs.size() * sizeof(HaloRec);
     const size_t rec32_bytes = recs32.size() * sizeof(HaloRec32);
     const size_t run_bytes = runs.size() * sizeof(Run);
-    const size_t halo_need = rec_bytes + rec32_bytes + run_bytes + 256;
-    if ((st = ensure(&S.halos, &S.halos_bytes, halo_need))) return st;
+    const size_t far_bytes = recs.size() * sizeof(FarRec);
+    const size_t off_runs = ((rec_bytes + rec32_bytes + far_bytes + 63) / 64) * 64, halo_need = off_runs + run_bytes;
+    if ((st = ensure(&S.halos, &S.halos_bytes, std::max<size_t>(halo_need, 1)))) return st;
     if ((st = ensure(&S.planes, &S.planes_bytes, n * np * sizeof(double)))) return st;
 
-    char* base = (char*)S.halos;
+    // one image of the model and one copy of it
+    std::vector<char> image(halo_need);
     DevModel m;
+    if (rec_bytes) {
+        std::memcpy(image.data(), recs.data(), rec_bytes);
+        std::memcpy(image.data() + rec_bytes, recs32.data(), rec32_bytes);
+        far_records(recs.data(), (int)recs.size(), (FarRec*)(image.data() + rec_bytes + rec32_bytes));
+        std::memcpy(image.data() + off_runs, runs.data(), run_bytes);
+        HIP_TRY(hipMemcpyAsync(S.halos, image.data(), halo_need, hipMemcpyHostToDevice, S.stream));
+    }
+    char* base = (char*)S.halos;
     m.recs = (HaloRec*)base;
     m.recs32 = (HaloRec32*)(base + rec_bytes);
-    m.runs = (Run*)(base + ((rec_bytes + rec32_bytes + 63) / 64) * 64);
+    m.frecs = (FarRec*)(base + rec_bytes + rec32_bytes);
+    m.runs = (Run*)(base + off_runs);
     m.nruns = (int)runs.size();
-    if (rec_bytes) HIP_TRY(hipMemcpyAsync(m.recs, recs.data(), rec_bytes, hipMemcpyHostToDevice, S.stream));
-    if (rec32_bytes) HIP_TRY(hipMemcpyAsync(m.recs32, recs32.data(), rec32_bytes, hipMemcpyHostToDevice, S.stream));
-    if (run_bytes) HIP_TRY(hipMemcpyAsync(m.runs, runs.data(), run_bytes, hipMemcpyHostToDevice, S.stream));
 
     double* dev_out[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     for (int k = 0; k < np; ++k)
@@ -273,7 +297,8 @@ int host_map(int kind, int mode, Use use, double* const host_out[5], const lt_gr
     g.jstart = jstart;
     g.pitch = nx;
     g.nsamples = 1;
-    if ((st = launch_map(m, kind, mode, dev_out, r, mult, g, precision, 0, S.stream, nhalos))) return st;
+    m.far = far_stats(recs.data(), nhalos, runs);
+    if ((st = launch_map(m, kind, mode, dev_out, r, mult, g, g, precision, 0, S.stream, nhalos))) return st;
     for (int k = 0; k < np; ++k)
         if (host_out[k])
             HIP_TRY(hipMemcpyAsync(host_out[k], dev_out[k], n * sizeof(double), hipMemcpyDeviceToHost, S.stream));
@@ -563,7 +588,7 @@ struct lt_model_s {
     DevModel dm;
     size_t bytes = 0;
     size_t rec_bytes = 0, rec32_bytes = 0;  // all samples
-    void* base = nullptr;                   // device: records [S*H], fp32 records [S*H], runs
+    void* base = nullptr;                   // device: records [S*H], fp32 records [S*H], far records [S*H], runs
     size_t off_runs = 0;                    // offset of the runs in `base` and in `staging`
     void* staging = nullptr;                // pinned host image of base (records and runs)
     hipEvent_t staged = nullptr;            // completes when the last upload has read `staging`
@@ -622,6 +647,7 @@ static int stage_samples(lt_model_s* m, const lt_potential_soa* lenses, int nsam
             std::memcpy(st + (size_t)s * H * sizeof(HaloRec), recs.data(), (size_t)H * sizeof(HaloRec));
             std::memcpy(st + m->rec_bytes + (size_t)s * H * sizeof(HaloRec32), recs32.data(),
                         (size_t)H * sizeof(HaloRec32));
+            far_records(recs.data(), H, (FarRec*)(st + m->rec_bytes + m->rec32_bytes) + (size_t)s * H);
         }
     }
     if (!batch_runs.empty()) std::memcpy(st + m->off_runs, batch_runs.data(), batch_runs.size() * sizeof(Run));
@@ -676,10 +702,12 @@ int lt_model_create_batch(lt_model* out, const lt_potential_soa* lenses, int nsa
     m->nhalos = nhalos;
     m->nsamples = nsamples;
     m->runs_host = runs;
+    m->dm.far = far_stats(recs.data(), nhalos, runs);  // kept when samples change: only speed depends on it
     for (int i = 0; i < nhalos; ++i) m->types.push_back(lenses[0].type[i]);
     m->rec_bytes = (size_t)nsamples * nhalos * sizeof(HaloRec);
     m->rec32_bytes = (size_t)nsamples * nhalos * sizeof(HaloRec32);
-    const size_t off_runs = ((m->rec_bytes + m->rec32_bytes + 63) / 64) * 64;
+    const size_t far_bytes = (size_t)nsamples * nhalos * sizeof(FarRec);
+    const size_t off_runs = ((m->rec_bytes + m->rec32_bytes + far_bytes + 63) / 64) * 64;
     m->off_runs = off_runs;
     m->bytes = off_runs + runs.size() * sizeof(Run) + 64;
     hipError_t e = hipMalloc(&m->base, m->bytes);
@@ -693,6 +721,7 @@ int lt_model_create_batch(lt_model* out, const lt_potential_soa* lenses, int nsa
     char* b = (char*)m->base;
     m->dm.recs = (HaloRec*)b;
     m->dm.recs32 = (HaloRec32*)(b + m->rec_bytes);
+    m->dm.frecs = (FarRec*)(b + m->rec_bytes + m->rec32_bytes);
     m->dm.runs = (Run*)(b + off_runs);
     m->dm.nruns = (int)runs.size();
     if ((st = stage_samples(m, lenses, nsamples))) {
@@ -760,23 +789,10 @@ int lt_model_bytes(lt_model m, long long* bytes)
     return LT_OK;
 }
 
-int lt_map_device(lt_model m, int kind, int mode, double* out0, double* out1, double* out2, double* out3, double* out4,
-                  double r, double mult, const lt_grid_desc* grid, int precision, int px, void* stream)
+}  // extern "C"
+
+static GridDesc grid_desc(const lt_model_s* m, const lt_grid_desc* grid)
 {
-    if (!m) return fail(LT_ERR_NOT_FOUND, "model is NULL");
-    if (!grid) return fail(LT_ERR_INVALID, "grid is NULL");
-    int st = check_kind_mode(kind, mode);
-    if (st) return st;
-    Use need = kind == LT_MAP_DPL || kind == LT_MAP_GRADIENT ? Use::Gradient
-               : kind == LT_MAP_POT ? Use::Potential
-               : kind == LT_MAP_MASS ? Use::Kmap : Use::Hessian;
-    if (need != m->use && !(need == Use::Hessian && m->use == Use::Kmap))
-        return fail(LT_ERR_INVALID, "model was created for another kind of map");
-    if (grid->nx <= 0 || grid->ny <= 0 || grid->pitch < grid->nx) return fail(LT_ERR_INVALID, "bad grid");
-    double* outs[5] = {out0, out1, out2, out3, out4};
-    if ((kind == LT_MAP_GRADIENT || kind == LT_MAP_DPL) && (!out0 || !out1))
-        return fail(LT_ERR_INVALID, "gradient output needs two planes");
-    if (kind != LT_MAP_HESSIAN && kind != LT_MAP_FIELDS && !out0) return fail(LT_ERR_INVALID, "out0 is NULL");
     GridDesc g{};
     g.xmin = grid->xmin;
     g.ymin = grid->ymin;
@@ -790,8 +806,44 @@ int lt_map_device(lt_model m, int kind, int mode, double* out0, double* out1, do
     g.nsamples = m->nsamples;
     g.halo_stride = m->nhalos;
     g.plane_stride = grid->pitch * (long long)grid->ny;
+    return g;
+}
+
+double lt::map_rows_cost(lt_model m, int kind, int precision, const lt_grid_desc* whole, bool* tiled)
+{
+    double cost = 0;
+    *tiled = far_shape(m->dm.far, kind, precision, grid_desc(m, whole), &cost) != FarShape::Direct;
+    return cost;
+}
+
+int lt::map_device_rows(lt_model m, int kind, int mode, double* const outs[5], double r, double mult,
+                        const lt_grid_desc* grid, const lt_grid_desc* whole, int precision, int px, void* stream)
+{
+    if (!m) return fail(LT_ERR_NOT_FOUND, "model is NULL");
+    if (!grid) return fail(LT_ERR_INVALID, "grid is NULL");
+    int st = check_kind_mode(kind, mode);
+    if (st) return st;
+    Use need = kind == LT_MAP_DPL || kind == LT_MAP_GRADIENT ? Use::Gradient
+               : kind == LT_MAP_POT ? Use::Potential
+               : kind == LT_MAP_MASS ? Use::Kmap : Use::Hessian;
+    if (need != m->use && !(need == Use::Hessian && m->use == Use::Kmap))
+        return fail(LT_ERR_INVALID, "model was created for another kind of map");
+    if (grid->nx <= 0 || grid->ny <= 0 || grid->pitch < grid->nx) return fail(LT_ERR_INVALID, "bad grid");
+    if ((kind == LT_MAP_GRADIENT || kind == LT_MAP_DPL) && (!outs[0] || !outs[1]))
+        return fail(LT_ERR_INVALID, "gradient output needs two planes");
+    if (kind != LT_MAP_HESSIAN && kind != LT_MAP_FIELDS && !outs[0]) return fail(LT_ERR_INVALID, "out0 is NULL");
     HIP_TRY(hipSetDevice(m->device));
-    return launch_map(m->dm, kind, mode, outs, r, mult, g, precision, px, (hipStream_t)stream, m->nhalos);
+    return launch_map(m->dm, kind, mode, outs, r, mult, grid_desc(m, grid), grid_desc(m, whole), precision, px,
+                      (hipStream_t)stream, m->nhalos);
+}
+
+extern "C" {
+
+int lt_map_device(lt_model m, int kind, int mode, double* out0, double* out1, double* out2, double* out3, double* out4,
+                  double r, double mult, const lt_grid_desc* grid, int precision, int px, void* stream)
+{
+    double* outs[5] = {out0, out1, out2, out3, out4};
+    return map_device_rows(m, kind, mode, outs, r, mult, grid, grid, precision, px, stream);
 }
 
 int lt_scale_device(double* x, double s, long long n, void* stream)

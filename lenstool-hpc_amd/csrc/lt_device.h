@@ -23,14 +23,14 @@ namespace lt {
 struct alignas(64) HaloRec {
     double xh, yh, cs, sn;          // 0..3
     double hc2, hs2;                // 4, 5
-    double kx, ky;                  // 6, 7   1/(1+e)^2, 1/(1-e)^2
-    double e2;                      // 8      2 sqrt(e)
+    double kx, ky;                  // 6, 7   1/(1+e)^2, 1/(1-e)^2; SIS: kx = max(sa, sb)
+    double far0;                    // 8      far test of lt_far.hip: the smallest cx1^2 r^2 of the halo's radii
     double cx1, gki, gkv;           // 9..11  (1-e)/(1+e); gradient: 2 sqrt(e) a^2, 2 sqrt(e) a b (a, b = 1/(1 +- e))
     double ra2, rb2;                // 12, 13 rcore^2, rcut^2
     double rca, rcb;                // 14, 15 cx1 rcore, cx1 rcut
     double ampg;                    // 16     gradient amplitude
     double amph;                    // 17     Hessian amplitude
-    double csx, snx, csy, sny;      // 18..21 cx1 a (cs, sn), cx1 b (cs, sn): the scaled Hessian frame
+    double csx, snx, csy, sny;      // 18..21 cx1 a (cs, sn), cx1 b (cs, sn): the scaled Hessian frame; SIS: sqrt(sa) (cs, sn), sqrt(sb) (cs, sn)
     double ra2c, rb2c;              // 22, 23 cx1^2 rcore^2, cx1^2 rcut^2
     union {                         // 24..28 by type:
         struct {

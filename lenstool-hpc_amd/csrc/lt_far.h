@@ -1,0 +1,49 @@
+// lt_far.h -- tile expansions of the halo sums (lt_far.hip): launcher and the rule that picks them.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <vector>
+
+#include "lt_device.h"
+#include "lt_kernels.h"
+
+namespace lt {
+
+constexpr int kFarMaxHalos = 2048;   // halos of a model (the sets live in LDS)
+constexpr int kFarMaxRuns = 16;      // runs of a model (every run is walked for every 16 x 16 block)
+
+// What the far test reads of a halo (48 bytes, packed so that a wavefront's 64 are contiguous): its centre and the
+// scaled frame in which a square of half side h is far when X^2 + Y^2 + f >= 36 h^2.
+struct alignas(16) FarRec {
+    double xh, yh;
+    float a, b, c, d, f;
+    float pad[3];
+};
+static_assert(sizeof(FarRec) == 48, "far record is 48 bytes");
+
+void far_records(const HaloRec* recs, int nhalos, FarRec* out);
+
+// What the rule looks at in a packed model: the direct sum's cost, the area over which the halos lie and the mean area
+// inside which a halo is near a tile of half side 1.
+struct FarStats {
+    int nhalos = 0, nruns = 0;
+    ModelCost cost;
+    double area = 0, near_area = 0;
+};
+
+FarStats far_stats(const HaloRec* recs, int nhalos, const std::vector<Run>& runs);
+
+// How a map is summed: directly, or by tile expansions in work-groups of 64 (4 or 16 waves), 128 or 256 pixels a
+// side.
+enum class FarShape { Direct, Root64, Root64Wide, Root128, Root256 };
+
+// The shape for a map. `whole`: the grid that the rows computed belong to (the grid itself, or the whole map where
+// a part of it is computed on its own). *cost (may be NULL): estimated instructions per pixel of the form chosen.
+FarShape far_shape(const FarStats& st, int kind, int precision, const GridDesc& whole, double* cost);
+
+// map o.kind of the grid in the shape that far_shape() gave (not Direct)
+hipError_t launch_far(const HaloRec* halos, const FarRec* recs, const Run* runs, int nruns, int nhalos, const GridDesc& g,
+                      const OutDesc& o, FarShape shape, hipStream_t s);
+
+}  // namespace lt

@@ -5,6 +5,8 @@
 
 #include <string>
 
+#include "lenstool_hip/lt_capi.h"
+
 namespace lt {
 
 // record `msg` as the calling thread's last error and return `code`
@@ -20,6 +22,11 @@ hipError_t launch_fill_bytes(void* dst, unsigned char v, size_t bytes, hipStream
 // with `dev` current: the device address of lt_critic_device_noalloc's scratch array on `dev`, looked
 // up once per device (ptr may be NULL: set-up only)
 int critic_noalloc_setup(int dev, void** ptr);
+// lt_map_device of `grid`, a part of the map `whole`, by the kernel that the whole map takes
+int map_device_rows(lt_model m, int kind, int mode, double* const outs[5], double r, double mult,
+                    const lt_grid_desc* grid, const lt_grid_desc* whole, int precision, int px, void* stream);
+// estimated instructions per pixel of that map, and whether it is computed in tiles of 64 or 128 rows
+double map_rows_cost(lt_model m, int kind, int precision, const lt_grid_desc* whole, bool* tiled);
 
 }  // namespace lt
 

@@ -51,6 +51,18 @@ enum class Use { Gradient, Hessian, Kmap, Potential };
 int pack_model(const lt_potential_soa* lens, int nhalos, Use use, std::vector<HaloRec>& recs,
                std::vector<HaloRec32>& recs32, std::vector<Run>& runs, std::string& err);
 
+// Instructions per pixel of the direct kernels, summed over a model's halos, by family (FAM_*): what the choices of
+// launch shape go by.
+enum : int { FAM_GRADIENT = 0, FAM_HESSIAN = 1, FAM_POTENTIAL = 2, FAM_TRACE = 3 };  // TRACE: xx + yy alone
+
+struct ModelCost {
+    double px[4] = {0, 0, 0, 0};
+};
+
+int family_of(int kind);
+ModelCost model_cost(const std::vector<Run>& runs);
+double direct_cost(const ModelCost& c, int kind, int precision);
+
 // Cosmology (lt_cosmo.cpp): angular distances in units of c/H0 and D_ls/D_s.
 double cosmo_observer_object(double z, const lt_cosmo_param& c);
 double cosmo_object_object(double z1, double z2, const lt_cosmo_param& c);

@@ -489,13 +489,6 @@ __device__ __forceinline__ void term64(const HaloRec& h, double px, double py, d
     else hess_sis(h, px, py, sT, sD, sB);
 }
 
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // sum over the 64 lanes of one component's lane sums a[j] (j < SEG) into pixel lane j's FP64 sum s,
 // through this wavefront's LDS slice (layout [source lane][pixel]): lane (p = lane % SEG,
 // q = lane / SEG) adds the sums of source lanes 16 q .. 16 q + 15 for pixel p in FP64, then the four

@@ -78,6 +78,13 @@ int pack_model(const lt_potential_soa* L, int n, Use use, std::vector<HaloRec>& 
             h.ampg = b0;
             h.amph = b0 * h.sa * h.sb;
             h.circ = (eps == 0.0) ? 1.0 : 0.0;
+            // far test of the tile expansions: the frame in which R^2 = X^2 + Y^2
+            const double ra = std::sqrt(h.sa), rb = std::sqrt(h.sb);
+            h.csx = ra * cs;
+            h.snx = ra * sn;
+            h.csy = rb * cs;
+            h.sny = rb * sn;
+            h.kx = std::fmax(h.sa, h.sb);
         } else if (piemd) {
             if (!L->rcore || (t == TYPE_DPIE && !L->rcut)) {
                 err = "lens model: rcore / rcut is NULL";
@@ -96,7 +103,7 @@ int pack_model(const lt_potential_soa* L, int n, Use use, std::vector<HaloRec>& 
             h.rcut = rcut;
             h.kx = 1.0 / ((1.0 + eps) * (1.0 + eps));
             h.ky = 1.0 / ((1.0 - eps) * (1.0 - eps));
-            h.e2 = 2.0 * sqe;
+            const double e2 = 2.0 * sqe;
             h.cx1 = cx1;
             h.gki = 2.0 * sqe / ((1.0 + eps) * (1.0 + eps));
             h.gkv = 2.0 * sqe / ((1.0 + eps) * (1.0 - eps));
@@ -114,13 +121,14 @@ int pack_model(const lt_potential_soa* L, int n, Use use, std::vector<HaloRec>& 
                 h.snx = cx1 * a * sn;
                 h.csy = cx1 * b * cs;
                 h.sny = cx1 * b * sn;
-                h.k1 = h.e2 * a / cx1;
+                h.k1 = e2 * a / cx1;
                 h.k2 = b / a;
-                h.k3 = h.e2 * b / cx1;
+                h.k3 = e2 * b / cx1;
                 h.k4 = 1.0 / (cx1 * cx1);
-                h.k5 = h.e2 * a;
+                h.k5 = e2 * a;
                 h.ra2c = cx1 * cx1 * rc * rc;
                 h.rb2c = cx1 * cx1 * rcut * rcut;
+                h.far0 = (t == TYPE_DPIE) ? std::fmin(h.ra2c, h.rb2c) : h.ra2c;
             }
             // potential constants (lt_terms64.h pot_piemd): c = 1 + cx1 = 2 / (1 + e)
             const double c = 2.0 / (1.0 + eps);
@@ -145,7 +153,7 @@ int pack_model(const lt_potential_soa* L, int n, Use use, std::vector<HaloRec>& 
         h.hs2 = h.amph * sin2;
         if (piemd) {
             const double a = 1.0 / (1.0 + eps);
-            const double e2a2 = h.e2 * a * a;
+            const double e2a2 = 2.0 * std::sqrt(eps) * a * a;
             h.qT = h.amph * e2a2;
             h.qc2 = h.hc2 * e2a2;
             h.qs2m2 = -2.0 * h.hs2 * e2a2;
@@ -156,7 +164,7 @@ int pack_model(const lt_potential_soa* L, int n, Use use, std::vector<HaloRec>& 
         HaloRec32& f = recs32[i];
         f = HaloRec32{};
         if (piemd) {
-            const double a = 1.0 / (1.0 + eps), e2 = h.e2;
+            const double a = 1.0 / (1.0 + eps), e2 = 2.0 * std::sqrt(eps);
             // The FP32 terms are the I_{0.5} Hessian times 1 / (2 sqrt(e) a^2): fold that factor back in.
             const double amp = h.amph * e2 * a * a;
             f.csx = (float)h.csx;
@@ -287,6 +295,36 @@ int pack_model(const lt_potential_soa* L, int n, Use use, std::vector<HaloRec>& 
         s += c;
     }
     return LT_OK;
+}
+
+int family_of(int kind)
+{
+    return kind == LT_MAP_GRADIENT || kind == LT_MAP_DPL ? FAM_GRADIENT
+           : kind == LT_MAP_POT                          ? FAM_POTENTIAL
+           : kind == LT_MAP_MASS                         ? FAM_TRACE
+                                                         : FAM_HESSIAN;
+}
+
+ModelCost model_cost(const std::vector<Run>& runs)
+{
+    // VALU instructions per halo and pixel of the FP64 kernels (gradient, Hessian, potential, trace)
+    static const double kDpie[4] = {126., 55., 228., 24.}, kPiemd[4] = {85., 34., 140., 15.},
+                        kSis[4] = {34., 34., 40., 20.}, kCirc[4] = {17., 21., 40., 11.};
+    ModelCost c;
+    for (const Run& r : runs)
+        for (int f = 0; f < 4; ++f)
+            c.px[f] += r.count * (r.type == TYPE_DPIE    ? kDpie[f]
+                                  : r.type == TYPE_PIEMD ? kPiemd[f]
+                                  : r.type == TYPE_SIS   ? (r.circ ? kCirc[f] : kSis[f])
+                                                         : 3.);
+    return c;
+}
+
+double direct_cost(const ModelCost& c, int kind, int precision)
+{
+    static const double kFp32Share[4] = {0.43, 0.6, 0.35, 0.6};  // of the FP64 kernels' time
+    const int fam = family_of(kind);
+    return c.px[fam] * (precision == LT_PREC_FP32C ? kFp32Share[fam] : 1.);
 }
 
 }  // namespace lt

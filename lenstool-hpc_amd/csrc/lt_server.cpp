@@ -103,7 +103,8 @@ int planes_of(int kind)
 
 // Rows per tile: about kTileWork Hessian-equivalent halo x pixels per launch (~2 ms of FP64 Hessian
 // work on the MI355X), from the measured cost of each kernel family per halo x pixel relative to
-// the FP64 Hessian; at least 4 rows (one work-group row).
+// the FP64 Hessian; at least 4 rows (one work-group row). Maps computed by tile expansions take whole
+// tiles of rows, and the form is chosen for the whole map, not for its row tiles.
 constexpr double kTileWork = 1.0e9;
 
 double relative_cost(int kind, int precision)
@@ -117,11 +118,17 @@ double relative_cost(int kind, int precision)
     }
 }
 
-int tile_rows(const lt_request& r, int nhalos)
+// instructions per halo x pixel of the FP64 Hessian kernel, the unit of kTileWork
+constexpr double kHessianInstr = 55.0;
+
+int tile_rows(const lt_request& r, int nhalos, lt_model m)
 {
-    const double per_row = (double)r.grid.nx * std::max(nhalos, 1) * relative_cost(r.kind, r.precision);
-    long long rows = (long long)(kTileWork / per_row);
-    rows = std::max(4LL, rows / 4 * 4);
+    bool tiled = false;
+    const double cost = map_rows_cost(m, r.kind, r.precision, &r.grid, &tiled) / kHessianInstr;
+    const double per_row =
+        (double)r.grid.nx * (tiled ? std::max(cost, 1.0) : std::max(nhalos, 1) * relative_cost(r.kind, r.precision));
+    const long long unit = tiled ? 128 : 4;  // whole expansion tiles, or a work-group row
+    const long long rows = std::max(unit, (long long)(kTileWork / per_row) / unit * unit);
     return (int)std::min<long long>(rows, r.grid.ny);
 }
 
@@ -266,8 +273,10 @@ struct lt_server_s {
         for (int k = 0; k < t.nplanes; ++k) p[k] = t.planes[k] + off;
         t.next_row += rows;
         ++t.tiles_issued;
-        int st = lt_map_device(m.use_model[ui], t.req.kind, t.req.mode, p[0], p[1], p[2], p[3], p[4], t.req.r,
-                               t.req.mult, &g, t.req.precision, 0, s.stream);
+        lt_grid_desc whole = t.req.grid;
+        whole.pitch = whole.nx;
+        int st = map_device_rows(m.use_model[ui], t.req.kind, t.req.mode, p, t.req.r, t.req.mult, &g, &whole,
+                                 t.req.precision, 0, s.stream);
         if (st == LT_OK && hipEventRecord(s.ev, s.stream) != hipSuccess) st = LT_ERR_HIP;
         if (st != LT_OK) {
             // nothing queued for this tile: count it as ended, issue no more of this request
@@ -434,7 +443,7 @@ int lt_server_submit(lt_server s, const lt_request* req, long long* ticket)
     if ((long long)lt_server_s::block_bytes(*t) > s->budget)
         return set_error(LT_ERR_CAPACITY, "request needs more device memory than the server's budget");
     t->halo_px = (double)m.nhalos * req->grid.nx * req->grid.ny;
-    t->rows_per_tile = tile_rows(*req, m.nhalos);
+    t->rows_per_tile = tile_rows(*req, m.nhalos, m.use_model[ui]);
     t->tiles_total = (req->grid.ny + t->rows_per_tile - 1) / t->rows_per_tile;
     t->t_submit = Clock::now();
     *ticket = t->id;

@@ -23,20 +23,38 @@ namespace lt {
 // folded into hc2 = amph cos2t and hs2 = amph sin2t.
 // ------------------------------------------------------------------------------------------------
 
+// Every term comes in two forms: at a pixel (px, py), and `_at` a lab-frame offset (tx, ty) from the
+// halo centre. FULL: reciprocals and inverse square roots with the third-order correction
+// (lt_math.h), for the expansion nodes of lt_far.hip, whose values many pixels share.
+template <bool FULL>
+__device__ __forceinline__ double rsq_c(double q)
+{
+    return FULL ? rsq64(q) : rsq64_n2(q);
+}
+
+template <bool FULL>
+__device__ __forceinline__ double rcp_c(double x)
+{
+    return FULL ? rcp64(x) : rcp64_n2(x);
+}
+
 struct PixelFrame {
     double x, y, x2, y2;
 };
 
-__device__ __forceinline__ PixelFrame halo_frame(const HaloRec& h, double px, double py)
+__device__ __forceinline__ PixelFrame halo_frame_at(const HaloRec& h, double tx, double ty)
 {
     PixelFrame f;
-    double tx = px - h.xh;
-    double ty = py - h.yh;
     f.x = __builtin_fma(tx, h.cs, ty * h.sn);
     f.y = __builtin_fma(ty, h.cs, -(tx * h.sn));
     f.x2 = f.x * f.x;
     f.y2 = f.y * f.y;
     return f;
+}
+
+__device__ __forceinline__ PixelFrame halo_frame(const HaloRec& h, double px, double py)
+{
+    return halo_frame_at(h, px - h.xh, py - h.yh);
 }
 
 // One I_{0.5} term of the PIEMD Hessian in the halo frame (Kassiola & Kovner 1993) in the
@@ -65,9 +83,8 @@ struct PiemdShared {
     double wq0, Qi2, A, Y, Qi, kx2, ky4;
 };
 
-__device__ __forceinline__ PiemdShared piemd_shared(const HaloRec& h, double px, double py)
+__device__ __forceinline__ PiemdShared piemd_shared(const HaloRec& h, double tx, double ty)
 {
-    const double tx = px - h.xh, ty = py - h.yh;
     const double X = __builtin_fma(tx, h.csx, ty * h.snx);
     PiemdShared s;
     s.Y = __builtin_fma(ty, h.csy, -(tx * h.sny));
@@ -81,10 +98,11 @@ __device__ __forceinline__ PiemdShared piemd_shared(const HaloRec& h, double px,
 }
 
 // one core radius r (r2c = cx1^2 r^2)
+template <bool FULL>
 __device__ __forceinline__ PiemdQ piemd_q_term(const HaloRec& h, const PiemdShared& s, double r, double r2c)
 {
     const double W2 = s.wq0 + r2c;
-    const double iW = rsq64_n2(W2);
+    const double iW = rsq_c<FULL>(W2);
     const double W = W2 * iW;
     const double Qr = W + r;
     const double U = __builtin_fma(s.Y, iW, h.k5);
@@ -96,23 +114,23 @@ __device__ __forceinline__ PiemdQ piemd_q_term(const HaloRec& h, const PiemdShar
     return o;
 }
 
-template <bool CUT>
-__device__ __forceinline__ void hess_piemd(const HaloRec& h, double px, double py, double& aT, double& aD,
-                                           double& aB)
+template <bool CUT, bool FULL>
+__device__ __forceinline__ void hess_piemd_at(const HaloRec& h, double tx, double ty, double& aT, double& aD,
+                                              double& aB)
 {
-    const PiemdShared s = piemd_shared(h, px, py);
-    const PiemdQ a = piemd_q_term(h, s, h.rc, h.ra2c);
+    const PiemdShared s = piemd_shared(h, tx, ty);
+    const PiemdQ a = piemd_q_term<FULL>(h, s, h.rc, h.ra2c);
     double dT, dD, dB;
     if (CUT) {
-        const PiemdQ b = piemd_q_term(h, s, h.rcut, h.rb2c);
+        const PiemdQ b = piemd_q_term<FULL>(h, s, h.rcut, h.rb2c);
         // one reciprocal for both radii: 1/|Qa|^2 = |Qb|^2 / (|Qa|^2 |Qb|^2), and the same for b
-        const double ip = rcp64_n2(a.q2 * b.q2);
+        const double ip = rcp_c<FULL>(a.q2 * b.q2);
         const double ia = b.q2 * ip, ib = a.q2 * ip;
         dT = a.iW - b.iW;
         dD = __builtin_fma(a.dd, ia, -(b.dd * ib));
         dB = __builtin_fma(a.xy, ia, -(b.xy * ib));
     } else {
-        const double ia = rcp64_n2(a.q2);
+        const double ia = rcp_c<FULL>(a.q2);
         dT = a.iW;
         dD = a.dd * ia;
         dB = a.xy * ia;
@@ -123,14 +141,22 @@ __device__ __forceinline__ void hess_piemd(const HaloRec& h, double px, double p
     aB = __builtin_fma(h.qs2h, dD, __builtin_fma(h.qc2, dB, aB));
 }
 
+template <bool CUT>
+__device__ __forceinline__ void hess_piemd(const HaloRec& h, double px, double py, double& aT, double& aD,
+                                           double& aB)
+{
+    hess_piemd_at<CUT, false>(h, px - h.xh, py - h.yh, aT, aD, aB);
+}
+
 // SIS / SIE: phi = b0 R, R^2 = (1-e) x^2 + (1+e) y^2; halo-frame Hessian
 // amph/R^3 (y^2, -xy, x^2) with amph = b0 (1-e)(1+e).
-__device__ __forceinline__ void hess_sis(const HaloRec& h, double px, double py, double& aT, double& aD,
-                                         double& aB)
+template <bool FULL>
+__device__ __forceinline__ void hess_sis_at(const HaloRec& h, double tx, double ty, double& aT, double& aD,
+                                            double& aB)
 {
-    PixelFrame f = halo_frame(h, px, py);
+    PixelFrame f = halo_frame_at(h, tx, ty);
     double R2 = __builtin_fma(h.sa, f.x2, h.sb * f.y2);
-    double iR = rsq64_n2(R2);
+    double iR = rsq_c<FULL>(R2);
     double g = iR * iR * iR;
     double dyx = f.y2 - f.x2;
     double xy = f.x * f.y;
@@ -139,18 +165,30 @@ __device__ __forceinline__ void hess_sis(const HaloRec& h, double px, double py,
     aB = __builtin_fma(g, __builtin_fma(0.5 * h.hs2, dyx, -(h.hc2 * xy)), aB);
 }
 
+__device__ __forceinline__ void hess_sis(const HaloRec& h, double px, double py, double& aT, double& aD,
+                                         double& aB)
+{
+    hess_sis_at<false>(h, px - h.xh, py - h.yh, aT, aD, aB);
+}
+
 // Circular SIS (e = 0): the Hessian b0/r^3 (y^2, -xy, x^2) holds in any frame, so it is formed from
 // the lab-frame offsets, with no rotation to the halo frame and back (T = b0 / r).
-__device__ __forceinline__ void hess_sis_circ(const HaloRec& h, double px, double py, double& aT, double& aD,
-                                              double& aB)
+template <bool FULL>
+__device__ __forceinline__ void hess_sis_circ_at(const HaloRec& h, double tx, double ty, double& aT, double& aD,
+                                                 double& aB)
 {
-    const double tx = px - h.xh, ty = py - h.yh;
     const double x2 = tx * tx, y2 = ty * ty;
-    const double iR = rsq64_n2(x2 + y2);
+    const double iR = rsq_c<FULL>(x2 + y2);
     const double ga = h.amph * (iR * iR * iR);
     aT = __builtin_fma(h.amph, iR, aT);
     aD = __builtin_fma(ga, y2 - x2, aD);
     aB = __builtin_fma(-ga, tx * ty, aB);
+}
+
+__device__ __forceinline__ void hess_sis_circ(const HaloRec& h, double px, double py, double& aT, double& aD,
+                                              double& aB)
+{
+    hess_sis_circ_at<false>(h, px - h.xh, py - h.yh, aT, aD, aB);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -170,11 +208,12 @@ struct QS64 {
     double R, Q2, S;  // Re Q, |Q|^2, S
 };
 
+template <bool FULL>
 __device__ __forceinline__ QS64 qs64(const HaloRec& h, double rem2, double I2, double vy, double r, double r2,
                                      double rcx)
 {
     const double q = r2 + rem2;
-    const double w = q * rsq64_n2(q);
+    const double w = q * rsq_c<FULL>(q);
     QS64 o;
     o.R = __builtin_fma(h.cx1, w, r);
     o.Q2 = __builtin_fma(o.R, o.R, I2);
@@ -186,23 +225,23 @@ __device__ __forceinline__ QS64 qs64(const HaloRec& h, double rem2, double I2, d
 // the dPIE the two logarithms and the two arguments are merged into one of each, with I = Im Q the same
 // for both radii: arg(Za / Zb) = atan2(I (Rb - Ra), Ra Rb + I^2) (Ra Rb + I^2 > 0: no unwrapping) and
 // ln|Za / Zb| = ln(|Qa|^2 Sb^2 / (|Qb|^2 Sa^2)) / 2.
-template <bool CUT>
-__device__ __forceinline__ void grad_piemd(const HaloRec& h, double px, double py, double& gx, double& gy)
+template <bool CUT, bool FULL>
+__device__ __forceinline__ void grad_piemd_at(const HaloRec& h, double tx, double ty, double& gx, double& gy)
 {
-    PixelFrame f = halo_frame(h, px, py);
+    PixelFrame f = halo_frame_at(h, tx, ty);
     const double rem2 = __builtin_fma(f.x2, h.kx, f.y2 * h.ky);
     const double I = h.gki * f.x;
     const double I2 = I * I;
     const double vy = h.gkv * f.y;
-    const QS64 a = qs64(h, rem2, I2, vy, h.rc, h.ra2, h.rca);
+    const QS64 a = qs64<FULL>(h, rem2, I2, vy, h.rc, h.ra2, h.rca);
     double arg, ratio;
     if (CUT) {
-        const QS64 b = qs64(h, rem2, I2, vy, h.rcut, h.rb2, h.rcb);
+        const QS64 b = qs64<FULL>(h, rem2, I2, vy, h.rcut, h.rb2, h.rcb);
         arg = atan2p_lt(I * (b.R - a.R), __builtin_fma(a.R, b.R, I2));
-        ratio = (a.Q2 * (b.S * b.S)) * rcp64_n2(b.Q2 * (a.S * a.S));
+        ratio = (a.Q2 * (b.S * b.S)) * rcp_c<FULL>(b.Q2 * (a.S * a.S));
     } else {
         arg = atan2p_lt(I, a.R);
-        ratio = a.Q2 * rcp64_n2(a.S * a.S);
+        ratio = a.Q2 * rcp_c<FULL>(a.S * a.S);
     }
     const double lnr = 0.5 * log_lt(ratio);
     const double re = h.ampg * arg;
@@ -211,9 +250,15 @@ __device__ __forceinline__ void grad_piemd(const HaloRec& h, double px, double p
     gy += __builtin_fma(im, h.cs, re * h.sn);
 }
 
-__device__ __forceinline__ void grad_sis(const HaloRec& h, double px, double py, double& gx, double& gy)
+template <bool CUT>
+__device__ __forceinline__ void grad_piemd(const HaloRec& h, double px, double py, double& gx, double& gy)
 {
-    PixelFrame f = halo_frame(h, px, py);
+    grad_piemd_at<CUT, false>(h, px - h.xh, py - h.yh, gx, gy);
+}
+
+__device__ __forceinline__ void grad_sis_at(const HaloRec& h, double tx, double ty, double& gx, double& gy)
+{
+    PixelFrame f = halo_frame_at(h, tx, ty);
     double R2 = __builtin_fma(h.sa, f.x2, h.sb * f.y2);
     double s = h.ampg * rsq64(R2);
     double rx = h.sa * f.x * s;
@@ -222,13 +267,22 @@ __device__ __forceinline__ void grad_sis(const HaloRec& h, double px, double py,
     gy += __builtin_fma(ry, h.cs, rx * h.sn);
 }
 
-// Circular SIS: b0 (x, y) / r in any frame, formed from the lab-frame offsets.
-__device__ __forceinline__ void grad_sis_circ(const HaloRec& h, double px, double py, double& gx, double& gy)
+__device__ __forceinline__ void grad_sis(const HaloRec& h, double px, double py, double& gx, double& gy)
 {
-    const double tx = px - h.xh, ty = py - h.yh;
+    grad_sis_at(h, px - h.xh, py - h.yh, gx, gy);
+}
+
+// Circular SIS: b0 (x, y) / r in any frame, formed from the lab-frame offsets.
+__device__ __forceinline__ void grad_sis_circ_at(const HaloRec& h, double tx, double ty, double& gx, double& gy)
+{
     const double s = h.ampg * rsq64(__builtin_fma(tx, tx, ty * ty));
     gx = __builtin_fma(s, tx, gx);
     gy = __builtin_fma(s, ty, gy);
+}
+
+__device__ __forceinline__ void grad_sis_circ(const HaloRec& h, double px, double py, double& gx, double& gy)
+{
+    grad_sis_circ_at(h, px - h.xh, py - h.yh, gx, gy);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -268,13 +322,14 @@ struct PotRad {
     double w, d, R, lq;  // w, w - r, Re Q, ln(|Q|^2 / (c r)^2)
 };
 
+template <bool FULL>
 __device__ __forceinline__ PotRad pot_rad(const HaloRec& h, double rem2, double I2, double r, double r2, double cr,
                                           double icr2)
 {
     const double q = r2 + rem2;
     PotRad o;
-    o.w = q * rsq64_n2(q);
-    o.d = rem2 * rcp64_n2(o.w + r);
+    o.w = q * rsq_c<FULL>(q);
+    o.d = rem2 * rcp_c<FULL>(o.w + r);
     const double cd = h.cx1 * o.d;
     o.R = cd + cr;
     o.lq = log1p_lt(__builtin_fma(cd, __builtin_fma(2., cr, cd), I2) * icr2);
@@ -282,7 +337,7 @@ __device__ __forceinline__ PotRad pot_rad(const HaloRec& h, double rem2, double 
 }
 
 // pi05 of a PIEMD (type 8) or dPIE (type 81) halo without its amplitude; mn = min(mn, rem^2).
-template <bool CUT>
+template <bool CUT, bool FULL = false>
 __device__ __forceinline__ double pot_piemd(const HaloRec& h, const PixelFrame& f, double& mn)
 {
     const double rem2 = __builtin_fma(f.x2, h.kx, f.y2 * h.ky);
@@ -290,15 +345,15 @@ __device__ __forceinline__ double pot_piemd(const HaloRec& h, const PixelFrame& 
     const double I = h.gki * f.x;
     const double I2 = I * I;
     const double v = h.gkv * f.y;
-    const PotRad a = pot_rad(h, rem2, I2, h.rc, h.ra2, h.pcra, h.picra2);
+    const PotRad a = pot_rad<FULL>(h, rem2, I2, h.rc, h.ra2, h.pcra, h.picra2);
     if (!CUT) {
         const double ls = log1p_lt((a.d + v) * h.picra);
         const double arg = atan2p_lt(I, a.R);
         const double ay = __builtin_fma(-0.5, a.lq, ls);
         return __builtin_fma(f.x, arg, __builtin_fma(f.y, ay, -(h.psra * a.lq)));
     }
-    const PotRad b = pot_rad(h, rem2, I2, h.rcut, h.rb2, h.pcrb, h.picrb2);
-    const double sig = (a.d + b.d) * rcp64_n2(a.w + b.w);
+    const PotRad b = pot_rad<FULL>(h, rem2, I2, h.rcut, h.rb2, h.pcrb, h.picrb2);
+    const double sig = (a.d + b.d) * rcp_c<FULL>(a.w + b.w);
     const double dR = h.pdr * __builtin_fma(-h.cx1, sig, h.pc);
     const double arg = atan2p_lt(I * dR, __builtin_fma(a.R, b.R, I2));
     const double Q2a = __builtin_fma(a.R, a.R, I2);
@@ -307,18 +362,24 @@ __device__ __forceinline__ double pot_piemd(const HaloRec& h, const PixelFrame& 
     const double Pa = __builtin_fma(ga, Sa + a.R, -I2);
     const double dP = __builtin_fma(Sb + b.R, h.pomcdr * sig, -(ga * (h.pcdr * (2. - sig))));
     const double N = __builtin_fma(Pa, dR * (a.R + b.R), Q2a * dP);
-    const double ay = 0.5 * log1p_lt(N * rcp64_n2((Sb * Sb) * Q2a));
+    const double ay = 0.5 * log1p_lt(N * rcp_c<FULL>((Sb * Sb) * Q2a));
     const double L = __builtin_fma(h.psra, a.lq, -(h.psrb * b.lq));
     return __builtin_fma(f.x, arg, __builtin_fma(f.y, ay, -L));
 }
 
 // One halo's potential at (px, py) (SIS: b0 R, R^2 = (1-e) x^2 + (1+e) y^2).
+template <bool FULL>
+__device__ __forceinline__ double pot_halo_at(const HaloRec& h, int type, double tx, double ty, double& mn)
+{
+    const PixelFrame f = halo_frame_at(h, tx, ty);
+    if (type == TYPE_SIS) return h.ampg * sqrt(__builtin_fma(h.sa, f.x2, h.sb * f.y2));
+    const double v = (type == TYPE_PIEMD) ? pot_piemd<false, FULL>(h, f, mn) : pot_piemd<true, FULL>(h, f, mn);
+    return h.ampg * v;
+}
+
 __device__ __forceinline__ double pot_halo(const HaloRec& h, int type, double px, double py, double& mn)
 {
-    const PixelFrame f = halo_frame(h, px, py);
-    if (type == TYPE_SIS) return h.ampg * sqrt(__builtin_fma(h.sa, f.x2, h.sb * f.y2));
-    const double v = (type == TYPE_PIEMD) ? pot_piemd<false>(h, f, mn) : pot_piemd<true>(h, f, mn);
-    return h.ampg * v;
+    return pot_halo_at<false>(h, type, px - h.xh, py - h.yh, mn);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -405,6 +466,14 @@ __device__ __forceinline__ void hess_epilogue(const OutDesc& o, int64_t idx, dou
 // ------------------------------------------------------------------------------------------------
 constexpr int WAVE = 64;
 constexpr int ROWS = 4;
+
+// orders a wavefront's own LDS accesses: what its lanes wrote before is what they read after
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // Sample s of a batch (blockIdx.z) uses its own halo records and output planes.
 __device__ __forceinline__ const HaloRec* select_sample(const GridDesc& g, const HaloRec* halos, OutDesc& o)
