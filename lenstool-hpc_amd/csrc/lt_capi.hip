@@ -136,6 +136,20 @@ struct DevModel {
     FarStats far;  // of the model (of a batch's first sample) as it was created
 };
 
+// Small maps: the halos of a row segment shared by several waves (lt_kernels64.hip), whatever px is asked for (every
+// px gives the same map). The sums through LDS cost about as much as 300 instructions a pixel, so the lighter the
+// model the earlier one wave per segment is enough: measured (us, one wave / split) 64^2 258 halos fields 97 / 14,
+// potential 392 / 44; 200^2 102 / 40 and 396 / 142; 512^2 168 / 150 and 667 / 543; 30 halos fields 256^2 14 / 8,
+// 400^2 20 / 16, 512^2 21 / 23; 11 halos (1 dPIE + 10 SIS) 200^2 8 / 8, 400^2 7 / 9. FP32C: 258 halos gradient 512^2
+// 166 / 166, 724^2 338 / 321, 1024^2 534 / 609; 60 mixed halos gradient 256^2 31 / 20, 400^2 33 / 52; 30 halos
+// fields 256^2 19 / 9, 400^2 19 / 20.
+bool split_halos(const ModelCost& model, int kind, int precision, const GridDesc& whole)
+{
+    const double npix = (double)whole.nx * (double)whole.ny, cost = direct_cost(model, kind, precision);
+    if (precision == LT_PREC_FP32C) return npix <= std::min(6e5, (kind == LT_MAP_POT ? 100. : 75.) * cost);
+    return npix <= std::min(1e6, 52. * cost);
+}
+
 // Launch the kernel that produces map `kind` from a device model. `whole`: the grid that g is rows of.
 int launch_map(const DevModel& m, int kind, int mode, double* const outs[5], double r, double mult,
                const GridDesc& g, const GridDesc& whole, int precision, int px, hipStream_t s, int nhalos)
@@ -172,6 +186,7 @@ int launch_map(const DevModel& m, int kind, int mode, double* const outs[5], dou
         if (e != hipSuccess) return hip_fail(e, "kernel launch");
         return LT_OK;
     }
+    if (px != LT_PX_HALO_LANES && split_halos(m.far.cost, kind, precision, whole)) px = kPxSplit;
     switch (kind) {
     case LT_MAP_GRADIENT:
     case LT_MAP_DPL:

@@ -11,7 +11,10 @@
 
 namespace lt {
 
-// FP64 kernels (lt_kernels64.hip). px = pixels per thread (1, 2 or 4).
+// px of a launch in the split form (lt_kernels64.hip): several waves share a row segment's halos
+constexpr int kPxSplit = -1;
+
+// FP64 kernels (lt_kernels64.hip). px = pixels per thread (1, 2 or 4) or kPxSplit.
 hipError_t launch_hessian64(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
                             const OutDesc& o, int px, hipStream_t s);
 hipError_t launch_gradient64(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,

@@ -37,6 +37,13 @@ namespace lt {
 
 constexpr int CHUNK = 8;
 
+// the split form (lt_kernels64.hip) by whole chunks: this wave's first chunk of a run, then every SPLIT-th
+template <int SPLIT>
+__device__ __forceinline__ int first_chunk(int start, int wave)
+{
+    return SPLIT == 1 ? start : start + CHUNK * ((wave - start) & (SPLIT - 1));
+}
+
 // The gradient kernel stages the FP32 records of a run through LDS in tiles of TILE records (8 KB),
 // which the four waves of the work-group then read with broadcast LDS loads. On gfx950 an FP32 VALU
 // instruction with an SGPR operand issues at half the rate of one whose operands are all VGPRs
@@ -45,18 +52,18 @@ constexpr int CHUNK = 8;
 // wavefront-uniform record leave them in SGPRs. TILE is a multiple of CHUNK, so the chunks (and the
 // sums) are those of the untiled walk.
 constexpr int TILE = 64;
-static_assert(TILE % CHUNK == 0, "tiles hold whole chunks");
+static_assert(TILE % (CHUNK * kSplit) == 0, "tiles hold whole chunks of every wave");
 
 // n records recs[i0 .. i0+n) into tile[0 .. n), 16 bytes per thread and step; the caller brackets
 // it with barriers (every thread of the work-group calls it with the same arguments)
-template <typename Rec>
+template <int THREADS, typename Rec>
 __device__ __forceinline__ void stage_tile(Rec* __restrict__ tile, const Rec* __restrict__ recs, int i0, int n)
 {
     static_assert(sizeof(Rec) % 16 == 0, "records are whole 16-byte vectors");
     constexpr int V = sizeof(Rec) / 16;
     const float4* src = reinterpret_cast<const float4*>(recs + i0);
     float4* dst = reinterpret_cast<float4*>(tile);
-    for (int j = threadIdx.y * WAVE + threadIdx.x; j < n * V; j += WAVE * ROWS) dst[j] = src[j];
+    for (int j = threadIdx.y * WAVE + threadIdx.x; j < n * V; j += THREADS) dst[j] = src[j];
 }
 
 // Record j of a tile by value, only its first NV 16-byte vectors read (the fields the FP32 terms
@@ -218,11 +225,12 @@ __device__ __forceinline__ void pin_record(const HaloRec32& h, double xh, double
 // lanes) straight into the FP64 run sums. The records are wavefront-uniform scalar loads (the
 // Hessian keeps them in SGPRs: staged through LDS they cost 20 VGPRs, two waves of occupancy, and
 // measured slower, 9.6 against 8.9 ms on the 503-halo 4096^2 map).
-template <int TYPE, int PX>
-__device__ __forceinline__ void run32(const HaloRec* __restrict__ h64, const HaloRec32* __restrict__ h32, int start,
-                                      int end, const double* px, double py, double* sT, double* sD, double* sB)
+template <int TYPE, int PX, int SPLIT>
+__device__ __forceinline__ void run32(const HaloRec* __restrict__ h64, const HaloRec32* __restrict__ h32, int wave,
+                                      int start, int end, const double* px, double py, double* sT, double* sD,
+                                      double* sB)
 {
-    for (int c0 = start; c0 < end; c0 += CHUNK) {
+    for (int c0 = first_chunk<SPLIT>(start, wave); c0 < end; c0 += CHUNK * SPLIT) {
         const int c1 = min(c0 + CHUNK, end);
         float fT[PX], fD[PX], fB[PX];
 #pragma unroll
@@ -296,13 +304,21 @@ __device__ __forceinline__ void hessian_fp64_pixel(const HaloRec* __restrict__ h
 // |det A (FP32C) - det A (FP64)| under 1e-6 everywhere. A few pixels per halo core pay it.
 constexpr double kDetGuard = 8.0;
 
-template <int PX, int KIND>
-__global__ __launch_bounds__(WAVE* ROWS) void k_hessian32(const HaloRec* __restrict__ h64,
+__device__ __forceinline__ bool past_det_guard(double T, double D, double B, double r)
+{
+    const double kap = 0.5 * T * r;
+    const double gb = 0.5 * (__builtin_fabs(D) + 2. * __builtin_fabs(B)) * __builtin_fabs(r);
+    return __builtin_fabs(1. - kap) + gb > kDetGuard;
+}
+
+template <int PX, int KIND, int SPLIT>
+__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_hessian32(const HaloRec* __restrict__ h64,
                                                           const HaloRec32* __restrict__ h32,
                                                           const Run* __restrict__ runs, int nruns,
                                                           GridDesc g, OutDesc o)
 {
-    const int row = blockIdx.y * ROWS + threadIdx.y;
+    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
     if (row >= g.ny) return;
     h64 = select_sample(g, h64, o);
     h32 += (int64_t)blockIdx.z * g.halo_stride;
@@ -321,7 +337,7 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_hessian32(const HaloRec* __restr
         for (int k = 0; k < PX; ++k) sT[k] = sD[k] = sB[k] = 0.;
         const int end = run.start + run.count;
         if (run.type == TYPE_SHEAR) {
-            for (int i = run.start; i < end; ++i) {
+            for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
                 const HaloRec& h = h64[i];
 #pragma unroll
                 for (int k = 0; k < PX; ++k) {
@@ -331,13 +347,13 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_hessian32(const HaloRec* __restr
                 }
             }
         } else if (run.type == TYPE_DPIE) {
-            run32<TYPE_DPIE, PX>(h64, h32, run.start, end, px, py, sT, sD, sB);
+            run32<TYPE_DPIE, PX, SPLIT>(h64, h32, wave, run.start, end, px, py, sT, sD, sB);
         } else if (run.type == TYPE_PIEMD) {
-            run32<TYPE_PIEMD, PX>(h64, h32, run.start, end, px, py, sT, sD, sB);
+            run32<TYPE_PIEMD, PX, SPLIT>(h64, h32, wave, run.start, end, px, py, sT, sD, sB);
         } else if (run.circ) {
-            run32<TYPE_SIS_CIRC, PX>(h64, h32, run.start, end, px, py, sT, sD, sB);
+            run32<TYPE_SIS_CIRC, PX, SPLIT>(h64, h32, wave, run.start, end, px, py, sT, sD, sB);
         } else {
-            run32<TYPE_SIS, PX>(h64, h32, run.start, end, px, py, sT, sD, sB);
+            run32<TYPE_SIS, PX, SPLIT>(h64, h32, wave, run.start, end, px, py, sT, sD, sB);
         }
         const double w = run.weight;
 #pragma unroll
@@ -347,13 +363,25 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_hessian32(const HaloRec* __restr
             tB[k] = __builtin_fma(w, sB[k], tB[k]);
         }
     }
+    if constexpr (SPLIT > 1) {
+        if constexpr (KIND == LT_MAP_MASS) {
+            if (!split_sum<PX, SPLIT>(wave, tT)) return;
+        } else {
+            if (!split_sum<PX, SPLIT>(wave, tT, tD, tB)) return;
+        }
+        const int col = col0 + wave * WAVE;
+        if constexpr (KIND == LT_MAP_FIELDS || KIND == LT_MAP_AMPLI || KIND == LT_MAP_SHEAR) {
+            if (nruns > 0 && past_det_guard(tT[0], tD[0], tB[0], o.r))
+                hessian_fp64_pixel(h64, runs, nruns, pixel_coord(g.xmin, col + g.istart, g.dx), py, tT[0], tD[0], tB[0]);
+        }
+        if (col < g.nx) hess_epilogue<KIND>(o, (int64_t)row * g.pitch + col, tT[0], tD[0], tB[0]);
+        return;
+    }
     if constexpr (KIND == LT_MAP_FIELDS || KIND == LT_MAP_AMPLI || KIND == LT_MAP_SHEAR) {
         // one pixel at a time (not unrolled) so that the FP64 loop adds no registers to the kernel; with
         // no runs there is nothing to recompute
         for (int k = 0; k < PX && nruns > 0; ++k) {
-            const double kap = 0.5 * tT[k] * o.r;
-            const double gb = 0.5 * (__builtin_fabs(tD[k]) + 2. * __builtin_fabs(tB[k])) * __builtin_fabs(o.r);
-            if (__builtin_fabs(1. - kap) + gb > kDetGuard) hessian_fp64_pixel(h64, runs, nruns, px[k], py, tT[k], tD[k], tB[k]);
+            if (past_det_guard(tT[k], tD[k], tB[k], o.r)) hessian_fp64_pixel(h64, runs, nruns, px[k], py, tT[k], tD[k], tB[k]);
         }
     }
 #pragma unroll
@@ -363,17 +391,18 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_hessian32(const HaloRec* __restr
     }
 }
 
-template <int PX>
+template <int PX, int SPLIT>
 static hipError_t launch_hessian32_px(const HaloRec* h64, const HaloRec32* h32, const Run* runs, int nruns,
                                       const GridDesc& g, const OutDesc& o, hipStream_t s)
 {
-    dim3 blk(WAVE, ROWS, 1), grd = grid_for(g, PX);
+    dim3 blk, grd;
+    geometry<PX, SPLIT>(g, grd, blk);
     switch (o.kind) {
-    case LT_MAP_FIELDS: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_FIELDS>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
-    case LT_MAP_AMPLI: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_AMPLI>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
-    case LT_MAP_SHEAR: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_SHEAR>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
-    case LT_MAP_MASS: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_MASS>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
-    default: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_HESSIAN>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
+    case LT_MAP_FIELDS: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_FIELDS, SPLIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
+    case LT_MAP_AMPLI: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_AMPLI, SPLIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
+    case LT_MAP_SHEAR: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_SHEAR, SPLIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
+    case LT_MAP_MASS: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_MASS, SPLIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
+    default: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_HESSIAN, SPLIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
     }
     return hipGetLastError();
 }
@@ -638,9 +667,7 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_hessian32h(const HaloRec* __rest
     const int col = col0 + lane;
     if (lane < SEG && col < g.nx) {
         if constexpr (KIND == LT_MAP_FIELDS || KIND == LT_MAP_AMPLI || KIND == LT_MAP_SHEAR) {
-            const double kap = 0.5 * tT * o.r;
-            const double gb = 0.5 * (__builtin_fabs(tD) + 2. * __builtin_fabs(tB)) * __builtin_fabs(o.r);
-            if (nruns > 0 && __builtin_fabs(1. - kap) + gb > kDetGuard) hessian_fp64_pixel(h64, runs, nruns, sp.pxl, sp.py, tT, tD, tB);
+            if (nruns > 0 && past_det_guard(tT, tD, tB, o.r)) hessian_fp64_pixel(h64, runs, nruns, sp.pxl, sp.py, tT, tD, tB);
         }
         hess_epilogue<KIND>(o, (int64_t)row * g.pitch + col, tT, tD, tB);
     }
@@ -666,10 +693,11 @@ hipError_t launch_hessian32(const HaloRec* h64, const HaloRec32* h32, const Run*
                             const OutDesc& o, int px, hipStream_t s)
 {
     switch (px) {
-    case 1: return launch_hessian32_px<1>(h64, h32, runs, nruns, g, o, s);
-    case 4: return launch_hessian32_px<4>(h64, h32, runs, nruns, g, o, s);
+    case kPxSplit: return launch_hessian32_px<1, kSplit>(h64, h32, runs, nruns, g, o, s);
+    case 1: return launch_hessian32_px<1, 1>(h64, h32, runs, nruns, g, o, s);
+    case 4: return launch_hessian32_px<4, 1>(h64, h32, runs, nruns, g, o, s);
     case LT_PX_HALO_LANES: return launch_hessian32h(h64, h32, runs, nruns, g, o, s);
-    default: return launch_hessian32_px<2>(h64, h32, runs, nruns, g, o, s);
+    default: return launch_hessian32_px<2, 1>(h64, h32, runs, nruns, g, o, s);
     }
 }
 
@@ -762,11 +790,11 @@ __device__ __forceinline__ void grad_sis32_circ(const GradRec32& h, float tx, fl
 
 // Halos [t0, t1) of a run, their FP32 records in tile[0 .. t1 - t0): FP32 terms summed per chunk of
 // CHUNK halos, FP64 terms (near lanes) straight into the FP64 run sums
-template <int TYPE, int PX>
-__device__ __forceinline__ void tileg32(const HaloRec* __restrict__ h64, const GradRec32* __restrict__ tile, int t0,
-                                        int t1, const double* px, double py, double* sx, double* sy)
+template <int TYPE, int PX, int SPLIT>
+__device__ __forceinline__ void tileg32(const HaloRec* __restrict__ h64, const GradRec32* __restrict__ tile, int first,
+                                        int t0, int t1, const double* px, double py, double* sx, double* sy)
 {
-    for (int c0 = t0; c0 < t1; c0 += CHUNK) {
+    for (int c0 = t0 + first; c0 < t1; c0 += CHUNK * SPLIT) {
         const int c1 = min(c0 + CHUNK, t1);
         float fx[PX], fy[PX];
 #pragma unroll
@@ -804,29 +832,31 @@ __device__ __forceinline__ void tileg32(const HaloRec* __restrict__ h64, const G
 // One run of halos of one type, its FP32 records staged tile by tile (staged: 12.9 ms on the
 // 503-halo 4096^2 map, scalar loads: 13.9 ms). Called by every thread of the work-group with the
 // same run (the barriers need all of them).
-template <int TYPE, int PX>
+template <int TYPE, int PX, int SPLIT>
 __device__ __forceinline__ void rung32(const HaloRec* __restrict__ h64, const GradRec32* __restrict__ g32,
-                                       GradRec32* __restrict__ tile, int start, int end, const double* px, double py,
+                                       GradRec32* __restrict__ tile, int wave, int start, int end, const double* px, double py,
                                        double* sx, double* sy)
 {
     for (int t0 = start; t0 < end; t0 += TILE) {
         const int t1 = min(t0 + TILE, end);
         __syncthreads();  // every wave is done with the previous tile
-        stage_tile(tile, g32, t0, t1 - t0);
+        stage_tile<WAVE*(SPLIT == 1 ? ROWS : SPLIT)>(tile, g32, t0, t1 - t0);
         __syncthreads();
-        tileg32<TYPE, PX>(h64, tile, t0, t1, px, py, sx, sy);
+        // a tile is TILE / CHUNK = SPLIT chunks, so a wave's first chunk is the same in every tile of the run
+        tileg32<TYPE, PX, SPLIT>(h64, tile, first_chunk<SPLIT>(start, wave) - start, t0, t1, px, py, sx, sy);
     }
 }
 
-template <int PX>
-__global__ __launch_bounds__(WAVE* ROWS) void k_gradient32(const HaloRec* __restrict__ h64,
+template <int PX, int SPLIT>
+__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_gradient32(const HaloRec* __restrict__ h64,
                                                            const GradRec32* __restrict__ g32,
                                                            const Run* __restrict__ runs, int nruns, GridDesc g,
                                                            OutDesc o)
 {
     // rows past the grid walk the runs too (the tile barriers need every thread) and store nothing
     __shared__ GradRec32 tile[TILE];
-    const int row = blockIdx.y * ROWS + threadIdx.y;
+    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
     const bool live = row < g.ny;
     h64 = select_sample(g, h64, o);
     g32 += (int64_t)blockIdx.z * g.halo_stride;
@@ -844,10 +874,10 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_gradient32(const HaloRec* __rest
 #pragma unroll
         for (int k = 0; k < PX; ++k) sx[k] = sy[k] = 0.;
         const int end = run.start + run.count;
-        if (run.type == TYPE_DPIE) rung32<TYPE_DPIE, PX>(h64, g32, tile, run.start, end, px, py, sx, sy);
-        else if (run.type == TYPE_PIEMD) rung32<TYPE_PIEMD, PX>(h64, g32, tile, run.start, end, px, py, sx, sy);
-        else if (run.circ) rung32<TYPE_SIS_CIRC, PX>(h64, g32, tile, run.start, end, px, py, sx, sy);
-        else rung32<TYPE_SIS, PX>(h64, g32, tile, run.start, end, px, py, sx, sy);
+        if (run.type == TYPE_DPIE) rung32<TYPE_DPIE, PX, SPLIT>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
+        else if (run.type == TYPE_PIEMD) rung32<TYPE_PIEMD, PX, SPLIT>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
+        else if (run.circ) rung32<TYPE_SIS_CIRC, PX, SPLIT>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
+        else rung32<TYPE_SIS, PX, SPLIT>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
 #pragma unroll
         for (int k = 0; k < PX; ++k) {
             tx[k] += sx[k];
@@ -855,6 +885,16 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_gradient32(const HaloRec* __rest
         }
     }
     const double m = o.kind == LT_MAP_DPL ? o.r : 1.0;
+    if constexpr (SPLIT > 1) {
+        if (!split_sum<PX, SPLIT>(wave, tx, ty)) return;
+        const int col = col0 + wave * WAVE;
+        if (live && col < g.nx) {
+            const int64_t idx = (int64_t)row * g.pitch + col;
+            o.p0[idx] = tx[0] * m;
+            o.p1[idx] = ty[0] * m;
+        }
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
         const int col = col0 + k * WAVE;
@@ -866,15 +906,24 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_gradient32(const HaloRec* __rest
     }
 }
 
+template <int PX, int SPLIT>
+static void launch_gradient32_px(const HaloRec* h64, const GradRec32* g32, const Run* runs, int nruns,
+                                 const GridDesc& g, const OutDesc& o, hipStream_t s)
+{
+    dim3 blk, grd;
+    geometry<PX, SPLIT>(g, grd, blk);
+    hipLaunchKernelGGL((k_gradient32<PX, SPLIT>), grd, blk, 0, s, h64, g32, runs, nruns, g, o);
+}
+
 hipError_t launch_gradient32(const HaloRec* h64, const HaloRec32* recs32, const Run* runs, int nruns,
                              const GridDesc& g, const OutDesc& o, int px, hipStream_t s)
 {
     const GradRec32* g32 = reinterpret_cast<const GradRec32*>(recs32);
-    dim3 blk(WAVE, ROWS, 1);
     switch (px) {
-    case 1: hipLaunchKernelGGL(k_gradient32<1>, grid_for(g, 1), blk, 0, s, h64, g32, runs, nruns, g, o); break;
-    case 4: hipLaunchKernelGGL(k_gradient32<4>, grid_for(g, 4), blk, 0, s, h64, g32, runs, nruns, g, o); break;
-    default: hipLaunchKernelGGL(k_gradient32<2>, grid_for(g, 2), blk, 0, s, h64, g32, runs, nruns, g, o); break;
+    case kPxSplit: launch_gradient32_px<1, kSplit>(h64, g32, runs, nruns, g, o, s); break;
+    case 1: launch_gradient32_px<1, 1>(h64, g32, runs, nruns, g, o, s); break;
+    case 4: launch_gradient32_px<4, 1>(h64, g32, runs, nruns, g, o, s); break;
+    default: launch_gradient32_px<2, 1>(h64, g32, runs, nruns, g, o, s); break;
     }
     return hipGetLastError();
 }
@@ -976,12 +1025,12 @@ __device__ __forceinline__ float pot32(const PotRec32& h, float tx, float ty, fl
     }
 }
 
-template <int TYPE, int PX>
-__device__ __forceinline__ void runp32(const HaloRec* __restrict__ h64, const PotRec32* __restrict__ p32, int start,
-                                       int end, const double* px, double py, double* s, float* mn)
+template <int TYPE, int PX, int SPLIT>
+__device__ __forceinline__ void runp32(const HaloRec* __restrict__ h64, const PotRec32* __restrict__ p32, int wave,
+                                       int start, int end, const double* px, double py, double* s, float* mn)
 {
 #pragma clang fp contract(off)
-    for (int c0 = start; c0 < end; c0 += CHUNK) {
+    for (int c0 = first_chunk<SPLIT>(start, wave); c0 < end; c0 += CHUNK * SPLIT) {
         const int c1 = min(c0 + CHUNK, end);
         float f[PX];
 #pragma unroll
@@ -1001,13 +1050,14 @@ __device__ __forceinline__ void runp32(const HaloRec* __restrict__ h64, const Po
     }
 }
 
-template <int PX>
-__global__ __launch_bounds__(WAVE* ROWS) void k_potential32(const HaloRec* __restrict__ h64,
+template <int PX, int SPLIT>
+__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_potential32(const HaloRec* __restrict__ h64,
                                                             const PotRec32* __restrict__ p32,
                                                             const Run* __restrict__ runs, int nruns, GridDesc g,
                                                             OutDesc o)
 {
-    const int row = blockIdx.y * ROWS + threadIdx.y;
+    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
     if (row >= g.ny) return;
     h64 = select_sample(g, h64, o);
     p32 += (int64_t)blockIdx.z * g.halo_stride;
@@ -1027,11 +1077,21 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_potential32(const HaloRec* __res
 #pragma unroll
         for (int k = 0; k < PX; ++k) s[k] = 0.;
         const int end = run.start + run.count;
-        if (run.type == TYPE_DPIE) runp32<TYPE_DPIE, PX>(h64, p32, run.start, end, px, py, s, mn);
-        else if (run.type == TYPE_PIEMD) runp32<TYPE_PIEMD, PX>(h64, p32, run.start, end, px, py, s, mn);
-        else runp32<TYPE_SIS, PX>(h64, p32, run.start, end, px, py, s, mn);
+        if (run.type == TYPE_DPIE) runp32<TYPE_DPIE, PX, SPLIT>(h64, p32, wave, run.start, end, px, py, s, mn);
+        else if (run.type == TYPE_PIEMD) runp32<TYPE_PIEMD, PX, SPLIT>(h64, p32, wave, run.start, end, px, py, s, mn);
+        else runp32<TYPE_SIS, PX, SPLIT>(h64, p32, wave, run.start, end, px, py, s, mn);
 #pragma unroll
         for (int k = 0; k < PX; ++k) tot[k] += s[k];
+    }
+    if constexpr (SPLIT > 1) {
+        // a wave that met a PIEMD centre makes the sum NaN
+#pragma unroll
+        for (int k = 0; k < PX; ++k)
+            if (mn[k] == 0.f) tot[k] = __builtin_nan("");
+        if (!split_sum<PX, SPLIT>(wave, tot)) return;
+        const int col = col0 + wave * WAVE;
+        if (col < g.nx) o.p0[(int64_t)row * g.pitch + col] = tot[0] * o.mult;
+        return;
     }
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
@@ -1042,15 +1102,24 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_potential32(const HaloRec* __res
     }
 }
 
+template <int PX, int SPLIT>
+static void launch_potential32_px(const HaloRec* h64, const PotRec32* p32, const Run* runs, int nruns,
+                                  const GridDesc& g, const OutDesc& o, hipStream_t s)
+{
+    dim3 blk, grd;
+    geometry<PX, SPLIT>(g, grd, blk);
+    hipLaunchKernelGGL((k_potential32<PX, SPLIT>), grd, blk, 0, s, h64, p32, runs, nruns, g, o);
+}
+
 hipError_t launch_potential32(const HaloRec* h64, const HaloRec32* recs32, const Run* runs, int nruns,
                               const GridDesc& g, const OutDesc& o, int px, hipStream_t s)
 {
     const PotRec32* p32 = reinterpret_cast<const PotRec32*>(recs32);
-    dim3 blk(WAVE, ROWS, 1);
     switch (px) {
-    case 1: hipLaunchKernelGGL(k_potential32<1>, grid_for(g, 1), blk, 0, s, h64, p32, runs, nruns, g, o); break;
-    case 4: hipLaunchKernelGGL(k_potential32<4>, grid_for(g, 4), blk, 0, s, h64, p32, runs, nruns, g, o); break;
-    default: hipLaunchKernelGGL(k_potential32<2>, grid_for(g, 2), blk, 0, s, h64, p32, runs, nruns, g, o); break;
+    case kPxSplit: launch_potential32_px<1, kSplit>(h64, p32, runs, nruns, g, o, s); break;
+    case 1: launch_potential32_px<1, 1>(h64, p32, runs, nruns, g, o, s); break;
+    case 4: launch_potential32_px<4, 1>(h64, p32, runs, nruns, g, o, s); break;
+    default: launch_potential32_px<2, 1>(h64, p32, runs, nruns, g, o, s); break;
     }
     return hipGetLastError();
 }

@@ -2,6 +2,11 @@
 // potential. One thread owns PX pixels of one row (columns lane, lane+64, ...); a 64x4 workgroup
 // covers 64*PX columns of 4 rows. Halo records are walked in wavefront-uniform order, run by run.
 //
+// Small maps leave most of the chip idle that way: 200 x 200 pixels are 313 waves of two pixels a lane for
+// 1024 SIMDs, each walking every halo one record load after another. The split form (SPLIT > 1) gives a
+// row segment of 64 PX pixels to SPLIT waves, wave s taking halos s, s + SPLIT, .. of the model (so that every
+// wave has its share of each type), and adds their sums through LDS in the order of the waves.
+//
 // Formulas (restated from the mathematics; reference equivalents cited):
 //   SIS gradient  src/gradient.cpp:260-299      PIEMD gradient  src/gradient.hpp:64-76,
 //   dPIE gradient src/gradient.cpp:744-809      PIEMD Hessian   src/gradient2.cpp:54-82, 92-205
@@ -16,12 +21,13 @@
 
 namespace lt {
 
-template <int PX, int KIND>
-__global__ __launch_bounds__(WAVE* ROWS) void k_hessian64(const HaloRec* __restrict__ halos,
+template <int PX, int KIND, int SPLIT>
+__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_hessian64(const HaloRec* __restrict__ halos,
                                                           const Run* __restrict__ runs, int nruns,
                                                           GridDesc g, OutDesc o)
 {
-    const int row = blockIdx.y * ROWS + threadIdx.y;
+    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
     if (row >= g.ny) return;
     halos = select_sample(g, halos, o);
     const int col0 = blockIdx.x * (WAVE * PX) + threadIdx.x;
@@ -40,14 +46,14 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_hessian64(const HaloRec* __restr
         const int end = run.start + run.count;
         switch (run.type) {
         case TYPE_DPIE:
-            for (int i = run.start; i < end; ++i) {
+            for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
                 const HaloRec& h = halos[i];
 #pragma unroll
                 for (int k = 0; k < PX; ++k) hess_piemd<true>(h, px[k], py, sT[k], sD[k], sB[k]);
             }
             break;
         case TYPE_PIEMD:
-            for (int i = run.start; i < end; ++i) {
+            for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
                 const HaloRec& h = halos[i];
 #pragma unroll
                 for (int k = 0; k < PX; ++k) hess_piemd<false>(h, px[k], py, sT[k], sD[k], sB[k]);
@@ -57,13 +63,13 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_hessian64(const HaloRec* __restr
             if (run.circ) {
                 // four halos per step: their records' scalar loads issue together, one wait per step
 #pragma unroll 4
-                for (int i = run.start; i < end; ++i) {
+                for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
                     const HaloRec& h = halos[i];
 #pragma unroll
                     for (int k = 0; k < PX; ++k) hess_sis_circ(h, px[k], py, sT[k], sD[k], sB[k]);
                 }
             } else {
-                for (int i = run.start; i < end; ++i) {
+                for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
                     const HaloRec& h = halos[i];
 #pragma unroll
                     for (int k = 0; k < PX; ++k) hess_sis(h, px[k], py, sT[k], sD[k], sB[k]);
@@ -71,7 +77,7 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_hessian64(const HaloRec* __restr
             }
             break;
         default:  // TYPE_SHEAR: constant lab-frame Hessian
-            for (int i = run.start; i < end; ++i) {
+            for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
                 const HaloRec& h = halos[i];
 #pragma unroll
                 for (int k = 0; k < PX; ++k) {
@@ -90,6 +96,16 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_hessian64(const HaloRec* __restr
             tB[k] = __builtin_fma(w, sB[k], tB[k]);
         }
     }
+    if constexpr (SPLIT > 1) {
+        if constexpr (KIND == LT_MAP_MASS) {
+            if (!split_sum<PX, SPLIT>(wave, tT)) return;
+        } else {
+            if (!split_sum<PX, SPLIT>(wave, tT, tD, tB)) return;
+        }
+        const int col = col0 + wave * WAVE;
+        if (col < g.nx) hess_epilogue<KIND>(o, (int64_t)row * g.pitch + col, tT[0], tD[0], tB[0]);
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
         const int col = col0 + k * WAVE;
@@ -97,12 +113,13 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_hessian64(const HaloRec* __restr
     }
 }
 
-template <int PX>
-__global__ __launch_bounds__(WAVE* ROWS) void k_gradient64(const HaloRec* __restrict__ halos,
+template <int PX, int SPLIT>
+__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_gradient64(const HaloRec* __restrict__ halos,
                                                            const Run* __restrict__ runs, int nruns,
                                                            GridDesc g, OutDesc o)
 {
-    const int row = blockIdx.y * ROWS + threadIdx.y;
+    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
     if (row >= g.ny) return;
     halos = select_sample(g, halos, o);
     const int col0 = blockIdx.x * (WAVE * PX) + threadIdx.x;
@@ -121,14 +138,14 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_gradient64(const HaloRec* __rest
         const int end = run.start + run.count;
         switch (run.type) {
         case TYPE_DPIE:
-            for (int i = run.start; i < end; ++i) {
+            for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
                 const HaloRec& h = halos[i];
 #pragma unroll
                 for (int k = 0; k < PX; ++k) grad_piemd<true>(h, px[k], py, sx[k], sy[k]);
             }
             break;
         case TYPE_PIEMD:
-            for (int i = run.start; i < end; ++i) {
+            for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
                 const HaloRec& h = halos[i];
 #pragma unroll
                 for (int k = 0; k < PX; ++k) grad_piemd<false>(h, px[k], py, sx[k], sy[k]);
@@ -138,13 +155,13 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_gradient64(const HaloRec* __rest
             if (run.circ) {
                 // four halos per step: their records' scalar loads issue together, one wait per step
 #pragma unroll 4
-                for (int i = run.start; i < end; ++i) {
+                for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
                     const HaloRec& h = halos[i];
 #pragma unroll
                     for (int k = 0; k < PX; ++k) grad_sis_circ(h, px[k], py, sx[k], sy[k]);
                 }
             } else {
-                for (int i = run.start; i < end; ++i) {
+                for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
                     const HaloRec& h = halos[i];
 #pragma unroll
                     for (int k = 0; k < PX; ++k) grad_sis(h, px[k], py, sx[k], sy[k]);
@@ -159,6 +176,16 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_gradient64(const HaloRec* __rest
         }
     }
     const double m = o.kind == LT_MAP_DPL ? o.r : 1.0;
+    if constexpr (SPLIT > 1) {
+        if (!split_sum<PX, SPLIT>(wave, tx, ty)) return;
+        const int col = col0 + wave * WAVE;
+        if (col < g.nx) {
+            const int64_t idx = (int64_t)row * g.pitch + col;
+            o.p0[idx] = tx[0] * m;
+            o.p1[idx] = ty[0] * m;
+        }
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
         const int col = col0 + k * WAVE;
@@ -170,12 +197,13 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_gradient64(const HaloRec* __rest
     }
 }
 
-template <int PX>
-__global__ __launch_bounds__(WAVE* ROWS) void k_potential64(const HaloRec* __restrict__ halos,
+template <int PX, int SPLIT>
+__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_potential64(const HaloRec* __restrict__ halos,
                                                             const Run* __restrict__ runs, int nruns,
                                                             GridDesc g, OutDesc o)
 {
-    const int row = blockIdx.y * ROWS + threadIdx.y;
+    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
     if (row >= g.ny) return;
     halos = select_sample(g, halos, o);
     const int col0 = blockIdx.x * (WAVE * PX) + threadIdx.x;
@@ -192,13 +220,23 @@ __global__ __launch_bounds__(WAVE* ROWS) void k_potential64(const HaloRec* __res
         double s[PX];
 #pragma unroll
         for (int k = 0; k < PX; ++k) s[k] = 0.;
-        for (int i = run.start; i < run.start + run.count; ++i) {
+        for (int i = first_halo<SPLIT>(run.start, wave); i < run.start + run.count; i += SPLIT) {
             const HaloRec& h = halos[i];
 #pragma unroll
             for (int k = 0; k < PX; ++k) s[k] += pot_halo(h, run.type, px[k], py, mn[k]);
         }
 #pragma unroll
         for (int k = 0; k < PX; ++k) tot[k] += s[k];
+    }
+    if constexpr (SPLIT > 1) {
+        // a wave that met a PIEMD centre makes the sum NaN
+#pragma unroll
+        for (int k = 0; k < PX; ++k)
+            if (mn[k] == 0.) tot[k] = __builtin_nan("");
+        if (!split_sum<PX, SPLIT>(wave, tot)) return;
+        const int col = col0 + wave * WAVE;
+        if (col < g.nx) o.p0[(int64_t)row * g.pitch + col] = tot[0] * o.mult;
+        return;
     }
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
@@ -265,17 +303,18 @@ __global__ __launch_bounds__(256) void k_epilogue(const double* __restrict__ a, 
 // ------------------------------------------------------------------------------------------------
 // launchers
 // ------------------------------------------------------------------------------------------------
-template <int PX>
+template <int PX, int SPLIT>
 static hipError_t launch_hessian64_px(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
                                       const OutDesc& o, hipStream_t s)
 {
-    dim3 blk(WAVE, ROWS, 1), grd = grid_for(g, PX);
+    dim3 blk, grd;
+    geometry<PX, SPLIT>(g, grd, blk);
     switch (o.kind) {
-    case LT_MAP_FIELDS: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_FIELDS>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
-    case LT_MAP_AMPLI: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_AMPLI>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
-    case LT_MAP_SHEAR: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_SHEAR>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
-    case LT_MAP_MASS: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_MASS>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
-    default: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_HESSIAN>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
+    case LT_MAP_FIELDS: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_FIELDS, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
+    case LT_MAP_AMPLI: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_AMPLI, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
+    case LT_MAP_SHEAR: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_SHEAR, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
+    case LT_MAP_MASS: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_MASS, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
+    default: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_HESSIAN, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
     }
     return hipGetLastError();
 }
@@ -284,9 +323,10 @@ hipError_t launch_hessian64(const HaloRec* halos, const Run* runs, int nruns, co
                             const OutDesc& o, int px, hipStream_t s)
 {
     switch (px) {
-    case 1: return launch_hessian64_px<1>(halos, runs, nruns, g, o, s);
-    case 4: return launch_hessian64_px<4>(halos, runs, nruns, g, o, s);
-    default: return launch_hessian64_px<2>(halos, runs, nruns, g, o, s);
+    case kPxSplit: return launch_hessian64_px<1, kSplit>(halos, runs, nruns, g, o, s);
+    case 1: return launch_hessian64_px<1, 1>(halos, runs, nruns, g, o, s);
+    case 4: return launch_hessian64_px<4, 1>(halos, runs, nruns, g, o, s);
+    default: return launch_hessian64_px<2, 1>(halos, runs, nruns, g, o, s);
     }
 }
 
@@ -315,26 +355,44 @@ hipError_t launch_points_gradient64(const HaloRec* halos, const Run* runs, int n
     return hipGetLastError();
 }
 
+template <int PX, int SPLIT>
+static void launch_gradient64_px(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g, const OutDesc& o,
+                           hipStream_t s)
+{
+    dim3 blk, grd;
+    geometry<PX, SPLIT>(g, grd, blk);
+    hipLaunchKernelGGL((k_gradient64<PX, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o);
+}
+
 hipError_t launch_gradient64(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
                              const OutDesc& o, int px, hipStream_t s)
 {
-    dim3 blk(WAVE, ROWS, 1);
     switch (px) {
-    case 1: hipLaunchKernelGGL(k_gradient64<1>, grid_for(g, 1), blk, 0, s, halos, runs, nruns, g, o); break;
-    case 4: hipLaunchKernelGGL(k_gradient64<4>, grid_for(g, 4), blk, 0, s, halos, runs, nruns, g, o); break;
-    default: hipLaunchKernelGGL(k_gradient64<2>, grid_for(g, 2), blk, 0, s, halos, runs, nruns, g, o); break;
+    case kPxSplit: launch_gradient64_px<1, kSplit>(halos, runs, nruns, g, o, s); break;
+    case 1: launch_gradient64_px<1, 1>(halos, runs, nruns, g, o, s); break;
+    case 4: launch_gradient64_px<4, 1>(halos, runs, nruns, g, o, s); break;
+    default: launch_gradient64_px<2, 1>(halos, runs, nruns, g, o, s); break;
     }
     return hipGetLastError();
+}
+
+template <int PX, int SPLIT>
+static void launch_potential64_px(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g, const OutDesc& o,
+                           hipStream_t s)
+{
+    dim3 blk, grd;
+    geometry<PX, SPLIT>(g, grd, blk);
+    hipLaunchKernelGGL((k_potential64<PX, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o);
 }
 
 hipError_t launch_potential64(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
                               const OutDesc& o, int px, hipStream_t s)
 {
-    dim3 blk(WAVE, ROWS, 1);
     switch (px) {
-    case 1: hipLaunchKernelGGL(k_potential64<1>, grid_for(g, 1), blk, 0, s, halos, runs, nruns, g, o); break;
-    case 4: hipLaunchKernelGGL(k_potential64<4>, grid_for(g, 4), blk, 0, s, halos, runs, nruns, g, o); break;
-    default: hipLaunchKernelGGL(k_potential64<2>, grid_for(g, 2), blk, 0, s, halos, runs, nruns, g, o); break;
+    case kPxSplit: launch_potential64_px<1, kSplit>(halos, runs, nruns, g, o, s); break;
+    case 1: launch_potential64_px<1, 1>(halos, runs, nruns, g, o, s); break;
+    case 4: launch_potential64_px<4, 1>(halos, runs, nruns, g, o, s); break;
+    default: launch_potential64_px<2, 1>(halos, runs, nruns, g, o, s); break;
     }
     return hipGetLastError();
 }

@@ -488,11 +488,58 @@ __device__ __forceinline__ const HaloRec* select_sample(const GridDesc& g, const
     return halos + s * g.halo_stride;
 }
 
+// this wave's halos of a run: first, first + SPLIT, ..
+template <int SPLIT>
+__device__ __forceinline__ int first_halo(int start, int wave)
+{
+    return SPLIT == 1 ? start : start + ((wave - start) & (SPLIT - 1));
+}
+
+// sums of PX pixels over the SPLIT waves of a row segment: wave k gets those of its k-th pixel column, in v[0]; false
+// for the waves that have none to store. Every wave of the work-group calls it.
+template <int PX, int SPLIT, typename... V>
+__device__ __forceinline__ bool split_sum(int wave, V&... v)
+{
+    __shared__ double part[SPLIT][sizeof...(V)][PX][WAVE];
+    const int lane = threadIdx.x;
+    int f = 0;
+    auto put = [&](const double* x) {
+#pragma unroll
+        for (int k = 0; k < PX; ++k) part[wave][f][k][lane] = x[k];
+        ++f;
+    };
+    (put(v), ...);
+    __syncthreads();
+    if (wave >= PX) return false;
+    f = 0;
+    auto get = [&](double* x) {
+        double t = part[0][f][wave][lane];
+#pragma unroll
+        for (int p = 1; p < SPLIT; ++p) t += part[p][f][wave][lane];
+        x[0] = t;
+        ++f;
+    };
+    (get(v), ...);
+    return true;
+}
+
 // Launch geometry: a 64 x 4 work-group, PX pixels per thread along a row, blockIdx.z = sample.
 inline dim3 grid_for(const GridDesc& g, int px)
 {
     return dim3((unsigned)((g.nx + WAVE * px - 1) / (WAVE * px)), (unsigned)((g.ny + ROWS - 1) / ROWS),
                 (unsigned)(g.nsamples > 0 ? g.nsamples : 1));
+}
+
+// waves of a row segment in the split form
+constexpr int kSplit = 8;
+
+// launch geometry: SPLIT 1 as grid_for(); else a work-group per row and 64 PX columns
+template <int PX, int SPLIT>
+inline void geometry(const GridDesc& g, dim3& grd, dim3& blk)
+{
+    grd = grid_for(g, PX);
+    blk = dim3(WAVE, SPLIT == 1 ? ROWS : SPLIT, 1);
+    if (SPLIT > 1) grd.y = (unsigned)g.ny;
 }
 
 }  // namespace lt
