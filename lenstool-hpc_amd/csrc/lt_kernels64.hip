@@ -248,43 +248,51 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_potential6
 }
 
 // Gradient at arbitrary points for a batch of lens models (blockIdx.y = sample), e.g. at the
-// observed images for the source barycentres. Same per-run accumulation as the grid kernel.
-__global__ __launch_bounds__(256) void k_points_gradient64(const HaloRec* __restrict__ halos,
-                                                           const Run* __restrict__ runs, int nruns,
-                                                           const double* __restrict__ px,
-                                                           const double* __restrict__ py, int npts,
-                                                           int64_t halo_stride, double* __restrict__ gx,
-                                                           double* __restrict__ gy)
+// observed images for the source barycentres: kSplit waves share the halos of 64 points, as in the split maps. Points
+// come by the thousand, and one wave per 64 of them walked all halos in a serial chain on a third of the SIMDs: 20000
+// points and 503 dPIE halos 290 us, now 78 (the 20M instructions' issue alone is 35; 313 work-groups on 256 CUs leave
+// the last ones two deep); 200000 points 25 us less of 720 with their copies, so no second form is kept. Parts of the
+// halos over several work-groups and a second kernel for their sum took 54 us here, but the call as a whole 23 more.
+__global__ __launch_bounds__(WAVE* kSplit) void k_points_gradient64(const HaloRec* __restrict__ halos,
+                                                                   const Run* __restrict__ runs, int nruns,
+                                                                   const double* __restrict__ px,
+                                                                   const double* __restrict__ py, int npts,
+                                                                   int64_t halo_stride, double* __restrict__ gx,
+                                                                   double* __restrict__ gy)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int i = blockIdx.x * WAVE + threadIdx.x;
     const int64_t s = blockIdx.y;
-    if (i >= npts) return;
     halos += s * halo_stride;
-    const double x = px[i], y = py[i];
-    double tx = 0., ty = 0.;
+    const int at = min(i, npts - 1);  // every lane takes part in the sums
+    const double x = px[at], y = py[at];
+    double tx[1] = {0.}, ty[1] = {0.};
     for (int r = 0; r < nruns; ++r) {
         const Run run = runs[r];
         double sx = 0., sy = 0.;
         const int end = run.start + run.count;
+        int h = first_halo<kSplit>(run.start, wave);
         switch (run.type) {
         case TYPE_DPIE:
-            for (int h = run.start; h < end; ++h) grad_piemd<true>(halos[h], x, y, sx, sy);
+            for (; h < end; h += kSplit) grad_piemd<true>(halos[h], x, y, sx, sy);
             break;
         case TYPE_PIEMD:
-            for (int h = run.start; h < end; ++h) grad_piemd<false>(halos[h], x, y, sx, sy);
+            for (; h < end; h += kSplit) grad_piemd<false>(halos[h], x, y, sx, sy);
             break;
         default:
             if (run.circ)
-                for (int h = run.start; h < end; ++h) grad_sis_circ(halos[h], x, y, sx, sy);
+                for (; h < end; h += kSplit) grad_sis_circ(halos[h], x, y, sx, sy);
             else
-                for (int h = run.start; h < end; ++h) grad_sis(halos[h], x, y, sx, sy);
+                for (; h < end; h += kSplit) grad_sis(halos[h], x, y, sx, sy);
             break;
         }
-        tx += sx;
-        ty += sy;
+        tx[0] += sx;
+        ty[0] += sy;
     }
-    gx[s * npts + i] = tx;
-    gy[s * npts + i] = ty;
+    if (!split_sum<1, kSplit>(wave, tx, ty) || i >= npts) return;
+    const int64_t o = s * npts + i;
+    gx[o] = tx[0];
+    gy[o] = ty[0];
 }
 
 // Epilogue alone, on Hessian planes already in device memory (the reference's map functions
@@ -347,11 +355,11 @@ hipError_t launch_epilogue64(const double* a, const double* b, const double* c, 
 }
 
 hipError_t launch_points_gradient64(const HaloRec* halos, const Run* runs, int nruns, const double* px,
-                                   const double* py, int npts, int nsamples, int64_t halo_stride, double* gx,
-                                   double* gy, hipStream_t s)
+                                    const double* py, int npts, int nsamples, int64_t halo_stride, double* gx,
+                                    double* gy, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_points_gradient64, dim3((npts + 255) / 256, nsamples), dim3(256), 0, s, halos, runs, nruns,
-                       px, py, npts, halo_stride, gx, gy);
+    hipLaunchKernelGGL(k_points_gradient64, dim3((npts + WAVE - 1) / WAVE, nsamples), dim3(WAVE, kSplit), 0, s, halos,
+                       runs, nruns, px, py, npts, halo_stride, gx, gy);
     return hipGetLastError();
 }
 

@@ -69,3 +69,17 @@ def test_split_maps(hip, oracle, n, nx, ny):
     m.close()
     np.testing.assert_array_equal(np.isnan(p32), ~fin)
     assert (np.abs(p32 - phi)[fin] <= 1e-5 * S[fin]).all()
+
+
+@pytest.mark.parametrize("n,npts", [(1, 1), (7, 64), (8, 65), (23, 63), (66, 129)])
+def test_split_points(hip, oracle, n, npts):
+    lens = _lens(n)
+    rng = np.random.default_rng(npts)
+    px, py = rng.uniform(-30, 30, npts), rng.uniform(-30, 30, npts)
+    print(f"[case] split points: {n} halos, {npts} points", flush=True)
+    gx, gy = hip.point_gradients(lens, px, py)
+    for i in range(npts):
+        e = oracle.point_gradient(lens, px[i], py[i], extended=True)
+        cg, _ = oracle.point_cond(lens, px[i], py[i])
+        tol = REL * (np.abs(np.array(e)).max() + 1.0) + EXT_SHARE * cg
+        assert abs(gx[i] - e[0]) <= tol and abs(gy[i] - e[1]) <= tol, i
