@@ -74,6 +74,7 @@ int batch_alloc(lt_chi_batch_s* b, const int* nimages, const lt_galaxy* images)
     size_t o_igx = c.take<double>(S * I), o_igy = c.take<double>(S * I);
     size_t o_sx = c.take<double>(S * K), o_sy = c.take<double>(S * K), o_sdr = c.take<double>(S * K);
     size_t o_sb = c.take<double>(S * 3);
+    size_t o_items = c.take<ScanItem>(S * (size_t)scan_items(b->n, b->nsets)), o_nitems = c.take<int32_t>(S);
     size_t o_cnt = c.take<int32_t>(S * K), o_hits = c.take<int32_t>(S * K * DELENSE_CAP);
     size_t o_px = c.take<double>(S * K * LT_MAXIMPERSOURCE), o_py = c.take<double>(S * K * LT_MAXIMPERSOURCE);
     size_t o_loc = c.take<int32_t>(S * K), o_st = c.take<int32_t>(S), o_terms = c.take<double>(S * I);
@@ -110,6 +111,8 @@ int batch_alloc(lt_chi_batch_s* b, const int* nimages, const lt_galaxy* images)
     d.src_y = (double*)(p + o_sy);
     d.src_dr = (double*)(p + o_sdr);
     d.src_bound = (double*)(p + o_sb);
+    d.items = (ScanItem*)(p + o_items);
+    d.nitems = (int32_t*)(p + o_nitems);
     d.count = (int32_t*)(p + o_cnt);
     d.hits = (int32_t*)(p + o_hits);
     d.pos_x = (double*)(p + o_px);
@@ -138,13 +141,6 @@ int batch_alloc(lt_chi_batch_s* b, const int* nimages, const lt_galaxy* images)
         LT_HIP_TRY(hipMemcpy((void*)d.img_y, iy.data(), I * sizeof(double), hipMemcpyHostToDevice));
         LT_HIP_TRY(hipMemcpy((void*)d.img_dr, idr.data(), I * sizeof(double), hipMemcpyHostToDevice));
     }
-    return LT_OK;
-}
-
-int reset_counters(lt_chi_batch_s* b, hipStream_t s)
-{
-    LT_HIP_TRY(launch_fill_i32(b->d.count, 0, (size_t)b->S * b->nsets, s));
-    LT_HIP_TRY(launch_fill_i32(b->d.status, 0, (size_t)b->S, s));
     return LT_OK;
 }
 
@@ -256,8 +252,7 @@ int lt_chi_batch_run(lt_chi_batch b, const lt_potential_soa* lenses, double* chi
     }
     if (!b->runs.empty())
         LT_HIP_TRY(hipMemcpyAsync(b->druns, b->runs.data(), b->runs.size() * sizeof(Run), hipMemcpyHostToDevice, s));
-    int st = reset_counters(b, s);
-    if (st) return st;
+    int st;
     // gradient grids of every sample (src/chi_CPU_barycenter.cpp:125-137), launched per chunk of samples
     // as soon as the chunk is packed, so that the host packs the next chunk while the device computes
     GridDesc g{};
@@ -365,8 +360,6 @@ int lt_delense_barycenter(lt_point* image_pos, int* locimagesfound, int* numimg,
     if (e == hipSuccess) e = hipMemcpy(b.d.src_x, sx.data(), nsets * sizeof(double), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(b.d.src_y, sy.data(), nsets * sizeof(double), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(b.d.src_dr, sdr.data(), nsets * sizeof(double), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = launch_fill_i32(b.d.count, 0, nsets, nullptr);
-    if (e == hipSuccess) e = launch_fill_i32(b.d.status, 0, 1, nullptr);
     if (e == hipSuccess) e = launch_delense(b.gx, b.gy, b.d, nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e == hipSuccess) e = hipMemcpy(cnt.data(), b.d.count, nsets * sizeof(int), hipMemcpyDeviceToHost);

@@ -12,6 +12,24 @@ namespace lt {
 // LT_MAXIMPERSOURCE of them are reported, more than that is flagged LT_ERR_OVERFLOW
 constexpr int DELENSE_CAP = 64;
 
+// Tiles of cells that the delensing scan leaves open for some of 64 sources (lt_delense.hip).
+constexpr int SCAN_TILE = 8;    // cells of a tile's side
+constexpr int SCAN_CHUNK = 64;  // sources of an item
+
+struct alignas(16) ScanItem {
+    uint64_t open;   // bit 8 j + i: source 8 i + j of the chunk
+    int32_t tile;    // row-major
+    int32_t chunk;   // 2 * chunk, + 1 when every triangle of the tile has its determinant bounded away from 0
+};
+
+__host__ __device__ inline int scan_tiles(int n) { return (n - 1 + SCAN_TILE - 1) / SCAN_TILE; }
+
+// items of a sample at most: one per tile and chunk
+__host__ __device__ inline int64_t scan_items(int n, int nsets)
+{
+    return (int64_t)scan_tiles(n) * scan_tiles(n) * ((nsets + SCAN_CHUNK - 1) / SCAN_CHUNK);
+}
+
 struct DelenseDesc {
     int32_t n;            // delensing grid is n x n pixels, (n-1)^2 cells
     int32_t nsets;        // image families (sources)
@@ -28,6 +46,8 @@ struct DelenseDesc {
     double* src_y;
     double* src_dr;
     double* src_bound;           // [nsamples*3] max |x|, |y|, min dr, max dr of the sample's sources
+    ScanItem* items;             // [nsamples*scan_items()] open tiles
+    int32_t* nitems;             // [nsamples] how many
     int32_t* count;              // [nsamples*nsets] hits found
     int32_t* hits;               // [nsamples*nsets*DELENSE_CAP] cell*2 + (lower triangle)
     double* pos_x;               // [nsamples*nsets*LT_MAXIMPERSOURCE] image barycentres

@@ -11,9 +11,12 @@
 // path. Hits are collected with atomics and then put back into scan order by a per-source sort.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "lenstool_hip/lt_status.h"
 #include "lt_delense.h"
 #include "lt_delense_geom.h"
+#include "lt_delense_tile.h"
 #include "lt_device.h"
 #include "lt_math.h"
 
@@ -68,26 +71,35 @@ __device__ __forceinline__ CellCorners load_corners(const double* __restrict__ g
 
 // ------------------------------------------------------------------------------------------------
 // per-sample bounds of the sources for the scan's cull: max |x|, |y| and the range of D_ls/D_s; a
-// non-finite source makes the bounds NaN, which switches the cull off for the whole sample
+// non-finite source makes the bounds NaN, which switches the cull off for the whole sample. One wavefront per
+// sample, which also clears the sample's counters.
 // ------------------------------------------------------------------------------------------------
-__global__ void k_source_bounds(DelenseDesc d)
+__global__ __launch_bounds__(64) void k_source_bounds(DelenseDesc d)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= d.nsamples) return;
-    double pmax = 0., lo = 0., hi = 0., sum = 0.;  // NaN and infinity reach the sum (fmin/fmax drop NaN)
-    for (int k = 0; k < d.nsets; ++k) {
+    const int s = blockIdx.x, lane = threadIdx.x;
+    double pmax = 0., lo = __builtin_inf(), hi = -__builtin_inf();
+    bool finite = true;  // fmin / fmax drop NaN
+    for (int k = lane; k < d.nsets; k += 64) {
         const int64_t sk = (int64_t)s * d.nsets + k;
         const double x = fabs(d.src_x[sk]), y = fabs(d.src_y[sk]), r = d.src_dr[sk];
-        sum += x + y + fabs(r);
+        finite = finite && x <= 1e100 && y <= 1e100 && fabs(r) <= 1e100;
         pmax = fmax(pmax, fmax(x, y));
-        lo = k ? fmin(lo, r) : r;
-        hi = k ? fmax(hi, r) : r;
+        lo = fmin(lo, r);
+        hi = fmax(hi, r);
+        d.count[sk] = 0;
     }
-    const bool finite = sum <= 1e300 && pmax <= 1e100 && fabs(lo) <= 1e100 && fabs(hi) <= 1e100;
-    const double nan = __builtin_nan("");
-    d.src_bound[3 * (int64_t)s] = finite ? pmax : nan;
-    d.src_bound[3 * (int64_t)s + 1] = finite ? lo : nan;
-    d.src_bound[3 * (int64_t)s + 2] = finite ? hi : nan;
+    finite = __ballot(!finite) == 0;
+    pmax = wave_max64(pmax);
+    lo = -wave_max64(-lo);
+    hi = wave_max64(hi);
+    if (lane == 0) {
+        const double nan = __builtin_nan("");
+        d.src_bound[3 * (int64_t)s] = finite ? pmax : nan;
+        d.src_bound[3 * (int64_t)s + 1] = finite ? lo : nan;
+        d.src_bound[3 * (int64_t)s + 2] = finite ? hi : nan;
+        d.nitems[s] = 0;
+        d.status[s] = 0;
+    }
 }
 
 // append a hit of source k of sample s in cell `cell` (0 = none, 1 upper, 2 lower triangle)
@@ -100,137 +112,186 @@ __device__ __forceinline__ void record_hit(const DelenseDesc& d, int s, int k, i
 }
 
 // ------------------------------------------------------------------------------------------------
-// delensing scan: one thread per (cell, sample), a wavefront per 8 x 8 tile of cells, all sources
-// (staged in LDS, SCAN_BLOCK per pass); hits appended per (sample, source)
+// delensing scan: a wavefront takes 64 columns of 8 rows of cells, eight tiles of 8 x 8. Each lane walks
+// down its column with the vertices on both sides of it, mapped to the source plane at both ends of the
+// sample's D_ls/D_s range, and keeps their box and the range of the cells' determinants; eight lanes'
+// make a tile (lt_delense_tile.h), which its lanes test against the sources, staged in LDS. Only
+// (tile, source) pairs that the test leaves open go through the reference's triangle test, in k_delense_open: a
+// wavefront's lanes take the 64 cells of the tile; tiles with a cell near a critical line (or values that are not
+// finite) take each cell's own bounds on the determinant (lt_delense_geom.h).
+// Bound by reading the planes: 1024 samples of 512 x 512 pixels in 1.31 ms, 3.7 TB/s with the rows that two
+// wavefronts share, and about 70 VALU instructions per row of 64 cells. With a cell a lane, each bounding its own
+// corners' distances and determinants, 300 of set-up per 64 cells took 4.18 ms. 152 registers, three wavefronts a
+// SIMD, hold the nine rows' loads in flight; held to 128 it spills and takes 1.41 ms.
 // ------------------------------------------------------------------------------------------------
-constexpr int SCAN_BLOCK = 256;  // threads per block (4 wavefronts: 16 x 16 cells); also the sources staged in LDS per pass
-constexpr int SCAN_SIDE = 16;    // cells per block side
-constexpr int SCAN_UNROLL = 4;   // sources culled per step of the per-cell scan loop
-constexpr int WAVE_SIZE = 64;
-static_assert(SCAN_BLOCK == 4 * WAVE_SIZE && SCAN_SIDE == 16, "four wavefronts of 8 x 8 cells per block");
+constexpr int SCAN_BLOCK = 256;  // threads per block (4 wavefronts: 64 x 32 cells); also the sources staged in LDS per pass
+constexpr int SCAN_WAVES = SCAN_BLOCK / 64;
 
-// One pass over cnt staged sources. SCAN_UNROLL sources per step: one margin (the smallest of their
-// culls) decides the step in straight-line code; the reference test runs only where a cull fails (a
-// few cells around each image, degenerate or non-finite cells), one source at a time. RHO_ONLY: every
-// lane's cell has d_ok (or is past the row end), so the margin needs only the distance.
-template <bool RHO_ONLY>
-__device__ __forceinline__ void scan_pass(const DelenseDesc& d, const CellCorners& c, const CellFilter& f,
-                                          const CellFilter32& f32, bool active, int s, int k0, int cell, int cnt,
-                                          const double* lsx, const double* lsy, const double* ldr, const float* lsx32,
-                                          const float* lsy32, const float* ldr32)
+// smallest / largest value over the eight lanes of a tile, in each of them
+__device__ __forceinline__ double tile_min(double v)
 {
-    int j0 = 0;
-    for (; j0 + SCAN_UNROLL <= cnt; j0 += SCAN_UNROLL) {
-        if constexpr (RHO_ONLY) {
-            // FP32 pre-test of the step (lt_delense_geom.h cell_filter32): sound on its own, and it decides
-            // nearly every step; the FP64 margin below runs only where it does not
-            float mg32 = far_margin_rho32(f32, lsx32[j0], lsy32[j0], ldr32[j0]);
-#pragma unroll
-            for (int u = 1; u < SCAN_UNROLL; ++u)
-                mg32 = __builtin_fminf(mg32, far_margin_rho32(f32, lsx32[j0 + u], lsy32[j0 + u], ldr32[j0 + u]));
-            if (!active | (mg32 > 0.f)) continue;
-        }
-        double mg = RHO_ONLY ? far_margin_rho(f, c, lsx[j0], lsy[j0], ldr[j0]) : far_margin(f, c, lsx[j0], lsy[j0], ldr[j0]);
-#pragma unroll
-        for (int u = 1; u < SCAN_UNROLL; ++u)
-            mg = fmin(mg, RHO_ONLY ? far_margin_rho(f, c, lsx[j0 + u], lsy[j0 + u], ldr[j0 + u])
-                                   : far_margin(f, c, lsx[j0 + u], lsy[j0 + u], ldr[j0 + u]));
-        if (!active | (f.on & (mg > 0.))) continue;
-#pragma unroll 1
-        for (int j = j0; j < j0 + SCAN_UNROLL; ++j)
-            if (!far_from_cell(f, c, lsx[j], lsy[j], ldr[j])) record_hit(d, s, k0 + j, cell, cell_hit(c, lsx[j], lsy[j], ldr[j]));
-    }
-#pragma unroll 1
-    for (; j0 < cnt; ++j0)
-        if (active && !far_from_cell(f, c, lsx[j0], lsy[j0], ldr[j0]))
-            record_hit(d, s, k0 + j0, cell, cell_hit(c, lsx[j0], lsy[j0], ldr[j0]));
+    v = __builtin_fmin(v, dpp_move64<0xB1>(v));     // quad_perm [1, 0, 3, 2]
+    v = __builtin_fmin(v, dpp_move64<0x4E>(v));     // quad_perm [2, 3, 0, 1]
+    return __builtin_fmin(v, dpp_move64<0x141>(v));  // row_half_mirror
 }
 
+__device__ __forceinline__ double tile_max(double v) { return -tile_min(-v); }
 
-
-// One pass over cnt staged sources with the tile pre-test (lt_delense_geom.h tile_filter32): lane j
-// tests source kc + j against the whole tile, and only the sources it keeps (few: those whose image lies
-// on or next to the tile) go through the per-cell tests, one source at a time for all cells.
-__device__ __forceinline__ void scan_tile(const DelenseDesc& d, const CellCorners& c, const CellFilter& f,
-                                          const CellFilter32& f32, const CellFilter32& tf, bool active, int s, int k0,
-                                          int cell, int cnt, const double* lsx, const double* lsy, const double* ldr,
-                                          const float* lsx32, const float* lsy32, const float* ldr32)
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_or(uint32_t v)
 {
-    const int lane = (int)threadIdx.x & (WAVE_SIZE - 1);
-    for (int kc = 0; kc < cnt; kc += WAVE_SIZE) {
-        const int j = kc + lane;  // < SCAN_BLOCK: kc < cnt <= SCAN_BLOCK is a multiple of the wavefront size
-        const float mg = j < cnt ? far_margin_rho32(tf, lsx32[j], lsy32[j], ldr32[j]) : 1.f;
-        unsigned long long keep = __ballot(!(mg > 0.f));
-        while (keep) {
-            const int jj = kc + __builtin_ctzll(keep);
-            keep &= keep - 1;
-            if (active && !(far_margin_rho32(f32, lsx32[jj], lsy32[jj], ldr32[jj]) > 0.f) &&
-                !far_from_cell(f, c, lsx[jj], lsy[jj], ldr[jj]))
-                record_hit(d, s, k0 + jj, cell, cell_hit(c, lsx[jj], lsy[jj], ldr[jj]));
-        }
-    }
+    return v | (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
+}
+
+__device__ __forceinline__ uint64_t tile_or(uint64_t v)
+{
+    const uint32_t lo = dpp_or<0x141>(dpp_or<0x4E>(dpp_or<0xB1>((uint32_t)v)));
+    const uint32_t hi = dpp_or<0x141>(dpp_or<0x4E>(dpp_or<0xB1>((uint32_t)(v >> 32))));
+    return ((uint64_t)hi << 32) | lo;
 }
 
 __global__ __launch_bounds__(SCAN_BLOCK) void k_delense(const double* __restrict__ gx, const double* __restrict__ gy,
                                                         DelenseDesc d)
 {
-    __shared__ double lsx[SCAN_BLOCK], lsy[SCAN_BLOCK], ldr[SCAN_BLOCK];
-    __shared__ float lsx32[SCAN_BLOCK], lsy32[SCAN_BLOCK], ldr32[SCAN_BLOCK];
+    __shared__ double lsx[SCAN_BLOCK], lsy[SCAN_BLOCK], lst[SCAN_BLOCK];
     const int n = d.n;
-    const int lane = (int)threadIdx.x & (WAVE_SIZE - 1), wv = (int)threadIdx.x / WAVE_SIZE;
-    const int xid = blockIdx.x * SCAN_SIDE + (wv & 1) * 8 + (lane & 7);
-    const int yid = blockIdx.y * SCAN_SIDE + (wv >> 1) * 8 + (lane >> 3);
+    const int lane = (int)threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int s = blockIdx.z;
-    const bool active = xid < n - 1 && yid < n - 1;
-    const int64_t base = (int64_t)s * d.grid_stride;
-    const int cell = yid * (n - 1) + xid;
-    // the first pass's sources, loaded before the cell set-up so that their latency overlaps it
-    const int cnt0 = min(SCAN_BLOCK, d.nsets);
-    double sx0 = 0., sy0 = 0., sdr0 = 0.;
-    if ((int)threadIdx.x < cnt0) {
-        const int64_t sk = (int64_t)s * d.nsets + threadIdx.x;
-        sx0 = d.src_x[sk];
-        sy0 = d.src_y[sk];
-        sdr0 = d.src_dr[sk];
-    }
-    // lanes past the grid read the last cell of their row or column (in bounds) and record nothing
-    const CellCorners c = load_corners(gx + base, gy + base, d, min(xid, n - 2), min(yid, n - 2));
+    const int x0 = blockIdx.x * 64, y0 = (blockIdx.y * SCAN_WAVES + wv) * SCAN_TILE;
+    const bool rows = y0 < n - 1;  // a wavefront past the grid only stages sources
+    const double* const px = gx + (int64_t)s * d.grid_stride;
+    const double* const py = gy + (int64_t)s * d.grid_stride;
     const double* sb = d.src_bound + 3 * (int64_t)s;
-    const CellFilter f = cell_filter(c, sb[0], sb[1], sb[2]);
-    const CellFilter32 f32 = cell_filter32(f, c);
-    const unsigned long long act = __ballot(active);
-    const bool rho_only = __all(!active || f.d_ok);  // uniform over the wavefront
-    // the tile pre-test when every active cell has d_ok: bounds about the cell at the tile's centre
-    // (lane 36, cell (4, 4) of the tile) when it is in the grid, else the first active lane's
-    CellFilter32 tf = f32;
-    tf.rf2 = __builtin_inff();
-    if (rho_only && act) {
-        const int r = ((act >> 36) & 1ull) ? 36 : __builtin_ctzll(act);
-        const double xr = read_lane64(c.xp, r), yr = read_lane64(c.yp, r), gxr = read_lane64(c.g0x, r),
-                     gyr = read_lane64(c.g0y, r);
-        const double drmax = __builtin_fmax(__builtin_fabs(sb[1]), __builtin_fabs(sb[2]));
-        const double t = active ? tile_reach(f, c, xr, yr, gxr, gyr, drmax) : 0.;
-        tf = tile_filter32(xr, yr, gxr, gyr, wave_max64(t), read_lane64(f.m, r), true);
+    const double pmax = sb[0], lo = sb[1], hi = sb[2];
+
+    TileTest tt = {};
+    if (rows) {
+        const int xid = min(x0 + lane, n - 2);  // lanes past the grid repeat its last column
+        const int ncells = min(SCAN_TILE, n - 1 - y0);
+        const double xa = d.xmin + xid * d.dx, xb = xa + d.dx;
+        double ga[SCAN_TILE + 1][4];
+#pragma unroll
+        for (int k = 0; k <= SCAN_TILE; ++k) {
+            const int64_t at = (int64_t)min(y0 + k, n - 1) * n + xid;
+            ga[k][0] = px[at];
+            ga[k][1] = py[at];
+            ga[k][2] = px[at + 1];
+            ga[k][3] = py[at + 1];
+        }
+        TileBound t = empty_tile();
+        Vertex2 a, b, top;
+#pragma unroll
+        for (int k = 0; k <= SCAN_TILE; ++k) {
+            if (k > ncells) continue;
+            const double y = d.ymin + (y0 + k) * d.dy;
+            const Vertex2 na = map_vertex(xa, y, ga[k][0], ga[k][1], lo, hi), nb = map_vertex(xb, y, ga[k][2], ga[k][3], lo, hi);
+            const Vertex2 bottom = edge(na, nb);
+            add_vertices(t, na, nb);
+            if (k) {
+                add_triangle(t, edge(a, na), top);
+                add_triangle(t, edge(b, nb), bottom);
+            }
+            a = na;
+            b = nb;
+            top = bottom;
+        }
+        const uint64_t fin = __ballot(__builtin_fabs(t.sum) <= 1e100);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            t.lo[k] = tile_min(t.lo[k]);
+            t.hi[k] = tile_max(t.hi[k]);
+        }
+        t.dmin = tile_min(t.dmin);
+        t.dmax = tile_max(t.dmax);
+        const double ya = d.ymin + y0 * d.dy, yb = d.ymin + (y0 + ncells) * d.dy;
+        const double pix = tile_max(__builtin_fmax(__builtin_fmax(__builtin_fabs(xa), __builtin_fabs(xb)),
+                                                   __builtin_fmax(__builtin_fabs(ya), __builtin_fabs(yb))));
+        tt = tile_test(t, pix, pmax, ((fin >> (lane & 56)) & 0xff) == 0xff);
     }
-    const bool tile = tf.rf2 < __builtin_inff();  // uniform over the wavefront
+    const bool inside = rows && x0 + (lane & 56) < n - 1;  // a tile of the grid
+    const int64_t cap = scan_items(n, d.nsets);
+
     for (int k0 = 0; k0 < d.nsets; k0 += SCAN_BLOCK) {
         const int cnt = min(SCAN_BLOCK, d.nsets - k0);
         __syncthreads();  // the previous pass is done with the staged sources
         if ((int)threadIdx.x < cnt) {
             const int64_t sk = (int64_t)s * d.nsets + k0 + threadIdx.x;
-            const double sx = k0 ? d.src_x[sk] : sx0, sy = k0 ? d.src_y[sk] : sy0, sdr = k0 ? d.src_dr[sk] : sdr0;
-            lsx[threadIdx.x] = sx;
-            lsy[threadIdx.x] = sy;
-            ldr[threadIdx.x] = sdr;
-            lsx32[threadIdx.x] = (float)sx;
-            lsy32[threadIdx.x] = (float)sy;
-            ldr32[threadIdx.x] = (float)sdr;
+            lsx[threadIdx.x] = d.src_x[sk];
+            lsy[threadIdx.x] = d.src_y[sk];
+            lst[threadIdx.x] = range_share(d.src_dr[sk], lo, hi);
         }
         __syncthreads();
-        if (!act) continue;  // a wavefront past the grid: nothing to scan (it still stages and syncs)
-        if (tile) scan_tile(d, c, f, f32, tf, active, s, k0, cell, cnt, lsx, lsy, ldr, lsx32, lsy32, ldr32);
-        else if (rho_only) scan_pass<true>(d, c, f, f32, active, s, k0, cell, cnt, lsx, lsy, ldr, lsx32, lsy32, ldr32);
-        else scan_pass<false>(d, c, f, f32, active, s, k0, cell, cnt, lsx, lsy, ldr, lsx32, lsy32, ldr32);
+        if (!rows) continue;
+        for (int c0 = 0; c0 < cnt; c0 += SCAN_CHUNK) {
+            // lane j of a tile tests sources j, j + 8, ..: bit 8 j + i of the tile's word is source 8 i + j
+            uint32_t bits = 0;
+            const int most = min(SCAN_CHUNK, cnt - c0);
+            for (int i = 0; i * SCAN_TILE < most; ++i) {
+                const int j = i * SCAN_TILE + (lane & 7), at = c0 + min(j, most - 1);
+                const bool miss = tt.boxed && box_margin(tt, lsx[at], lsy[at], lst[at]) > 0.;
+                if (j < most && !miss) bits |= 1u << i;
+            }
+            const uint64_t open = tile_or((uint64_t)bits << (8 * (lane & 7)));
+            const bool item = inside && (lane & 7) == 0 && (open || !tt.det_ok);
+            const uint64_t all = __ballot(item);
+            if (!all) continue;
+            int base = 0;
+            if (lane == 0) base = atomicAdd(&d.nitems[s], __builtin_popcountll(all));
+            base = __builtin_amdgcn_readfirstlane(base);
+            if (item) {
+                ScanItem it;
+                it.open = open;
+                it.tile = (y0 / SCAN_TILE) * scan_tiles(n) + (x0 + lane) / SCAN_TILE;
+                it.chunk = ((k0 + c0) / SCAN_CHUNK) * 2 + (tt.det_ok ? 1 : 0);
+                d.items[s * cap + base + __builtin_popcountll(all & ((1ull << lane) - 1))] = it;
+            }
+        }
+    }
+}
+
+// The tiles that k_delense left open, one wavefront per tile and 64 sources, a lane per cell. In a kernel of their
+// own: they lie along the critical lines and around the images, and a wavefront of the scan that met eight of them
+// took longer than all others together (both in one kernel: 45 us for one sample of 40 sources on 512 x 512, 3561 for
+// 1024; apart 7 + 10 and 1312 + 773). Bound by the cells' set-up along the critical lines.
+__global__ __launch_bounds__(SCAN_BLOCK) void k_delense_open(const double* __restrict__ gx, const double* __restrict__ gy,
+                                                             DelenseDesc d)
+{
+    const int n = d.n;
+    const int s = blockIdx.y;
+    const int lane = (int)threadIdx.x & 63;
+    const int64_t cap = scan_items(n, d.nsets);
+    const int nitems = d.nitems[s], step = (int)gridDim.x * SCAN_WAVES;
+    const double* sb = d.src_bound + 3 * (int64_t)s;
+    for (int i = blockIdx.x * SCAN_WAVES + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); i < nitems; i += step) {
+        const ScanItem it = d.items[s * cap + i];
+        const int xid = (it.tile % scan_tiles(n)) * SCAN_TILE + (lane & 7), yid = (it.tile / scan_tiles(n)) * SCAN_TILE + (lane >> 3);
+        const bool active = xid < n - 1 && yid < n - 1;
+        const int cell = yid * (n - 1) + xid;
+        const CellCorners c = load_corners(gx + (int64_t)s * d.grid_stride, gy + (int64_t)s * d.grid_stride, d, min(xid, n - 2), min(yid, n - 2));
+        const int k0 = (it.chunk >> 1) * SCAN_CHUNK;
+        const int64_t s0 = (int64_t)s * d.nsets + k0;
+        // the chunk's sources, one a lane: taken from there without a wait on memory
+        const int64_t mine = s0 + min(lane, min(SCAN_CHUNK, d.nsets - k0) - 1);
+        const double lx = d.src_x[mine], ly = d.src_y[mine], ldr = d.src_dr[mine];
+        if (it.chunk & 1) {
+            uint64_t open = it.open;
+            while (open) {
+                const int p = __builtin_ctzll(open), k = (p & 7) * 8 + (p >> 3);
+                open &= open - 1;
+                if (active) record_hit(d, s, k0 + k, cell, cell_hit(c, read_lane64(lx, k), read_lane64(ly, k), read_lane64(ldr, k)));
+            }
+            continue;
+        }
+        const CellFilter f = cell_filter(c, sb[0], sb[1], sb[2]);
+        for (int k = 0; k < min(SCAN_CHUNK, d.nsets - k0); ++k) {
+            // outside the tile's box a cell needs its own determinants only
+            const double sx = read_lane64(lx, k), sy = read_lane64(ly, k), dr = read_lane64(ldr, k);
+            const double du = __builtin_fma(dr, __builtin_fma(dr, f.c2u, f.c1u), f.c0);
+            const double dl = __builtin_fma(dr, __builtin_fma(dr, f.c2l, f.c1l), f.c0);
+            const bool out = !((it.open >> ((k & 7) * 8 + (k >> 3))) & 1);
+            const bool miss = out & f.on & (__builtin_fmin(abs_d(du), abs_d(dl)) > f.tau);
+            if (active && !miss && !far_from_cell(f, c, sx, sy, dr)) record_hit(d, s, k0 + k, cell, cell_hit(c, sx, sy, dr));
+        }
     }
 }
 
@@ -294,8 +355,9 @@ __global__ void k_delense_finish(const double* __restrict__ gx, const double* __
 
 // ------------------------------------------------------------------------------------------------
 // chi^2 matching (src/chi_computation.cpp:10-195, with its two early-stopping loop conditions at
-// :110 and :118): one thread per (sample, source) writes the per-image chi terms; one thread per
-// sample then sums them in the reference's order.
+// :110 and :118): a wavefront per sample, a lane per source writes the per-image chi terms; the wavefront
+// then sums them in the reference's order, 64 terms loaded at a time (one thread that loaded each as it
+// summed took 15 us for a sample of 120 images, 36 for 1024 samples).
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ double pdist(double ax, double ay, double bx, double by)
 {
@@ -304,12 +366,9 @@ __device__ __forceinline__ double pdist(double ax, double ay, double bx, double 
     return sqrt(x * x + y * y);
 }
 
-__global__ void k_chi_match(DelenseDesc d)
+__device__ __forceinline__ void chi_match(const DelenseDesc& d, int s, int k)
 {
 #pragma clang fp contract(off)
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = blockIdx.y;
-    if (k >= d.nsets) return;
     const int64_t sk = (int64_t)s * d.nsets + k;
     const int first = d.first_image[k], ni = d.nimages[k];
     int nfound[LT_MAXIMPERSOURCE];
@@ -369,17 +428,29 @@ __global__ void k_chi_match(DelenseDesc d)
     }
 }
 
-__global__ void k_chi_reduce(DelenseDesc d)
+__global__ __launch_bounds__(64) void k_chi(DelenseDesc d)
 {
 #pragma clang fp contract(off)
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= d.nsamples) return;
-    double chi = 0.;
+    const int s = blockIdx.x, lane = threadIdx.x;
     int found = 0;
-    for (int k = 0; k < d.nsets; ++k) found += d.loc[(int64_t)s * d.nsets + k];
-    for (int i = 0; i < d.nimg_total; ++i) chi += d.terms[(int64_t)s * d.nimg_total + i];
-    d.chi[s] = chi;
-    d.found[s] = found;
+    for (int k = lane; k < d.nsets; k += 64) {
+        chi_match(d, s, k);
+        found += d.loc[(int64_t)s * d.nsets + k];
+    }
+    __syncthreads();  // the terms are written
+    const double* const terms = d.terms + (int64_t)s * d.nimg_total;
+    double chi = 0.;
+    for (int i = 0; i < d.nimg_total; i += 64) {
+        const int n = min(64, d.nimg_total - i);
+        const double t = terms[i + min(lane, n - 1)];
+        for (int j = 0; j < n; ++j) chi += read_lane64(t, j);
+    }
+#pragma unroll
+    for (int m = 32; m; m >>= 1) found += __shfl_xor(found, m);
+    if (lane == 0) {
+        d.chi[s] = chi;
+        d.found[s] = found;
+    }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -393,13 +464,19 @@ hipError_t launch_barycentres(const double* img_gx, const double* img_gy, const 
 
 hipError_t launch_delense(const double* gx, const double* gy, const DelenseDesc& d, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_source_bounds, dim3((d.nsamples + 63) / 64), dim3(64), 0, s, d);
+    hipLaunchKernelGGL(k_source_bounds, dim3((unsigned)d.nsamples), dim3(64), 0, s, d);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     dim3 blk(SCAN_BLOCK);
-    dim3 grd((unsigned)((d.n - 1 + SCAN_SIDE - 1) / SCAN_SIDE), (unsigned)((d.n - 1 + SCAN_SIDE - 1) / SCAN_SIDE),
-             (unsigned)d.nsamples);
+    constexpr int rows = SCAN_WAVES * SCAN_TILE;
+    dim3 grd((unsigned)((d.n - 1 + 63) / 64), (unsigned)((d.n - 1 + rows - 1) / rows), (unsigned)d.nsamples);
     hipLaunchKernelGGL(k_delense, grd, blk, 0, s, gx, gy, d);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    // open tiles: about 4096 work-groups over the samples, at most 256 (as many tiles as 512 x 512 pixels leave) and at
+    // least 8 of them for a sample
+    const int groups = std::min(256, std::max(8, 4096 / d.nsamples));
+    hipLaunchKernelGGL(k_delense_open, dim3((unsigned)groups, (unsigned)d.nsamples), blk, 0, s, gx, gy, d);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_delense_finish, dim3((d.nsets + 63) / 64, d.nsamples), dim3(64), 0, s, gx, gy, d);
@@ -408,10 +485,7 @@ hipError_t launch_delense(const double* gx, const double* gy, const DelenseDesc&
 
 hipError_t launch_chi(const DelenseDesc& d, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_chi_match, dim3((d.nsets + 63) / 64, d.nsamples), dim3(64), 0, s, d);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_chi_reduce, dim3((d.nsamples + 63) / 64), dim3(64), 0, s, d);
+    hipLaunchKernelGGL(k_chi, dim3((unsigned)d.nsamples), dim3(64), 0, s, d);
     return hipGetLastError();
 }
 

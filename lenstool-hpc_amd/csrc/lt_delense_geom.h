@@ -232,6 +232,8 @@ __host__ __device__ inline float far_margin_rho32(const CellFilter32& g, float p
     return __builtin_fmaf(ex, ex, ey * ey) - g.rf2;
 }
 
+// The FP32 forms from here to tile_filter32() and the margins above them are checked on the host; the scan
+// itself uses the tile test of lt_delense_tile.h, then cell_filter() and far_from_cell().
 // Tile-level pre-test: one FP32 test per (tile of cells, source) instead of one per (cell, source).
 // For the cells i of a tile, all with d_ok, a reference cell r of the tile, and the exact differences
 // delta_i = p_i - p_r, gamma_i = g0_i - g0_r of their corner g (position and gradient), the exact

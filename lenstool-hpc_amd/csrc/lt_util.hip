@@ -55,19 +55,6 @@ hipError_t launch_scale(double* x, double s, size_t n, hipStream_t st)
     return hipGetLastError();
 }
 
-__global__ __launch_bounds__(256) void k_fill_i32(int32_t* __restrict__ p, int32_t v, size_t n)
-{
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
-}
-
-hipError_t launch_fill_i32(int32_t* p, int32_t v, size_t n, hipStream_t s)
-{
-    if (!n) return hipSuccess;
-    hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for(n)), dim3(256), 0, s, p, v, n);
-    return hipGetLastError();
-}
-
 // Byte fill: 16-byte vectors over the aligned body, single bytes at both ends.
 __global__ __launch_bounds__(256) void k_fill16(uint4* __restrict__ p, uint4 v, size_t nvec)
 {
