@@ -13,6 +13,7 @@
 
 #include "lenstool_hip/lt_capi.h"
 #include "lt_far.h"
+#include "lt_hostio.h"
 #include "lt_internal.h"
 #include "lt_kernels.h"
 
@@ -47,7 +48,7 @@ int current_device(int* dev)
         if (e != hipSuccess || n <= 0) return set_error(LT_ERR_NO_DEVICE, "no GPU visible to the HIP runtime");
         LT_HIP_TRY(hipGetDevice(&g_device));
     }
-    if (g_device >= 64) return set_error(LT_ERR_NO_DEVICE, "device index out of range");
+    if (g_device >= kMaxDevices) return set_error(LT_ERR_NO_DEVICE, "device index out of range");
     LT_HIP_TRY(hipSetDevice(g_device));
     *dev = g_device;
     return LT_OK;
@@ -60,36 +61,6 @@ namespace {
 int fail(int code, const std::string& msg) { return set_error(code, msg); }
 int hip_fail(hipError_t e, const char* where) { return hip_error(e, where); }
 #define HIP_TRY(expr) LT_HIP_TRY(expr)
-
-// Per-device state of the synchronous host-array entry points: a stream and grow-only buffers.
-struct DeviceState {
-    std::mutex mu;
-    hipStream_t stream = nullptr;
-    void* halos = nullptr;
-    size_t halos_bytes = 0;
-    void* planes = nullptr;
-    size_t planes_bytes = 0;
-};
-
-constexpr int kMaxDevices = 64;
-DeviceState g_state[kMaxDevices];
-
-int ensure(void** buf, size_t* have, size_t need)
-{
-    if (need <= *have) return LT_OK;
-    if (*buf) HIP_TRY(hipFree(*buf));
-    *buf = nullptr;
-    *have = 0;
-    size_t n = need + need / 4;
-    hipError_t e = hipMalloc(buf, n);
-    if (e != hipSuccess) {
-        *buf = nullptr;
-        (void)hipGetLastError();
-        return fail(LT_ERR_NOMEM, "device allocation of " + std::to_string(n) + " bytes failed");
-    }
-    *have = n;
-    return LT_OK;
-}
 
 // Pixels per thread chosen by lt_autotune, per (kernel family, precision, halo-count and pixel-count
 // octave); 2 where nothing was tuned. Every px gives bit-identical results: only speed differs.
@@ -268,9 +239,9 @@ int host_map(int kind, int mode, Use use, double* const host_out[5], const lt_gr
 
     int dev;
     if ((st = current_device(&dev))) return st;
-    DeviceState& S = g_state[dev];
+    HostState& S = host_state(dev);
     std::lock_guard<std::mutex> lock(S.mu);
-    if (!S.stream) HIP_TRY(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
+    if ((st = host_ready(S))) return st;
 
     const size_t n = (size_t)nx * (size_t)ny;
     const size_t rec_bytes = recs.size() * sizeof(HaloRec);
@@ -278,18 +249,19 @@ int host_map(int kind, int mode, Use use, double* const host_out[5], const lt_gr
     const size_t run_bytes = runs.size() * sizeof(Run);
     const size_t far_bytes = recs.size() * sizeof(FarRec);
     const size_t off_runs = ((rec_bytes + rec32_bytes + far_bytes + 63) / 64) * 64, halo_need = off_runs + run_bytes;
-    if ((st = ensure(&S.halos, &S.halos_bytes, std::max<size_t>(halo_need, 1)))) return st;
-    if ((st = ensure(&S.planes, &S.planes_bytes, n * np * sizeof(double)))) return st;
+    if ((st = host_ensure(&S.halos, &S.halos_bytes, std::max<size_t>(halo_need, 1)))) return st;
+    if ((st = host_ensure(&S.planes, &S.planes_bytes, n * np * sizeof(double)))) return st;
 
-    // one image of the model and one copy of it
-    std::vector<char> image(halo_need);
+    // one image of the model, in the pinned area where it fits, and one copy of it
+    std::vector<char> large(halo_need <= kHostPinned ? 0 : halo_need);
+    char* const image = large.empty() ? S.pinned : large.data();
     DevModel m;
     if (rec_bytes) {
-        std::memcpy(image.data(), recs.data(), rec_bytes);
-        std::memcpy(image.data() + rec_bytes, recs32.data(), rec32_bytes);
-        far_records(recs.data(), (int)recs.size(), (FarRec*)(image.data() + rec_bytes + rec32_bytes));
-        std::memcpy(image.data() + off_runs, runs.data(), run_bytes);
-        HIP_TRY(hipMemcpyAsync(S.halos, image.data(), halo_need, hipMemcpyHostToDevice, S.stream));
+        std::memcpy(image, recs.data(), rec_bytes);
+        std::memcpy(image + rec_bytes, recs32.data(), rec32_bytes);
+        far_records(recs.data(), (int)recs.size(), (FarRec*)(image + rec_bytes + rec32_bytes));
+        std::memcpy(image + off_runs, runs.data(), run_bytes);
+        HIP_TRY(hipMemcpyAsync(S.halos, image, halo_need, hipMemcpyHostToDevice, S.stream));
     }
     char* base = (char*)S.halos;
     m.recs = (HaloRec*)base;
@@ -313,12 +285,15 @@ int host_map(int kind, int mode, Use use, double* const host_out[5], const lt_gr
     g.pitch = nx;
     g.nsamples = 1;
     m.far = far_stats(recs.data(), nhalos, runs);
-    if ((st = launch_map(m, kind, mode, dev_out, r, mult, g, g, precision, 0, S.stream, nhalos))) return st;
+    if ((st = launch_map(m, kind, mode, dev_out, r, mult, g, g, precision, 0, S.stream, nhalos))) {
+        (void)hipStreamSynchronize(S.stream);  // the upload reads the pinned area
+        return st;
+    }
+    HostCopy copies[5];
+    int nc = 0;
     for (int k = 0; k < np; ++k)
-        if (host_out[k])
-            HIP_TRY(hipMemcpyAsync(host_out[k], dev_out[k], n * sizeof(double), hipMemcpyDeviceToHost, S.stream));
-    HIP_TRY(hipStreamSynchronize(S.stream));
-    return LT_OK;
+        if (host_out[k]) copies[nc++] = {host_out[k], dev_out[k], n * sizeof(double)};
+    return host_download(S, copies, nc);
 }
 
 }  // namespace
@@ -356,7 +331,7 @@ int lt_sync(void)
 {
     int dev, st;
     if ((st = current_device(&dev))) return st;
-    if (g_state[dev].stream) HIP_TRY(hipStreamSynchronize(g_state[dev].stream));
+    if (hipStream_t s = host_state(dev).stream) HIP_TRY(hipStreamSynchronize(s));
     return LT_OK;
 }
 
@@ -366,7 +341,7 @@ int lt_dev_alloc(void** ptr, long long bytes)
     *ptr = nullptr;
     int dev, st;
     if ((st = current_device(&dev))) return st;
-    hipError_t e = hipMalloc(ptr, (size_t)(bytes > 0 ? bytes : 1));
+    hipError_t e = device_alloc(ptr, (size_t)(bytes > 0 ? bytes : 1));
     if (e != hipSuccess) {
         (void)hipGetLastError();
         *ptr = nullptr;
@@ -725,7 +700,7 @@ int lt_model_create_batch(lt_model* out, const lt_potential_soa* lenses, int nsa
     const size_t off_runs = ((m->rec_bytes + m->rec32_bytes + far_bytes + 63) / 64) * 64;
     m->off_runs = off_runs;
     m->bytes = off_runs + runs.size() * sizeof(Run) + 64;
-    hipError_t e = hipMalloc(&m->base, m->bytes);
+    hipError_t e = device_alloc(&m->base, m->bytes);
     if (e == hipSuccess) e = hipHostMalloc(&m->staging, m->bytes);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&m->staged, hipEventDisableTiming);
     if (e != hipSuccess) {

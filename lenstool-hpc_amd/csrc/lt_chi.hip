@@ -10,6 +10,7 @@
 
 #include "lenstool_hip/lt_capi.h"
 #include "lt_delense.h"
+#include "lt_hostio.h"
 #include "lt_internal.h"
 #include "lt_kernels.h"
 
@@ -21,9 +22,11 @@ struct lt_chi_batch_s {
     lt_grid_param frame{};
     double dx = 0, dy = 0;
     std::vector<int> types;
-    HaloRec* staging = nullptr;  // pinned host image of the samples' records (one async upload per run)
-    hipEvent_t staged = nullptr;  // recorded after that upload: the next run refills staging after it
+    // pinned host image of the inputs (the start of `block`: runs, families, the samples' records), and the results
+    char* staging = nullptr;
+    hipEvent_t staged = nullptr;  // recorded after the upload: the next run refills staging after it
     std::vector<Run> runs;
+    size_t off_recs = 0, input_bytes = 0, off_results = 0, result_bytes = 0;
     void* block = nullptr;
     HaloRec* recs = nullptr;
     Run* druns = nullptr;
@@ -62,30 +65,31 @@ int validate_families(int nsets, const int* nimages, const lt_galaxy* images, in
     return LT_OK;
 }
 
-int batch_alloc(lt_chi_batch_s* b, const int* nimages, const lt_galaxy* images)
+// The buffers of a batch in one block at p (NULL: sizes and offsets alone); returns its size. The inputs lie in front,
+// the results of all samples together.
+size_t batch_layout(lt_chi_batch_s* b, char* p)
 {
     const size_t S = b->S, K = b->nsets, I = b->nimg, N2 = (size_t)b->n * b->n;
     Carver c;
-    size_t o_recs = c.take<HaloRec>(S * std::max(b->H, 1));
     size_t o_runs = c.take<Run>(std::max<size_t>(b->runs.size(), 1));
-    size_t o_gx = c.take<double>(S * N2), o_gy = c.take<double>(S * N2);
     size_t o_nim = c.take<int32_t>(K), o_first = c.take<int32_t>(K);
     size_t o_ix = c.take<double>(I), o_iy = c.take<double>(I), o_idr = c.take<double>(I);
+    size_t o_recs = c.take<HaloRec>(S * std::max(b->H, 1));
+    b->off_recs = o_recs;
+    b->input_bytes = c.off;
+    size_t o_chi = c.take<double>(S), o_found = c.take<int32_t>(S), o_st = c.take<int32_t>(S);
+    b->off_results = o_chi;
+    b->result_bytes = c.off - o_chi;
+    size_t o_gx = c.take<double>(S * N2), o_gy = c.take<double>(S * N2);
     size_t o_igx = c.take<double>(S * I), o_igy = c.take<double>(S * I);
     size_t o_sx = c.take<double>(S * K), o_sy = c.take<double>(S * K), o_sdr = c.take<double>(S * K);
     size_t o_sb = c.take<double>(S * 3);
     size_t o_items = c.take<ScanItem>(S * (size_t)scan_items(b->n, b->nsets)), o_nitems = c.take<int32_t>(S);
     size_t o_cnt = c.take<int32_t>(S * K), o_hits = c.take<int32_t>(S * K * DELENSE_CAP);
     size_t o_px = c.take<double>(S * K * LT_MAXIMPERSOURCE), o_py = c.take<double>(S * K * LT_MAXIMPERSOURCE);
-    size_t o_loc = c.take<int32_t>(S * K), o_st = c.take<int32_t>(S), o_terms = c.take<double>(S * I);
-    size_t o_chi = c.take<double>(S), o_found = c.take<int32_t>(S);
-    hipError_t e = hipMalloc(&b->block, c.off);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        b->block = nullptr;
-        return set_error(LT_ERR_NOMEM, "chi batch: device allocation of " + std::to_string(c.off) + " bytes failed");
-    }
-    char* p = (char*)b->block;
+    size_t o_loc = c.take<int32_t>(S * K), o_terms = c.take<double>(S * I);
+    if (!p) return c.off;
+    b->block = p;
     b->recs = (HaloRec*)(p + o_recs);
     b->druns = (Run*)(p + o_runs);
     b->gx = (double*)(p + o_gx);
@@ -122,45 +126,53 @@ int batch_alloc(lt_chi_batch_s* b, const int* nimages, const lt_galaxy* images)
     d.terms = (double*)(p + o_terms);
     d.chi = (double*)(p + o_chi);
     d.found = (int32_t*)(p + o_found);
+    return c.off;
+}
+
+// the image families as they lie in the block, at its host image
+void stage_families(const lt_chi_batch_s* b, char* image, const int* nimages, const lt_galaxy* images)
+{
+    const auto at = [&](const void* dev) { return image + ((const char*)dev - (const char*)b->block); };
+    int32_t* const num = (int32_t*)at(b->d.nimages), * const first = (int32_t*)at(b->d.first_image);
+    double* const x = (double*)at(b->d.img_x), * const y = (double*)at(b->d.img_y), * const dr = (double*)at(b->d.img_dr);
+    for (int k = 0, i = 0; k < b->nsets; i += nimages[k++]) {
+        num[k] = nimages[k];
+        first[k] = i;
+    }
+    for (int i = 0; i < b->nimg; ++i) {
+        x[i] = images[i].center.x;
+        y[i] = images[i].center.y;
+        dr[i] = images[i].dr;
+    }
+}
+
+int batch_alloc(lt_chi_batch_s* b, const int* nimages, const lt_galaxy* images)
+{
+    const size_t bytes = batch_layout(b, nullptr);
+    hipError_t e = device_alloc(&b->block, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        b->block = nullptr;
+        return set_error(LT_ERR_NOMEM, "chi batch: device allocation of " + std::to_string(bytes) + " bytes failed");
+    }
+    batch_layout(b, (char*)b->block);
     if (nimages && images) {
-        std::vector<int32_t> first(K);
-        std::vector<double> ix(I), iy(I), idr(I);
-        int at = 0;
-        for (size_t k = 0; k < K; ++k) {
-            first[k] = at;
-            at += nimages[k];
-        }
-        for (size_t i = 0; i < I; ++i) {
-            ix[i] = images[i].center.x;
-            iy[i] = images[i].center.y;
-            idr[i] = images[i].dr;
-        }
-        LT_HIP_TRY(hipMemcpy((void*)d.nimages, nimages, K * sizeof(int32_t), hipMemcpyHostToDevice));
-        LT_HIP_TRY(hipMemcpy((void*)d.first_image, first.data(), K * sizeof(int32_t), hipMemcpyHostToDevice));
-        LT_HIP_TRY(hipMemcpy((void*)d.img_x, ix.data(), I * sizeof(double), hipMemcpyHostToDevice));
-        LT_HIP_TRY(hipMemcpy((void*)d.img_y, iy.data(), I * sizeof(double), hipMemcpyHostToDevice));
-        LT_HIP_TRY(hipMemcpy((void*)d.img_dr, idr.data(), I * sizeof(double), hipMemcpyHostToDevice));
+        std::vector<char> image(b->off_recs);
+        stage_families(b, image.data(), nimages, images);
+        LT_HIP_TRY(hipMemcpy(b->block, image.data(), image.size(), hipMemcpyHostToDevice));
     }
     return LT_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-int lt_chi_batch_create(lt_chi_batch* out, int nsamples, int nhalos, const int* types, int nbgridcells,
-                        const lt_grid_param* frame, int nsets, const int* nimages, const lt_galaxy* images)
+// sizes, types and run structure of a batch (the block is not there yet)
+int batch_setup(lt_chi_batch_s* b, int nsamples, int nhalos, const int* types, int nbgridcells, const lt_grid_param* frame,
+                int nsets, const int* nimages, const lt_galaxy* images)
 {
-    if (!out) return set_error(LT_ERR_INVALID, "out is NULL");
-    *out = nullptr;
     if (nsamples <= 0 || nhalos < 0 || (nhalos && !types) || nbgridcells < 2 || !frame)
         return set_error(LT_ERR_INVALID, "chi batch: bad sizes");
     int nimg, st;
     if ((st = validate_families(nsets, nimages, images, &nimg))) return st;
-    int dev;
-    if ((st = current_device(&dev))) return st;
-    lt_chi_batch_s* b = new lt_chi_batch_s();
-    b->device = dev;
+    if ((st = current_device(&b->device))) return st;
     b->S = nsamples;
     b->H = nhalos;
     b->n = nbgridcells;
@@ -183,22 +195,109 @@ int lt_chi_batch_create(lt_chi_batch* out, int nsamples, int nhalos, const int* 
         s0 += c;
     }
     for (int t : b->types)
-        if (t != 5 && t != 8 && t != 81) {
-            delete b;
+        if (t != 5 && t != 8 && t != 81)
             return set_error(LT_ERR_TYPE, "chi batch: halo type " + std::to_string(t) + " has no gradient");
+    return LT_OK;
+}
+
+// The host image that a run fills and uploads holds the families and is free to be written; queues everything up to the
+// results' copy into it and waits for them.
+int batch_run(lt_chi_batch_s* b, const lt_potential_soa* lenses, double* chi, int* found, int* status, hipStream_t s)
+{
+    std::vector<HaloRec> recs;
+    std::vector<HaloRec32> recs32;
+    std::vector<Run> runs;
+    std::string err;
+    int st;
+    // halo types of every sample, and the circular-SIS flag of each run: set when every halo of the run
+    // is a circular SIS in every sample (the packer's per-sample rule, ANDed), known before any launch
+    for (Run& r : b->runs) r.circ = r.type == TYPE_SIS ? 1 : 0;
+    for (int i = 0; i < b->S; ++i) {
+        const lt_potential_soa& L = lenses[i];
+        for (int h = 0; h < b->H; ++h)
+            if (!L.type || L.type[h] != b->types[h])
+                return set_error(LT_ERR_INVALID, "sample " + std::to_string(i) + ": halo types differ from the batch's");
+        for (Run& r : b->runs)
+            for (int h = r.start; h < r.start + r.count && r.circ; ++h)
+                r.circ = L.ellipticity_potential && L.ellipticity_potential[h] == 0.0;
+    }
+    if (!b->runs.empty()) std::memcpy(b->staging, b->runs.data(), b->runs.size() * sizeof(Run));
+    // gradient grids of every sample (src/chi_CPU_barycenter.cpp:125-137), launched per chunk of samples
+    // as soon as the chunk is packed, so that the host packs the next chunk while the device computes: small ones
+    // first, so that the device starts early
+    GridDesc g{};
+    g.xmin = b->frame.xmin;
+    g.ymin = b->frame.ymin;
+    g.dx = b->dx;
+    g.dy = b->dy;
+    g.nx = b->n;
+    g.ny = b->n;
+    g.pitch = b->n;
+    g.halo_stride = b->H;
+    g.plane_stride = (int64_t)b->n * b->n;
+    OutDesc o{};
+    o.kind = LT_MAP_GRADIENT;
+    o.r = 1.0;
+    o.mult = 1.0;
+    const int most = std::max(64, (b->S + 7) / 8);
+    int chunk = std::min(most, 16);
+    for (int c0 = 0, cn; c0 < b->S; c0 += cn, chunk = std::min(most, 2 * chunk)) {
+        cn = std::min(chunk, b->S - c0);
+        HaloRec* const staged = (HaloRec*)(b->staging + b->off_recs);
+        for (int i = c0; i < c0 + cn; ++i) {
+            st = pack_model(&lenses[i], b->H, Use::Gradient, recs, recs32, runs, err);
+            if (!st && runs.size() != b->runs.size()) {
+                st = LT_ERR_INVALID;
+                err = "run structure differs";
+            }
+            if (st) return set_error(st, "sample " + std::to_string(i) + ": " + err);
+            if (b->H) std::memcpy(&staged[(size_t)i * b->H], recs.data(), (size_t)b->H * sizeof(HaloRec));
         }
-    if ((st = batch_alloc(b, nimages, images))) {
+        // the first copy takes the runs and the families with it
+        const size_t from = c0 ? b->off_recs + (size_t)c0 * b->H * sizeof(HaloRec) : 0;
+        const size_t to = b->off_recs + (size_t)(c0 + cn) * b->H * sizeof(HaloRec);
+        if (to > from) LT_HIP_TRY(hipMemcpyAsync((char*)b->block + from, b->staging + from, to - from, hipMemcpyHostToDevice, s));
+        g.nsamples = cn;
+        o.p0 = b->gx + (size_t)c0 * g.plane_stride;
+        o.p1 = b->gy + (size_t)c0 * g.plane_stride;
+        // 4 pixels per thread: with few halos per sample each halo record's scalar load is shared by
+        // more pixels (1024 samples of 11 halos on 512^2: 9.9 ms per batch step against 10.4 at 2; the
+        // planes are bit-identical for every pixels-per-thread)
+        LT_HIP_TRY(launch_gradient64(b->recs + (size_t)c0 * b->H, b->druns, (int)b->runs.size(), g, o, 4, s));
+    }
+    LT_HIP_TRY(launch_points_gradient64(b->recs, b->druns, (int)b->runs.size(), b->d.img_x, b->d.img_y, b->nimg,
+                                        b->S, b->H, b->img_gx, b->img_gy, s));
+    LT_HIP_TRY(launch_barycentres(b->img_gx, b->img_gy, b->d, s));
+    LT_HIP_TRY(launch_delense(b->gx, b->gy, b->d, s));
+    LT_HIP_TRY(launch_chi(b->d, s));
+    char* const res = b->staging + b->off_results;
+    LT_HIP_TRY(hipMemcpyAsync(res, (char*)b->block + b->off_results, b->result_bytes, hipMemcpyDeviceToHost, s));
+    LT_HIP_TRY(hipStreamSynchronize(s));
+    const auto at = [&](const void* dev) { return b->staging + ((const char*)dev - (const char*)b->block); };
+    std::memcpy(chi, at(b->d.chi), (size_t)b->S * sizeof(double));
+    if (found) std::memcpy(found, at(b->d.found), (size_t)b->S * sizeof(int));
+    if (status) std::memcpy(status, at(b->d.status), (size_t)b->S * sizeof(int));
+    return LT_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int lt_chi_batch_create(lt_chi_batch* out, int nsamples, int nhalos, const int* types, int nbgridcells,
+                        const lt_grid_param* frame, int nsets, const int* nimages, const lt_galaxy* images)
+{
+    if (!out) return set_error(LT_ERR_INVALID, "out is NULL");
+    *out = nullptr;
+    lt_chi_batch_s* b = new lt_chi_batch_s();
+    int st = batch_setup(b, nsamples, nhalos, types, nbgridcells, frame, nsets, nimages, images);
+    if (!st) st = batch_alloc(b, nimages, images);
+    if (st) {
+        if (b->block) (void)hipFree(b->block);
         delete b;
         return st;
     }
-    if (!b->runs.empty() &&
-        hipMemcpy(b->druns, b->runs.data(), b->runs.size() * sizeof(Run), hipMemcpyHostToDevice) != hipSuccess) {
-        (void)hipFree(b->block);
-        delete b;
-        return set_error(LT_ERR_HIP, "chi batch: run upload failed");
-    }
-    if (hipHostMalloc((void**)&b->staging, (size_t)nsamples * std::max(nhalos, 1) * sizeof(HaloRec),
-                      hipHostMallocDefault) != hipSuccess ||
+    if (hipHostMalloc((void**)&b->staging, b->off_results + b->result_bytes, hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&b->staged, hipEventDisableTiming) != hipSuccess) {
         (void)hipGetLastError();
         if (b->staging) (void)hipHostFree(b->staging);
@@ -206,6 +305,7 @@ int lt_chi_batch_create(lt_chi_batch* out, int nsamples, int nhalos, const int* 
         delete b;
         return set_error(LT_ERR_NOMEM, "chi batch: pinned staging allocation failed");
     }
+    stage_families(b, b->staging, nimages, images);
     *out = b;
     return LT_OK;
 }
@@ -231,83 +331,11 @@ int lt_chi_batch_run(lt_chi_batch b, const lt_potential_soa* lenses, double* chi
     if (!b) return set_error(LT_ERR_NOT_FOUND, "chi batch is NULL");
     if (!lenses || !chi) return set_error(LT_ERR_INVALID, "chi batch run: NULL argument");
     LT_HIP_TRY(hipSetDevice(b->device));
-    hipStream_t s = (hipStream_t)stream;
-    std::vector<HaloRec> recs;
-    std::vector<HaloRec32> recs32;
-    std::vector<Run> runs;
-    std::string err;
     // the previous run's upload may still read the staging area if that run stopped on an error
     LT_HIP_TRY(hipEventSynchronize(b->staged));
-    // halo types of every sample, and the circular-SIS flag of each run: set when every halo of the run
-    // is a circular SIS in every sample (the packer's per-sample rule, ANDed), known before any launch
-    for (Run& r : b->runs) r.circ = r.type == TYPE_SIS ? 1 : 0;
-    for (int i = 0; i < b->S; ++i) {
-        const lt_potential_soa& L = lenses[i];
-        for (int h = 0; h < b->H; ++h)
-            if (!L.type || L.type[h] != b->types[h])
-                return set_error(LT_ERR_INVALID, "sample " + std::to_string(i) + ": halo types differ from the batch's");
-        for (Run& r : b->runs)
-            for (int h = r.start; h < r.start + r.count && r.circ; ++h)
-                r.circ = L.ellipticity_potential && L.ellipticity_potential[h] == 0.0;
-    }
-    if (!b->runs.empty())
-        LT_HIP_TRY(hipMemcpyAsync(b->druns, b->runs.data(), b->runs.size() * sizeof(Run), hipMemcpyHostToDevice, s));
-    int st;
-    // gradient grids of every sample (src/chi_CPU_barycenter.cpp:125-137), launched per chunk of samples
-    // as soon as the chunk is packed, so that the host packs the next chunk while the device computes
-    GridDesc g{};
-    g.xmin = b->frame.xmin;
-    g.ymin = b->frame.ymin;
-    g.dx = b->dx;
-    g.dy = b->dy;
-    g.nx = b->n;
-    g.ny = b->n;
-    g.pitch = b->n;
-    g.halo_stride = b->H;
-    g.plane_stride = (int64_t)b->n * b->n;
-    OutDesc o{};
-    o.kind = LT_MAP_GRADIENT;
-    o.r = 1.0;
-    o.mult = 1.0;
-    const int chunk = std::max(64, (b->S + 7) / 8);
-    for (int c0 = 0; c0 < b->S; c0 += chunk) {
-        const int cn = std::min(chunk, b->S - c0);
-        for (int i = c0; i < c0 + cn; ++i) {
-            st = pack_model(&lenses[i], b->H, Use::Gradient, recs, recs32, runs, err);
-            if (!st && runs.size() != b->runs.size()) {
-                st = LT_ERR_INVALID;
-                err = "run structure differs";
-            }
-            if (st) {
-                // uploads of earlier chunks may still read the staging area: the next run waits for them
-                const hipError_t e = hipEventRecord(b->staged, s);
-                if (e != hipSuccess) return hip_error(e, "chi batch: event record");
-                return set_error(st, "sample " + std::to_string(i) + ": " + err);
-            }
-            if (b->H) std::memcpy(&b->staging[(size_t)i * b->H], recs.data(), (size_t)b->H * sizeof(HaloRec));
-        }
-        if (b->H)
-            LT_HIP_TRY(hipMemcpyAsync(b->recs + (size_t)c0 * b->H, b->staging + (size_t)c0 * b->H,
-                                      (size_t)cn * b->H * sizeof(HaloRec), hipMemcpyHostToDevice, s));
-        g.nsamples = cn;
-        o.p0 = b->gx + (size_t)c0 * g.plane_stride;
-        o.p1 = b->gy + (size_t)c0 * g.plane_stride;
-        // 4 pixels per thread: with few halos per sample each halo record's scalar load is shared by
-        // more pixels (1024 samples of 11 halos on 512^2: 9.9 ms per batch step against 10.4 at 2; the
-        // planes are bit-identical for every pixels-per-thread)
-        LT_HIP_TRY(launch_gradient64(b->recs + (size_t)c0 * b->H, b->druns, (int)b->runs.size(), g, o, 4, s));
-    }
-    LT_HIP_TRY(hipEventRecord(b->staged, s));
-    LT_HIP_TRY(launch_points_gradient64(b->recs, b->druns, (int)b->runs.size(), b->d.img_x, b->d.img_y, b->nimg,
-                                        b->S, b->H, b->img_gx, b->img_gy, s));
-    LT_HIP_TRY(launch_barycentres(b->img_gx, b->img_gy, b->d, s));
-    LT_HIP_TRY(launch_delense(b->gx, b->gy, b->d, s));
-    LT_HIP_TRY(launch_chi(b->d, s));
-    LT_HIP_TRY(hipMemcpyAsync(chi, b->d.chi, (size_t)b->S * sizeof(double), hipMemcpyDeviceToHost, s));
-    if (found) LT_HIP_TRY(hipMemcpyAsync(found, b->d.found, (size_t)b->S * sizeof(int), hipMemcpyDeviceToHost, s));
-    if (status) LT_HIP_TRY(hipMemcpyAsync(status, b->d.status, (size_t)b->S * sizeof(int), hipMemcpyDeviceToHost, s));
-    LT_HIP_TRY(hipStreamSynchronize(s));
-    return LT_OK;
+    const int st = batch_run(b, lenses, chi, found, status, (hipStream_t)stream);
+    if (st) (void)hipEventRecord(b->staged, (hipStream_t)stream);
+    return st;
 }
 
 int lt_chi_batch_images(lt_chi_batch b, int sample, lt_point* image_pos, int* locimagesfound)
@@ -380,11 +408,27 @@ int lt_chi_barycentersource(double* chi, int* error, int nbgridcells, int nsets,
                             const lt_grid_param* frame, const int* nimages, const lt_galaxy* images)
 {
     if (!chi || !lens) return set_error(LT_ERR_INVALID, "chi: NULL argument");
-    lt_chi_batch b = nullptr;
-    int st = lt_chi_batch_create(&b, 1, nhalos, lens->type, nbgridcells, frame, nsets, nimages, images);
+    lt_chi_batch_s b;
     int found = 0, sst = LT_OK;
-    if (st == LT_OK) st = lt_chi_batch_run(b, lens, chi, &found, &sst, nullptr);
-    lt_chi_batch_destroy(b);
+    int st = batch_setup(&b, 1, nhalos, lens->type, nbgridcells, frame, nsets, nimages, images);
+    if (st == LT_OK) {
+        // an optimiser makes this call again and again: its buffers stay, one copy each way
+        HostState& S = host_state(b.device);
+        std::lock_guard<std::mutex> lock(S.mu);
+        HostScratch room;
+        const size_t bytes = batch_layout(&b, nullptr), host_bytes = b.off_results + b.result_bytes;
+        std::vector<char> large;
+        st = host_ready(S);
+        if (!st) st = room.take(S, bytes);
+        if (!st) {
+            batch_layout(&b, room.p);
+            if (host_bytes > kHostPinned) large.resize(host_bytes);
+            b.staging = large.empty() ? S.pinned : large.data();
+            stage_families(&b, b.staging, nimages, images);
+            st = batch_run(&b, lens, chi, &found, &sst, S.stream);
+            if (st) (void)hipStreamSynchronize(S.stream);  // the upload reads the staging area
+        }
+    }
     if (st == LT_OK && sst != LT_OK) st = set_error(sst, "chi: more than 20 images for one source (kept the first 20)");
     if (error) *error = st;
     return st;
@@ -441,26 +485,38 @@ int lt_point_gradients(double* gx, double* gy, const double* px, const double* p
     if (st) return set_error(st, err);
     int dev;
     if ((st = current_device(&dev))) return st;
+    HostState& S = host_state(dev);
+    std::lock_guard<std::mutex> lock(S.mu);
+    if ((st = host_ready(S))) return st;
+    const size_t bytes = (size_t)npts * sizeof(double);
     Carver c;
-    size_t o_r = c.take<HaloRec>(std::max<size_t>(recs.size(), 1)), o_u = c.take<Run>(std::max<size_t>(runs.size(), 1));
-    size_t o_x = c.take<double>(npts), o_y = c.take<double>(npts), o_gx = c.take<double>(npts), o_gy = c.take<double>(npts);
-    void* blk = nullptr;
-    LT_HIP_TRY(hipMalloc(&blk, c.off));
-    char* p = (char*)blk;
-    hipError_t e = hipSuccess;
-    if (!recs.empty()) e = hipMemcpy(p + o_r, recs.data(), recs.size() * sizeof(HaloRec), hipMemcpyHostToDevice);
-    if (e == hipSuccess && !runs.empty())
-        e = hipMemcpy(p + o_u, runs.data(), runs.size() * sizeof(Run), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(p + o_x, px, npts * sizeof(double), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(p + o_y, py, npts * sizeof(double), hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = launch_points_gradient64((HaloRec*)(p + o_r), (Run*)(p + o_u), (int)runs.size(), (double*)(p + o_x),
-                                     (double*)(p + o_y), npts, 1, 0, (double*)(p + o_gx), (double*)(p + o_gy), nullptr);
-    if (e == hipSuccess) e = hipMemcpy(gx, p + o_gx, npts * sizeof(double), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(gy, p + o_gy, npts * sizeof(double), hipMemcpyDeviceToHost);
-    (void)hipFree(blk);
-    if (e != hipSuccess) return hip_error(e, "point gradients");
-    return LT_OK;
+    const size_t o_u = c.take<Run>(std::max<size_t>(runs.size(), 1)), o_r = c.take<HaloRec>(std::max<size_t>(recs.size(), 1));
+    const size_t o_x = c.take<double>(npts), o_y = c.take<double>(npts), input = c.off;
+    const size_t o_gx = c.take<double>(npts), o_gy = o_gx + bytes, need = o_gy + bytes;
+    HostScratch room;
+    if ((st = room.take(S, need))) return st;
+    char* const p = room.p;
+    if (input <= kHostPinned) {
+        // the model and the points in one copy from the pinned area
+        if (!runs.empty()) std::memcpy(S.pinned + o_u, runs.data(), runs.size() * sizeof(Run));
+        if (!recs.empty()) std::memcpy(S.pinned + o_r, recs.data(), recs.size() * sizeof(HaloRec));
+        std::memcpy(S.pinned + o_x, px, bytes);
+        std::memcpy(S.pinned + o_y, py, bytes);
+        LT_HIP_TRY(hipMemcpyAsync(p, S.pinned, input, hipMemcpyHostToDevice, S.stream));
+    } else {
+        if (!runs.empty()) LT_HIP_TRY(hipMemcpy(p + o_u, runs.data(), runs.size() * sizeof(Run), hipMemcpyHostToDevice));
+        if (!recs.empty()) LT_HIP_TRY(hipMemcpy(p + o_r, recs.data(), recs.size() * sizeof(HaloRec), hipMemcpyHostToDevice));
+        LT_HIP_TRY(hipMemcpy(p + o_x, px, bytes, hipMemcpyHostToDevice));
+        LT_HIP_TRY(hipMemcpy(p + o_y, py, bytes, hipMemcpyHostToDevice));
+    }
+    hipError_t e = launch_points_gradient64((HaloRec*)(p + o_r), (Run*)(p + o_u), (int)runs.size(), (double*)(p + o_x),
+                                            (double*)(p + o_y), npts, 1, 0, (double*)(p + o_gx), (double*)(p + o_gy), S.stream);
+    if (e != hipSuccess) {
+        (void)hipStreamSynchronize(S.stream);
+        return hip_error(e, "point gradients");
+    }
+    const HostCopy copies[2] = {{gx, p + o_gx, bytes}, {gy, p + o_gy, bytes}};
+    return host_download(S, copies, 2);
 }
 
 }  // extern "C"

@@ -1,0 +1,60 @@
+// lt_hostio.h -- what the synchronous host-array calls keep per device between calls (a stream, device buffers, a
+// pinned area) and their copies between the caller's arrays and the device.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <mutex>
+
+namespace lt {
+
+constexpr size_t kHostPiece = 1 << 21;             // bytes of a piece of a copy
+constexpr int kHostThreads = 4;                    // threads of a large copy to the host, two pieces of the pinned area each
+constexpr size_t kHostPinned = 2 * kHostThreads * kHostPiece;
+constexpr size_t kHostKept = 64 << 20;             // device bytes that a call's scratch may keep
+
+// One per device; a call holds `mu` from its first use to its end.
+struct HostState {
+    std::mutex mu;
+    hipStream_t stream = nullptr;
+    char* pinned = nullptr;         // kHostPinned bytes
+    void* halos = nullptr;          // grow-only buffers of the map calls
+    size_t halos_bytes = 0;
+    void* planes = nullptr;
+    size_t planes_bytes = 0;
+    void* scratch = nullptr;        // at most kHostKept bytes, see HostScratch
+    size_t scratch_bytes = 0;
+    hipStream_t copy_stream[kHostThreads] = {};
+    hipEvent_t copied[kHostThreads][2] = {};
+};
+
+constexpr int kMaxDevices = 64;
+HostState& host_state(int dev);
+// the stream and the pinned area of the current device's state, made on the first call
+int host_ready(HostState& h);
+// grow-only device buffer
+int host_ensure(void** buf, size_t* have, size_t need);
+
+// hipMalloc that gives back the kept buffers of the device, if no call is using them, rather than fail.
+hipError_t device_alloc(void** p, size_t bytes);
+
+// Device memory of one call: the kept buffer, or an allocation of its own that goes with it.
+struct HostScratch {
+    char* p = nullptr;
+    bool own = false;
+    int take(HostState& h, size_t bytes);
+    ~HostScratch();
+};
+
+// A copy device -> host. Small ones go through the start of the pinned area.
+struct HostCopy {
+    void* host;
+    const void* dev;
+    size_t bytes;
+};
+
+// All the copies device -> host, after the work queued on h.stream; returns when they are done.
+int host_download(HostState& h, const HostCopy* copies, int n);
+
+}  // namespace lt

@@ -15,7 +15,6 @@ int set_error(int code, const std::string& msg);
 int hip_error(hipError_t e, const char* where);
 // the calling thread's device (made current); LT_ERR_NO_DEVICE without a GPU
 int current_device(int* dev);
-// fill n ints of device memory with v (a kernel, so it can sit in a captured graph)
 // fill `bytes` bytes of device memory with v (kernels only: no memset node when captured)
 hipError_t launch_fill_bytes(void* dst, unsigned char v, size_t bytes, hipStream_t s);
 // with `dev` current: the device address of lt_critic_device_noalloc's scratch array on `dev`, looked
