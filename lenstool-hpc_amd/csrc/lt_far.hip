@@ -39,6 +39,7 @@
 #include "lt_device.h"
 #include "lt_far.h"
 #include "lt_kernels.h"
+#define LT_HORNER_COEF "s"
 #include "lt_math.h"
 #include "lt_terms64.h"
 
@@ -321,8 +322,13 @@ __device__ __forceinline__ void store4(double* p, int lane, const d4& v)
     for (int k = 0; k < 4; ++k) p[64 * k + lane] = v[k];
 }
 
+// Bound by the FP64 pipes: VALU issue (70 % of the cycles on the 503-halo 4096^2 fields, 88 % on the 2048^2 potential) and,
+// for light models, matrix instructions beside it (38 % and 26 % on 256 maps of 11 halos). Work-groups of 4 waves are held to
+// three waves a SIMD (168 registers): 256 maps of 2048^2 in 7.1 ms, 8.7 with two, 8.8 with four, which spills. The
+// logarithm's and arctangent's coefficients stay in scalar registers, 36 vector registers less: the potential
+// 2048^2, 503 halos, 825 -> 800 us, displacement 701 x 643, 160 mixed halos, 152 -> 146.
 template <int FAM, int KIND, int LV, int UNIT>
-__global__ __launch_bounds__(WAVE* far_waves(LV), LV == 3 ? 4 : 2) void k_far(const HaloRec* __restrict__ halos,
+__global__ __launch_bounds__(WAVE* far_waves(LV), LV == 3 ? 4 : 3) void k_far(const HaloRec* __restrict__ halos,
                                                                                      const FarRec* __restrict__ recs,
                                                                                      const Run* __restrict__ runs,
                                                                                      int nruns, int nhalos, GridDesc g,

@@ -79,13 +79,19 @@ constexpr double kLogR[7] = {
 // atan(t) = t + t^3 P(t^2) with |t| <= tan(pi/8) and one corrected reciprocal; the octant is put
 // back with pi/4, pi/2 - r, pi - r and the sign of y. atan2(0, 0) = 0 (pi for x = -0), NaN in ->
 // NaN out. About 40 instructions against the hundred of the library atan2.
+// Where a polynomial's coefficients are kept: in vector registers, or (lt_far.hip, whose kernels are short of those) in
+// scalar ones, for which a value a wavefront is set again when they run out.
+#ifndef LT_HORNER_COEF
+#define LT_HORNER_COEF "v"
+#endif
+
 // one Horner step p z + c as a three-operand FMA: written out so that the coefficient c, which the
 // compiler keeps in a register across the halo loop, is read in place instead of being copied into
 // the accumulator of the two-operand form (one instruction per step instead of two)
 __device__ __forceinline__ double horner_step(double p, double z, double c)
 {
     double r;
-    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(p), "v"(z), "v"(c));
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(p), "v"(z), LT_HORNER_COEF(c));
     return r;
 }
 
