@@ -34,9 +34,9 @@ struct FarStats {
 
 FarStats far_stats(const HaloRec* recs, int nhalos, const std::vector<Run>& runs);
 
-// How a map is summed: directly, or by tile expansions in work-groups of 64 (4 or 16 waves), 128 or 256 pixels a
-// side.
-enum class FarShape { Direct, Root64, Root64Wide, Root128, Root256 };
+// How a map is summed: directly, or by tile expansions in work-groups of 64 (4 or 16 waves, or two of
+// 8 or four of 4 for one root), 128 or 256 pixels a side.
+enum class FarShape { Direct, Root64, Root64Wide, Root64Half, Root64Quarter, Root128, Root256 };
 
 // The shape for a map. `whole`: the grid that the rows computed belong to (the grid itself, or the whole map where
 // a part of it is computed on its own). *cost (may be NULL): estimated instructions per pixel of the form chosen.

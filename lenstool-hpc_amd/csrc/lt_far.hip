@@ -327,15 +327,17 @@ __device__ __forceinline__ void store4(double* p, int lane, const d4& v)
 // three waves a SIMD (168 registers): 256 maps of 2048^2 in 7.1 ms, 8.7 with two, 8.8 with four, which spills. The
 // logarithm's and arctangent's coefficients stay in scalar registers, 36 vector registers less: the potential
 // 2048^2, 503 halos, 825 -> 800 us, displacement 701 x 643, 160 mixed halos, 152 -> 146.
-template <int FAM, int KIND, int LV, int UNIT>
-__global__ __launch_bounds__(WAVE* far_waves(LV), LV == 3 ? 4 : 3) void k_far(const HaloRec* __restrict__ halos,
+// PARTS 2 and 4: the halves or the subs of a root go to a work-group each, all of which sum its nodes: a map of fewer than
+// 128 roots would leave the other CUs idle (displacement 701 x 643, 160 mixed halos, 121 roots: 147 us, halved 87).
+template <int FAM, int KIND, int LV, int UNIT, int PARTS>
+__global__ __launch_bounds__(WAVE* far_waves(LV) / PARTS, LV == 3 && PARTS < 4 ? 4 : 3) void k_far(const HaloRec* __restrict__ halos,
                                                                                      const FarRec* __restrict__ recs,
                                                                                      const Run* __restrict__ runs,
                                                                                      int nruns, int nhalos, GridDesc g,
                                                                                      OutDesc o)
 {
     constexpr int NF = fields_of<FAM>();
-    constexpr int NW = far_waves(LV), NS = NW / 4;  // waves = units, subs
+    constexpr int NW = far_waves(LV) / PARTS, NS = NW / 4;  // waves = units, subs
     constexpr int SIDE = far_side(LV, UNIT);
     __shared__ double part[NW][NF][FN];  // node sums of each wave; later the coefficients that it expands
     __shared__ double rootc[LV == 3 ? NF : 1][FN], subc[NS][NF][FN];
@@ -352,14 +354,19 @@ __global__ __launch_bounds__(WAVE* far_waves(LV), LV == 3 ? 4 : 3) void k_far(co
     recs += (int64_t)blockIdx.z * g.halo_stride;
     const int lane = threadIdx.x & 63, q = lane >> 4, j = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sub = wave >> 2, wv = wave & 3;
+    const int place = sub + (int)blockIdx.y % PARTS * NS;  // of the sub in the root
     const int nwords = (nhalos + 63) >> 6;
     const int i0 = (floor_div(g.istart, SIDE) + (int)blockIdx.x) * SIDE;
-    const int j0 = (floor_div(g.jstart, SIDE) + (int)blockIdx.y) * SIDE;
+    const int j0 = (floor_div(g.jstart, SIDE) + (int)blockIdx.y / PARTS) * SIDE;
+    if constexpr (PARTS > 1) {  // a part past the grid
+        const int down = j0 - g.jstart + (place >> 1) * (SIDE / 2), across = PARTS == 4 ? i0 - g.istart + (place & 1) * (SIDE / 2) : 0;
+        if (down + SIDE / 2 <= 0 || down >= g.ny || across + SIDE / 2 <= 0 || across >= g.nx) return;
+    }
     const Axis ax = root_axis(g.xmin, g.dx, i0, SIDE), ay = root_axis(g.ymin, g.dy, j0, SIDE);
     // centre and half sides (signed as the pixel steps) of the wave's sub
     const double shx = LV == 3 ? 0.5 * ax.h : ax.h, shy = LV == 3 ? 0.5 * ay.h : ay.h;
-    const double scx = LV == 3 ? ax.c + ((sub & 1) ? shx : -shx) : ax.c;
-    const double scy = LV == 3 ? ay.c + ((sub >> 1) ? shy : -shy) : ay.c;
+    const double scx = LV == 3 ? ax.c + ((place & 1) ? shx : -shx) : ax.c;
+    const double scy = LV == 3 ? ay.c + ((place >> 1) ? shy : -shy) : ay.c;
     const double hm = __builtin_fmax(__builtin_fabs(shx), __builtin_fabs(shy)), sb2 = kFarBound2 * hm * hm;
 
     // ---- root and sub: sets, node sums by all waves, then one wave per field transforms. The value at a
@@ -404,7 +411,7 @@ __global__ __launch_bounds__(WAVE* far_waves(LV), LV == 3 ? 4 : 3) void k_far(co
     d4 n[NF];
     if constexpr (LV == 3) {
         split_sets<FAM>(recs, list, nlist, wv, 4, nullptr, scx, scy, sb2, sfar[sub], snear[sub]);
-        node_sums<FAM, false>(halos, runs, nruns, HaloSet{top, nullptr, nullptr}, 0x0001000100010001ull << wave, ax.c, ay.c,
+        node_sums<FAM, false>(halos, runs, nruns, HaloSet{top, nullptr, nullptr}, (NW == 4 ? 0x1111111111111111ull : NW == 8 ? 0x0101010101010101ull : 0x0001000100010001ull) << wave, ax.c, ay.c,
                               ax.h, ay.h, n);
 #pragma unroll
         for (int f = 0; f < NF; ++f) store4(part[wave][f], lane, n[f]);
@@ -433,7 +440,7 @@ __global__ __launch_bounds__(WAVE* far_waves(LV), LV == 3 ? 4 : 3) void k_far(co
         v -= r;
         d4 c = {0., 0., 0., 0.};
         if constexpr (LV == 3) {
-            c = shift_half(load4(rootc[wv], lane), sub & 1, sub >> 1, q, j);
+            c = shift_half(load4(rootc[wv], lane), place & 1, place >> 1, q, j);
             r += rootref[wv];
         }
         store4(subc[sub][wv], lane, transform(v, j, q, c));
@@ -442,8 +449,8 @@ __global__ __launch_bounds__(WAVE* far_waves(LV), LV == 3 ? 4 : 3) void k_far(co
     __syncthreads();
 
     // ---- the wave's unit; no work-group barrier from here on
-    const int urow = j0 + (sub >> 1) * 2 * UNIT + (wv >> 1) * UNIT - g.jstart;
-    const int ucol = i0 + (sub & 1) * 2 * UNIT + (wv & 1) * UNIT - g.istart;
+    const int urow = j0 + (place >> 1) * 2 * UNIT + (wv >> 1) * UNIT - g.jstart;
+    const int ucol = i0 + (place & 1) * 2 * UNIT + (wv & 1) * UNIT - g.istart;
     if (urow + UNIT - 1 < 0 || urow >= g.ny || ucol + UNIT - 1 < 0 || ucol >= g.nx) return;
     const double uhx = 0.5 * shx, uhy = 0.5 * shy;
     const double ucx = scx + ((wv & 1) ? uhx : -uhx), ucy = scy + ((wv >> 1) ? uhy : -uhy);
@@ -616,17 +623,19 @@ static unsigned tiles_over(int start, int n, int side);
 
 // Tile expansions cost, per pixel, the halos near its 32-pixel square, 256 nodes over the area of a square for each
 // halo first expanded there, and the expansion itself (72 matrix instructions per 1024 pixels and three fields,
-// in VALU issue slots). From that count and the number of work-groups follows a time (in cycles of a CU, four
-// instructions a cycle and 64 lanes; efficiencies and the fixed share of a work-group as measured: a work-group of 16
-// waves spends about 45 000 cycles beside its sums (120 000 with 128 pixels a side), one of 4 waves 8000, or 35 000
-// where it has the CU to itself):
-//   cluster lens, 258 halos, fields: 512^2 estimated 112 us, measured 117, directly 150; 400^2 156, 144 and 101.
-//   light models (1 dPIE + 10 SIS): 256 maps of 2048^2 in 8.9 ms with 4 waves, 17.6 with 16.
+// in VALU issue slots). From that count and the number of work-groups follows a time in cycles of a CU (four
+// instructions a cycle and 64 lanes), with the efficiencies and fixed shares that were measured: a root of 64 pixels takes 1.15 times its
+// count and about 100 000 cycles beside it (its barriers and the longest wave), a half or a quarter of one 1.25 and 1.5 times
+// its share, the root's nodes included, and about half as much. Over 176 maps (20 to 1000 halos, four kinds, 240^2 to 2100^2)
+// the shape taken is 2 % behind the best of the six in the mean. Some of them, us (direct, 4 waves, 16, halves, quarters):
+//   dpl 672 x 635, 160 mixed halos: 233, 174, 158, 100; fields 450 x 413, 258 dPIE: 129, 214, 174, 110;
+//   potential 450 x 413, 1000 dPIE: 1638, 2409, 2262, 1300; fields 900 x 863, 258: 498, 118, 101, 121.
+//   light models (1 dPIE + 10 SIS): 256 maps of 2048^2 in 7.1 ms with 4 waves, 17.6 with 16.
 //   503 halos, 4096^2: root 128 565 us, root 64 1145; 2000 on 8192^2: root 256 2.6 ms, root 128 5.3.
 // Where roots of 128 pixels halve the count of 64 with these shares added (fine pixels, many halos), the shape depends on the steps and the model alone,
 // so that a part of a map takes the same form as the whole; roots of 256 again have to halve the count of 128: their
 // work-groups are few and uneven (a 300 x 200 part of the 4096^2 map: 271 us, 111 with 128, 183 directly).
-// Elsewhere the quickest shape is taken, or the direct sum where none is ahead of it by a tenth.
+// Elsewhere the quickest shape is taken, or the direct sum.
 FarShape far_shape(const FarStats& st, int kind, int precision, const GridDesc& g, double* cost)
 {
     const int fam = family_of(kind);
@@ -662,7 +671,7 @@ FarShape far_shape(const FarStats& st, int kind, int precision, const GridDesc& 
         return wide ? FarShape::Root256 : FarShape::Root128;
     }
     const double npix = (double)g.nx * (double)g.ny;
-    double best = 0.9 * npix * direct / (64. * 256. * 0.68) + 15e3;
+    double best = npix * direct / (64. * 256. * 0.62) + 15e3;
     FarShape shape = FarShape::Direct;
     auto offer = [&](FarShape f, double t, double c) {
         if (t >= best) return;
@@ -671,10 +680,13 @@ FarShape far_shape(const FarStats& st, int kind, int precision, const GridDesc& 
         if (cost) *cost = c;
     };
     const double n64 = tiles(64), n128 = tiles(128);
-    const double slow = fam == FAM_POTENTIAL ? 1.6 : 1.;  // more registers, fewer waves
-    offer(FarShape::Root64, slow * (n64 < 512. ? c64 * 64. / 0.4 + 35e3 : n64 / 256. * (c64 * 64. / 0.55 + 8e3)), c64);
-    offer(FarShape::Root64Wide, slow * std::ceil(n64 / 256.) * (c64 * 64. / 0.6 + 45e3), c64);
-    offer(FarShape::Root128, std::ceil(n128 / 256.) * (c128 * 256. / 0.6 + 120e3), c128);
+    const double root = d * (1. - near(64)) * FN / 4096., fixed = fam == FAM_POTENTIAL ? 130e3 : 100e3;
+    const auto rounds = [](double groups) { return groups <= 256. ? 1. : std::fmin(std::ceil(groups / 256.), 1.35 * groups / 256.); };
+    offer(FarShape::Root64, n64 < 512. ? 1.2 * 64. * c64 * rounds(n64) + fixed : n64 / 256. * (c64 * 64. / 0.55 + 8e3), c64);
+    offer(FarShape::Root64Wide, 1.15 * 64. * c64 * rounds(n64) + fixed, c64);
+    offer(FarShape::Root64Half, 1.25 * 32. * (c64 + root) * rounds(2. * n64) + 0.55 * fixed, c64);
+    offer(FarShape::Root64Quarter, 1.5 * 16. * (c64 + 3. * root) * rounds(4. * n64) + 0.45 * fixed, c64);
+    offer(FarShape::Root128, rounds(n128) * 1.4 * c128 * 256. + 160e3, c128);
     return shape;
 }
 
@@ -685,14 +697,14 @@ static unsigned tiles_over(int start, int n, int side)
     return (unsigned)(fd((int64_t)start + n - 1) - fd(start) + 1);
 }
 
-template <int FAM, int KIND, int LV, int UNIT>
+template <int FAM, int KIND, int LV, int UNIT, int PARTS = 1>
 static void launch_far_shape(const HaloRec* halos, const FarRec* recs, const Run* runs, int nruns, int nhalos, const GridDesc& g,
                              const OutDesc& o, hipStream_t s)
 {
     constexpr int side = far_side(LV, UNIT);
-    const dim3 grd(tiles_over(g.istart, g.nx, side), tiles_over(g.jstart, g.ny, side),
+    const dim3 grd(tiles_over(g.istart, g.nx, side), PARTS * tiles_over(g.jstart, g.ny, side),
                    (unsigned)(g.nsamples > 0 ? g.nsamples : 1));
-    hipLaunchKernelGGL((k_far<FAM, KIND, LV, UNIT>), grd, dim3(WAVE * far_waves(LV)), 0, s, halos, recs, runs, nruns,
+    hipLaunchKernelGGL((k_far<FAM, KIND, LV, UNIT, PARTS>), grd, dim3(WAVE * far_waves(LV) / PARTS), 0, s, halos, recs, runs, nruns,
                        nhalos, g, o);
 }
 
@@ -703,6 +715,8 @@ static hipError_t launch_far_kind(const HaloRec* halos, const FarRec* recs, cons
     switch (shape) {
     case FarShape::Root64: launch_far_shape<FAM, KIND, 2, 32>(halos, recs, runs, nruns, nhalos, g, o, s); break;
     case FarShape::Root64Wide: launch_far_shape<FAM, KIND, 3, 16>(halos, recs, runs, nruns, nhalos, g, o, s); break;
+    case FarShape::Root64Half: launch_far_shape<FAM, KIND, 3, 16, 2>(halos, recs, runs, nruns, nhalos, g, o, s); break;
+    case FarShape::Root64Quarter: launch_far_shape<FAM, KIND, 3, 16, 4>(halos, recs, runs, nruns, nhalos, g, o, s); break;
     case FarShape::Root128: launch_far_shape<FAM, KIND, 3, 32>(halos, recs, runs, nruns, nhalos, g, o, s); break;
     case FarShape::Root256: launch_far_shape<FAM, KIND, 3, 64>(halos, recs, runs, nruns, nhalos, g, o, s); break;
     default: return hipErrorInvalidValue;
