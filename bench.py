@@ -37,8 +37,7 @@ PEAK_FP64_TFLOPS = 78.6   # MI355X vector FP64
 PEAK_FP32_TFLOPS = 157.3  # MI355X vector FP32 (published figure, counts packed FP32)
 PEAK_HBM_GBS = 8000.0
 METRIC = "halo·pixel evals/s, Hessian maps (FP32-comp vs FP64 GPU); p50/p99 map latency"
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hessian_fields_fp64_4096_503halos_traffic.md")
-COUNTERS_FILE = os.path.join(ROOT, "profiles", "hessian_fields_4096_503halos_valu_counters.md")
+COUNTERS_FILE = os.path.join(ROOT, "profiles", "fields_tile_expansions_4096_503halos.md")
 SIMDS = 1024          # 256 CUs x 4 SIMDs
 CLOCK_HZ = 2.4e9      # MI355X peak engine clock
 
@@ -66,28 +65,19 @@ def run_maps(model, outs, grid, r, precision, steps, warmup, stream, px=0, kind=
 
 
 def read_counters():
-    """Per dPIE halo x pixel figures of the FP64 Hessian + fields kernel from its committed rocprofv3
-    counter summary: hardware FP64 flops (64 lanes x (ADD + MUL + 2 FMA) from SQ_INSTS_VALU_*_F64) and
-    VALU issue slots (SQ_ACTIVE_INST_VALU); None when absent."""
+    """Figures of one launch of the default map from its committed rocprofv3 counter summary: hardware FP64
+    flops (64 lanes x (ADD + MUL + 2 FMA) and matrix operations), VALU issue slots, matrix busy cycles and HBM
+    bytes; None when absent."""
     if not os.path.exists(COUNTERS_FILE):
         return None
     txt = open(COUNTERS_FILE).read()
     out = {}
-    for key in ("fp64_hw_flop_per_halo_px", "valu_issue_slots_per_halo_px"):
-        m = re.search(key + r":\s*([0-9.eE+]+)", txt)
+    for key in ("fp64_hw_flop", "valu_issue_slots", "mfma_busy_cycles", "traffic_bytes"):
+        m = re.search(key + r"_per_launch:\s*([0-9.eE+]+)", txt)
         if not m:
             return None
         out[key] = float(m.group(1))
     return out
-
-
-def read_traffic():
-    """HBM bytes per launch measured with rocprofv3 --pmc (FETCH_SIZE, WRITE_SIZE), committed as a
-    summary next to the kernel traces; None when absent."""
-    if not os.path.exists(TRAFFIC_FILE):
-        return None
-    m = re.search(r"traffic_bytes_per_launch:\s*([0-9.eE+]+)", open(TRAFFIC_FILE).read())
-    return float(m.group(1)) if m else None
 
 
 def cpu_model():
@@ -460,26 +450,25 @@ def main():
     flops_per_map = lens.halo_flops("hessian") * grid.npix
     algorithmic = flops_per_map / (avg_ms * 1e-3) / 1e12
     peak = PEAK_FP64_TFLOPS if prec == lthip.PREC_FP64 else PEAK_FP32_TFLOPS
-    traffic = read_traffic() if prec == lthip.PREC_FP64 else None
     counters = read_counters() if prec == lthip.PREC_FP64 else None
-    rate_dev = halo_px / (avg_ms * 1e-3)  # halo x px per second of kernel time
     if counters:
-        achieved = counters["fp64_hw_flop_per_halo_px"] * rate_dev / 1e12
+        sec = avg_ms * 1e-3
+        achieved = counters["fp64_hw_flop"] / sec / 1e12
         roofline = {"bound": "valu", "achieved": achieved, "peak": peak, "unit": "TFLOP/s", "frac": achieved / peak,
-                    "traffic": traffic,
-                    "flops": "hardware FP64 flops, 64 lanes x (ADD + MUL + 2 FMA) per wavefront instruction, "
-                             f"{counters['fp64_hw_flop_per_halo_px']:.2f} per dPIE halo x px (rocprofv3 "
-                             "SQ_INSTS_VALU_{ADD,MUL,FMA}_F64, profiles/hessian_fields_4096_503halos_valu_counters.md)",
-                    "valu_issue_frac": counters["valu_issue_slots_per_halo_px"] * 4 * rate_dev / (SIMDS * CLOCK_HZ),
-                    "valu_issue": f"SQ_ACTIVE_INST_VALU slots ({counters['valu_issue_slots_per_halo_px']:.3f} per "
-                                  "dPIE halo x px) x 4 cycles / (1024 SIMDs x 2.4 GHz x time)",
+                    "traffic": counters["traffic_bytes"],
+                    "flops": f"hardware FP64 flops of a launch ({counters['fp64_hw_flop']:.3e}; rocprofv3 "
+                             "SQ_INSTS_VALU_{ADD,MUL,FMA}_F64 and MFMA_MOPS_F64, "
+                             "profiles/fields_tile_expansions_4096_503halos.md)",
+                    "valu_issue_frac": counters["valu_issue_slots"] * 4 / (SIMDS * CLOCK_HZ * sec),
+                    "mfma_busy_frac": counters["mfma_busy_cycles"] / (SIMDS * CLOCK_HZ * sec),
+                    "valu_issue": "SQ_ACTIVE_INST_VALU slots x 4 cycles / (1024 SIMDs x 2.4 GHz x time)",
                     "algorithmic": {"achieved": algorithmic, "frac": algorithmic / peak,
-                                    "convention": "262 flop per dPIE Hessian halo*px (division, sqrt = 8 each); "
-                                                  "this kernel has no division or sqrt, so the convention "
-                                                  "overstates its work and can exceed the peak"}}
+                                    "convention": "262 flop per dPIE Hessian halo*px (division, sqrt = 8 each) as if every "
+                                                  "halo were summed at every pixel; the tile expansions sum most "
+                                                  "of them at nodes that many pixels share, so it exceeds the peak"}}
     else:
         roofline = {"bound": "valu", "achieved": algorithmic, "peak": peak, "unit": "TFLOP/s",
-                    "frac": algorithmic / peak, "traffic": traffic,
+                    "frac": algorithmic / peak, "traffic": None,
                     "flops": "algorithmic convention: 262 flop per dPIE Hessian halo*px (division, sqrt = 8 each)"}
 
     res = {

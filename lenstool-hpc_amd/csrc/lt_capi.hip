@@ -116,6 +116,7 @@ struct DevModel {
 // fields 256^2 19 / 9, 400^2 19 / 20.
 bool split_halos(const ModelCost& model, int kind, int precision, const GridDesc& whole)
 {
+    if (whole.ny > 65535) return false;  // a work-group per row, in a dimension of the grid that may hold no more
     const double npix = (double)whole.nx * (double)whole.ny, cost = direct_cost(model, kind, precision);
     if (precision == LT_PREC_FP32C) return npix <= std::min(6e5, (kind == LT_MAP_POT ? 100. : 75.) * cost);
     return npix <= std::min(1e6, 52. * cost);
