@@ -357,7 +357,8 @@ __global__ void k_delense_finish(const double* __restrict__ gx, const double* __
 // chi^2 matching (src/chi_computation.cpp:10-195, with its two early-stopping loop conditions at
 // :110 and :118): a wavefront per sample, a lane per source writes the per-image chi terms; the wavefront
 // then sums them in the reference's order, 64 terms loaded at a time (one thread that loaded each as it
-// summed took 15 us for a sample of 120 images, 36 for 1024 samples).
+// summed took 15 us for a sample of 120 images, 36 for 1024 samples). The matching is a serial chain on what it indexes by
+// image, so that lies in LDS: 14 us a sample with the sum, 20 from private arrays in memory.
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ double pdist(double ax, double ay, double bx, double by)
 {
@@ -366,60 +367,79 @@ __device__ __forceinline__ double pdist(double ax, double ay, double bx, double 
     return sqrt(x * x + y * y);
 }
 
-__device__ __forceinline__ void chi_match(const DelenseDesc& d, int s, int k)
+// Per lane: the family's observed and found images and the matching's state, in LDS (indexed by image: in private
+// arrays they live in memory).
+struct ChiLds {
+    double ox[LT_MAXIMPERSOURCE][64], oy[LT_MAXIMPERSOURCE][64], fx[LT_MAXIMPERSOURCE][64], fy[LT_MAXIMPERSOURCE][64];
+    double tx[LT_MAXIMPERSOURCE][64], ty[LT_MAXIMPERSOURCE][64], dist[LT_MAXIMPERSOURCE][64];
+    int nfound[LT_MAXIMPERSOURCE][64];
+};
+
+__device__ __forceinline__ void chi_match(const DelenseDesc& d, int s, int k, int nf, ChiLds& m)
 {
 #pragma clang fp contract(off)
+    const int l = threadIdx.x;
     const int64_t sk = (int64_t)s * d.nsets + k;
     const int first = d.first_image[k], ni = d.nimages[k];
-    int nfound[LT_MAXIMPERSOURCE];
-    double tx[LT_MAXIMPERSOURCE], ty[LT_MAXIMPERSOURCE], dist[LT_MAXIMPERSOURCE];
-    for (int i = 0; i < LT_MAXIMPERSOURCE; ++i) {
-        nfound[i] = 0;
-        tx[i] = ty[i] = 0.;
+#pragma unroll 4
+    for (int i = 0; i < ni; ++i) {
+        m.ox[i][l] = d.img_x[first + i];
+        m.oy[i][l] = d.img_y[first + i];
+        m.tx[i][l] = m.ty[i][l] = 0.;
+        m.nfound[i][l] = 0;
     }
-    const int nf = d.loc[sk];
+#pragma unroll 4
+    for (int i = 0; i < nf; ++i) {
+        m.fx[i][l] = d.pos_x[sk * LT_MAXIMPERSOURCE + i];
+        m.fy[i][l] = d.pos_y[sk * LT_MAXIMPERSOURCE + i];
+    }
     for (int ii = 0; ii < nf; ++ii) {
-        const double px = d.pos_x[sk * LT_MAXIMPERSOURCE + ii], py = d.pos_y[sk * LT_MAXIMPERSOURCE + ii];
+        const double px = m.fx[ii][l], py = m.fy[ii][l];
         int idx = 0;
-        dist[0] = pdist(px, py, d.img_x[first], d.img_y[first]);
+        double least = pdist(px, py, m.ox[0][l], m.oy[0][l]);
+        m.dist[0][l] = least;
         for (int i = 1; i < ni; i++) {
-            dist[i] = pdist(px, py, d.img_x[first + i], d.img_y[first + i]);
-            if (dist[i] < dist[idx]) idx = i;
+            const double v = pdist(px, py, m.ox[i][l], m.oy[i][l]);
+            m.dist[i][l] = v;
+            if (v < least) {
+                idx = i;
+                least = v;
+            }
         }
-        if (nfound[idx] == 0) {
-            tx[idx] = px;
-            ty[idx] = py;
-            nfound[idx]++;
-        } else if (nfound[idx] > 0) {
+        if (m.nfound[idx][l] == 0) {
+            m.tx[idx][l] = px;
+            m.ty[idx][l] = py;
+            m.nfound[idx][l]++;
+        } else if (m.nfound[idx][l] > 0) {
             double tmpx, tmpy;
-            if (dist[idx] < pdist(d.img_x[first + idx], d.img_y[first + idx], tx[idx], ty[idx])) {
-                tmpx = tx[idx];
-                tmpy = ty[idx];
-                tx[idx] = px;
-                ty[idx] = py;
+            if (least < pdist(m.ox[idx][l], m.oy[idx][l], m.tx[idx][l], m.ty[idx][l])) {
+                tmpx = m.tx[idx][l];
+                tmpy = m.ty[idx][l];
+                m.tx[idx][l] = px;
+                m.ty[idx][l] = py;
             } else {
                 tmpx = px;
                 tmpy = py;
             }
             int second = 0;
             for (int i = 1; i < ni && (i != idx); i++)
-                if (dist[i] > dist[second]) second = i;
-            for (int i = 0; i < ni && nfound[i] == 0; i++) {
-                if (dist[i] < dist[second]) {
+                if (m.dist[i][l] > m.dist[second][l]) second = i;
+            for (int i = 0; i < ni && m.nfound[i][l] == 0; i++) {
+                if (m.dist[i][l] < m.dist[second][l]) {
                     second = i;
                     idx = i;
-                    tx[idx] = tmpx;
-                    ty[idx] = tmpy;
+                    m.tx[idx][l] = tmpx;
+                    m.ty[idx][l] = tmpy;
                 }
             }
-            nfound[idx]++;
+            m.nfound[idx][l]++;
         }
     }
     for (int i = 0; i < ni; i++) {
         double term;
-        if (nfound[i] > 0) {
-            double p1 = d.img_x[first + i] - tx[i];
-            double p2 = d.img_y[first + i] - ty[i];
+        if (m.nfound[i][l] > 0) {
+            double p1 = m.ox[i][l] - m.tx[i][l];
+            double p2 = m.oy[i][l] - m.ty[i][l];
             term = p1 * p1 + p2 * p2;
         } else {
             term = 1000. * ni;
@@ -431,11 +451,13 @@ __device__ __forceinline__ void chi_match(const DelenseDesc& d, int s, int k)
 __global__ __launch_bounds__(64) void k_chi(DelenseDesc d)
 {
 #pragma clang fp contract(off)
+    __shared__ ChiLds lds;
     const int s = blockIdx.x, lane = threadIdx.x;
     int found = 0;
     for (int k = lane; k < d.nsets; k += 64) {
-        chi_match(d, s, k);
-        found += d.loc[(int64_t)s * d.nsets + k];
+        const int nf = d.loc[(int64_t)s * d.nsets + k];
+        chi_match(d, s, k, nf, lds);
+        found += nf;
     }
     __syncthreads();  // the terms are written
     const double* const terms = d.terms + (int64_t)s * d.nimg_total;
