@@ -104,22 +104,38 @@ struct DevModel {
     FarRec* frecs = nullptr;
     Run* runs = nullptr;
     int nruns = 0;
+    bool unit = true;  // every run's weight is 1
     FarStats far;  // of the model (of a batch's first sample) as it was created
 };
 
-// Small maps: the halos of a row segment shared by several waves (lt_kernels64.hip), whatever px is asked for (every
-// px gives the same map). The sums through LDS cost about as much as 300 instructions a pixel, so the lighter the
-// model the earlier one wave per segment is enough: measured (us, one wave / split) 64^2 258 halos fields 97 / 14,
-// potential 392 / 44; 200^2 102 / 40 and 396 / 142; 512^2 168 / 150 and 667 / 543; 30 halos fields 256^2 14 / 8,
-// 400^2 20 / 16, 512^2 21 / 23; 11 halos (1 dPIE + 10 SIS) 200^2 8 / 8, 400^2 7 / 9. FP32C: 258 halos gradient 512^2
-// 166 / 166, 724^2 338 / 321, 1024^2 534 / 609; 60 mixed halos gradient 256^2 31 / 20, 400^2 33 / 52; 30 halos
-// fields 256^2 19 / 9, 400^2 19 / 20.
-bool split_halos(const ModelCost& model, int kind, int precision, const GridDesc& whole)
+bool unit_weights(const std::vector<Run>& runs)
 {
-    if (whole.ny > 65535) return false;  // a work-group per row, in a dimension of the grid that may hold no more
-    const double npix = (double)whole.nx * (double)whole.ny, cost = direct_cost(model, kind, precision);
-    if (precision == LT_PREC_FP32C) return npix <= std::min(6e5, (kind == LT_MAP_POT ? 100. : 75.) * cost);
-    return npix <= std::min(1e6, 52. * cost);
+    return std::all_of(runs.begin(), runs.end(), [](const Run& r) { return r.weight == 1.0; });
+}
+
+// Small maps: the halos of a row segment in eight parts (lt_kernels64.hip), whatever px is asked for (every
+// px gives the same map), up to this many pixels (0: never). Whether a map is summed so depends on the map alone, so
+// that a batch equals its single maps: a wave takes each part where the launch (all samples of a batch) has no more pixels
+// than that either, one wave takes them all where it has.
+//
+// Waves: the sums through LDS cost about as much as 300 instructions a pixel, so the lighter the model the earlier one
+// wave per segment is enough: measured (us, one wave / split) 64^2 258 halos fields 97 / 14, potential 392 / 44; 200^2
+// 102 / 40 and 396 / 142; 512^2 168 / 150 and 667 / 543; 30 halos fields 256^2 14 / 8, 400^2 20 / 16, 512^2 21 / 23;
+// FP32C: 258 halos gradient 512^2 166 / 166, 724^2 338 / 321, 1024^2 534 / 609; 60 mixed halos gradient 256^2 31 / 20,
+// 400^2 33 / 52; 30 halos fields 256^2 19 / 9, 400^2 19 / 20.
+//
+// Batches, where one wave takes the parts: each part of a run costs a start of its loop and the sums' additions, so a
+// part has to hold some work (kPart instructions a pixel); below that there is nothing to gain for single maps either
+// (11 halos: 7 us in both forms). Measured over 256 maps (us, plain sums / a wave for each part / one wave for all): 100^2, 60
+// mixed halos, magnitudes 265 / 335 / 283, FP32C 208 / 740 / 220, displacement 518 / 549 / 543, FP32C 288 / 1120 / 321;
+// 103 dPIE, shear 599 / 661 / 610, FP32C 405 / 900 / 425. 11 halos, magnitudes: 46 / 110, FP32C 45 / 231, now plain.
+double split_pixels(const ModelCost& model, int kind, int precision)
+{
+    const double cost = direct_cost(model, kind, precision);
+    static const double kPart[4] = {55., 75., 75., 35.};  // gradient, Hessian, potential, trace
+    if (cost < kPart[family_of(kind)] * model.nparts[precision == LT_PREC_FP32C]) return 0.;
+    if (precision == LT_PREC_FP32C) return std::min(6e5, (kind == LT_MAP_POT ? 100. : 75.) * cost);
+    return std::min(1e6, 52. * cost);
 }
 
 // Launch the kernel that produces map `kind` from a device model. `whole`: the grid that g is rows of.
@@ -158,21 +174,26 @@ int launch_map(const DevModel& m, int kind, int mode, double* const outs[5], dou
         if (e != hipSuccess) return hip_fail(e, "kernel launch");
         return LT_OK;
     }
-    if (px != LT_PX_HALO_LANES && split_halos(m.far.cost, kind, precision, whole)) px = kPxSplit;
+    // (a work-group per row in SUM_WAVES, in a dimension of the grid that may hold no more than 65535)
+    const double npix = (double)whole.nx * (double)whole.ny, most = split_pixels(m.far.cost, kind, precision);
+    if (px != LT_PX_HALO_LANES && whole.ny <= 65535 && npix <= most)
+        px = npix * std::max(g.nsamples, 1) <= most ? kPxSplit : kPxParts;
+    GridDesc gp = g;
+    gp.parts = m.far.cost.parts[precision == LT_PREC_FP32C];
     switch (kind) {
     case LT_MAP_GRADIENT:
     case LT_MAP_DPL:
-        if (precision == LT_PREC_FP32C) e = launch_gradient32(m.recs, m.recs32, m.runs, m.nruns, g, o, px, s);
-        else e = launch_gradient64(m.recs, m.runs, m.nruns, g, o, px, s);
+        if (precision == LT_PREC_FP32C) e = launch_gradient32(m.recs, m.recs32, m.runs, m.nruns, gp, o, px, s);
+        else e = launch_gradient64(m.recs, m.runs, m.nruns, gp, o, px, s);
         break;
     case LT_MAP_POT:
-        if (precision == LT_PREC_FP32C) e = launch_potential32(m.recs, m.recs32, m.runs, m.nruns, g, o, px, s);
-        else e = launch_potential64(m.recs, m.runs, m.nruns, g, o, px, s);
+        if (precision == LT_PREC_FP32C) e = launch_potential32(m.recs, m.recs32, m.runs, m.nruns, gp, o, px, s);
+        else e = launch_potential64(m.recs, m.runs, m.nruns, gp, o, px, s);
         break;
     default:
         // FP32C covers the Hessian-derived and the gradient maps
-        if (precision == LT_PREC_FP32C) e = launch_hessian32(m.recs, m.recs32, m.runs, m.nruns, g, o, px, s);
-        else e = launch_hessian64(m.recs, m.runs, m.nruns, g, o, px, s);
+        if (precision == LT_PREC_FP32C) e = launch_hessian32(m.recs, m.recs32, m.runs, m.nruns, gp, o, px, m.unit, s);
+        else e = launch_hessian64(m.recs, m.runs, m.nruns, gp, o, px, m.unit, s);
         break;
     }
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
@@ -270,6 +291,7 @@ int host_map(int kind, int mode, Use use, double* const host_out[5], const lt_gr
     m.frecs = (FarRec*)(base + rec_bytes + rec32_bytes);
     m.runs = (Run*)(base + off_runs);
     m.nruns = (int)runs.size();
+    m.unit = unit_weights(runs);
 
     double* dev_out[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     for (int k = 0; k < np; ++k)
@@ -715,6 +737,7 @@ int lt_model_create_batch(lt_model* out, const lt_potential_soa* lenses, int nsa
     m->dm.frecs = (FarRec*)(b + m->rec_bytes + m->rec32_bytes);
     m->dm.runs = (Run*)(b + off_runs);
     m->dm.nruns = (int)runs.size();
+    m->dm.unit = unit_weights(runs);
     if ((st = stage_samples(m, lenses, nsamples))) {
         free_model(m);
         return st;

@@ -127,7 +127,7 @@ struct GridDesc {
     int64_t halo_stride;
     int64_t plane_stride;
     int32_t nsamples;
-    int32_t pad;
+    int32_t parts;  // SUM_PARTS (lt_terms64.h): bit p set when part p of the model's sum has halos
 };
 
 // What the epilogue writes. kind / mode follow lt_status.h (LT_MAP_*).

@@ -11,12 +11,17 @@
 
 namespace lt {
 
-// px of a launch in the split form (lt_kernels64.hip): several waves share a row segment's halos
-constexpr int kPxSplit = -1;
+// parts of a pixel's sum in the split form (lt_kernels64.hip), and the halos of an FP32C chunk (lt_kernels32.hip)
+constexpr int kSplit = 8;
+constexpr int kChunk32 = 8;
 
-// FP64 kernels (lt_kernels64.hip). px = pixels per thread (1, 2 or 4) or kPxSplit.
+// px of a launch in the split form: a wave for each part of a row segment's halos, or the same sums by one wave
+constexpr int kPxSplit = -1;
+constexpr int kPxParts = -2;
+
+// FP64 kernels (lt_kernels64.hip). px = pixels per thread (1, 2 or 4), kPxSplit or kPxParts; unit: every run's weight is 1.
 hipError_t launch_hessian64(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
-                            const OutDesc& o, int px, hipStream_t s);
+                            const OutDesc& o, int px, bool unit, hipStream_t s);
 hipError_t launch_gradient64(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
                              const OutDesc& o, int px, hipStream_t s);
 hipError_t launch_potential64(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
@@ -32,7 +37,7 @@ hipError_t launch_epilogue64(const double* a, const double* b, const double* c, 
 
 // FP32-compensated kernels (lt_kernels32.hip).
 hipError_t launch_hessian32(const HaloRec* halos64, const HaloRec32* halos32, const Run* runs, int nruns,
-                            const GridDesc& g, const OutDesc& o, int px, hipStream_t s);
+                            const GridDesc& g, const OutDesc& o, int px, bool unit, hipStream_t s);
 // gradient / displacement maps; the model must be packed for gradient use (GradRec32 records)
 hipError_t launch_gradient32(const HaloRec* halos64, const HaloRec32* recs32, const Run* runs, int nruns,
                              const GridDesc& g, const OutDesc& o, int px, hipStream_t s);
@@ -60,6 +65,9 @@ enum : int { FAM_GRADIENT = 0, FAM_HESSIAN = 1, FAM_POTENTIAL = 2, FAM_TRACE = 3
 
 struct ModelCost {
     double px[4] = {0, 0, 0, 0};
+    // the split form's parts, in FP64 and in FP32C (where a part is whole chunks): which have halos, and over the runs how many
+    int parts[2] = {0, 0};
+    double nparts[2] = {0, 0};
 };
 
 int family_of(int kind);

@@ -35,9 +35,9 @@
 
 namespace lt {
 
-constexpr int CHUNK = 8;
+constexpr int CHUNK = kChunk32;
 
-// the split form (lt_kernels64.hip) by whole chunks: this wave's first chunk of a run, then every SPLIT-th
+// a part of a run (lt_terms64.h) by whole chunks: its first chunk, then every SPLIT-th
 template <int SPLIT>
 __device__ __forceinline__ int first_chunk(int start, int wave)
 {
@@ -64,6 +64,18 @@ __device__ __forceinline__ void stage_tile(Rec* __restrict__ tile, const Rec* __
     const float4* src = reinterpret_cast<const float4*>(recs + i0);
     float4* dst = reinterpret_cast<float4*>(tile);
     for (int j = threadIdx.y * WAVE + threadIdx.x; j < n * V; j += THREADS) dst[j] = src[j];
+}
+
+// the same for n chunks of a part, STEP records apart from recs[i0], one behind the other; of the records before `end`
+template <int THREADS, int STEP, typename Rec>
+__device__ __forceinline__ void stage_chunks(Rec* __restrict__ tile, const Rec* __restrict__ recs, int i0, int n, int end)
+{
+    constexpr int V = sizeof(Rec) / 16;
+    float4* dst = reinterpret_cast<float4*>(tile);
+    for (int j = threadIdx.y * WAVE + threadIdx.x; j < n * CHUNK * V; j += THREADS) {
+        const int c = j / (CHUNK * V), rec = i0 + c * STEP + j % (CHUNK * V) / V;
+        if (rec < end) dst[j] = reinterpret_cast<const float4*>(recs + rec)[j % V];
+    }
 }
 
 // Record j of a tile by value, only its first NV 16-byte vectors read (the fields the FP32 terms
@@ -311,30 +323,22 @@ __device__ __forceinline__ bool past_det_guard(double T, double D, double B, dou
     return __builtin_fabs(1. - kap) + gb > kDetGuard;
 }
 
-template <int PX, int KIND, int SPLIT>
-__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_hessian32(const HaloRec* __restrict__ h64,
-                                                          const HaloRec32* __restrict__ h32,
-                                                          const Run* __restrict__ runs, int nruns,
-                                                          GridDesc g, OutDesc o)
+// part `wave` of SPLIT of the Hessian sums at PX pixels of a row, run by run (UNIT: lt_kernels64.hip)
+template <int PX, int SPLIT, bool UNIT>
+__device__ __forceinline__ void hessian_sums32(const HaloRec* __restrict__ h64, const HaloRec32* __restrict__ h32,
+                                               const Run* __restrict__ runs, int nruns, int wave, const double* px,
+                                               double py, double* tT, double* tD, double* tB)
 {
-    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
-    if (row >= g.ny) return;
-    h64 = select_sample(g, h64, o);
-    h32 += (int64_t)blockIdx.z * g.halo_stride;
-    const int col0 = blockIdx.x * (WAVE * PX) + threadIdx.x;
-    const double py = pixel_coord(g.ymin, row + g.jstart, g.dy);
-    double px[PX];
-#pragma unroll
-    for (int k = 0; k < PX; ++k) px[k] = pixel_coord(g.xmin, col0 + k * WAVE + g.istart, g.dx);
-    double tT[PX], tD[PX], tB[PX];
 #pragma unroll
     for (int k = 0; k < PX; ++k) tT[k] = tD[k] = tB[k] = 0.;
     for (int r = 0; r < nruns; ++r) {
         const Run run = runs[r];
-        double sT[PX], sD[PX], sB[PX];
+        const int first = run.type == TYPE_SHEAR ? first_halo<SPLIT>(run.start, wave) : first_chunk<SPLIT>(run.start, wave);
+        if (SPLIT > 1 && first >= run.start + run.count) continue;
+        double rT[PX], rD[PX], rB[PX];
+        double *const sT = UNIT ? tT : rT, *const sD = UNIT ? tD : rD, *const sB = UNIT ? tB : rB;
 #pragma unroll
-        for (int k = 0; k < PX; ++k) sT[k] = sD[k] = sB[k] = 0.;
+        for (int k = 0; k < PX; ++k) rT[k] = rD[k] = rB[k] = 0.;
         const int end = run.start + run.count;
         if (run.type == TYPE_SHEAR) {
             for (int i = first_halo<SPLIT>(run.start, wave); i < end; i += SPLIT) {
@@ -355,6 +359,7 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_hessian32(
         } else {
             run32<TYPE_SIS, PX, SPLIT>(h64, h32, wave, run.start, end, px, py, sT, sD, sB);
         }
+        if (UNIT) continue;
         const double w = run.weight;
 #pragma unroll
         for (int k = 0; k < PX; ++k) {
@@ -363,11 +368,44 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_hessian32(
             tB[k] = __builtin_fma(w, sB[k], tB[k]);
         }
     }
-    if constexpr (SPLIT > 1) {
+}
+
+template <int PX, int KIND, int FORM, bool UNIT>
+__global__ __launch_bounds__(WAVE* rows_of(FORM), FORM == SUM_PARTS && PX == 2 ? 6 : 1) void k_hessian32(const HaloRec* __restrict__ h64,
+                                                                   const HaloRec32* __restrict__ h32,
+                                                                   const Run* __restrict__ runs, int nruns, GridDesc g,
+                                                                   OutDesc o)
+{
+    const int wave = FORM == SUM_WAVES ? __builtin_amdgcn_readfirstlane(threadIdx.y) : 0;
+    const int row = FORM == SUM_WAVES ? blockIdx.y : blockIdx.y * ROWS + threadIdx.y;
+    if (row >= g.ny) return;
+    h64 = select_sample(g, h64, o);
+    h32 += (int64_t)blockIdx.z * g.halo_stride;
+    const int col0 = blockIdx.x * (WAVE * PX) + threadIdx.x;
+    const double py = pixel_coord(g.ymin, row + g.jstart, g.dy);
+    double px[PX];
+#pragma unroll
+    for (int k = 0; k < PX; ++k) px[k] = pixel_coord(g.xmin, col0 + k * WAVE + g.istart, g.dx);
+    double tT[PX], tD[PX], tB[PX];
+    if constexpr (FORM == SUM_PARTS) {
+#pragma unroll
+        for (int k = 0; k < PX; ++k) tT[k] = tD[k] = tB[k] = 0.;
+#pragma unroll 1
+        for (int m = g.parts; m; m &= m - 1) {
+            double sT[PX], sD[PX], sB[PX];
+            hessian_sums32<PX, kSplit, UNIT>(h64, h32, runs, nruns, __builtin_ctz(m), px, py, sT, sD, sB);
+            add_part<PX>(tT, sT);
+            add_part<PX>(tD, sD);
+            add_part<PX>(tB, sB);
+        }
+    } else {
+        hessian_sums32<PX, parts_of(FORM), UNIT>(h64, h32, runs, nruns, wave, px, py, tT, tD, tB);
+    }
+    if constexpr (FORM == SUM_WAVES) {
         if constexpr (KIND == LT_MAP_MASS) {
-            if (!split_sum<PX, SPLIT>(wave, tT)) return;
+            if (!split_sum<PX, kSplit>(wave, tT)) return;
         } else {
-            if (!split_sum<PX, SPLIT>(wave, tT, tD, tB)) return;
+            if (!split_sum<PX, kSplit>(wave, tT, tD, tB)) return;
         }
         const int col = col0 + wave * WAVE;
         if constexpr (KIND == LT_MAP_FIELDS || KIND == LT_MAP_AMPLI || KIND == LT_MAP_SHEAR) {
@@ -391,18 +429,18 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_hessian32(
     }
 }
 
-template <int PX, int SPLIT>
+template <int PX, int FORM, bool UNIT = false>
 static hipError_t launch_hessian32_px(const HaloRec* h64, const HaloRec32* h32, const Run* runs, int nruns,
                                       const GridDesc& g, const OutDesc& o, hipStream_t s)
 {
     dim3 blk, grd;
-    geometry<PX, SPLIT>(g, grd, blk);
+    geometry<PX, FORM>(g, grd, blk);
     switch (o.kind) {
-    case LT_MAP_FIELDS: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_FIELDS, SPLIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
-    case LT_MAP_AMPLI: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_AMPLI, SPLIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
-    case LT_MAP_SHEAR: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_SHEAR, SPLIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
-    case LT_MAP_MASS: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_MASS, SPLIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
-    default: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_HESSIAN, SPLIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
+    case LT_MAP_FIELDS: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_FIELDS, FORM, UNIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
+    case LT_MAP_AMPLI: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_AMPLI, FORM, UNIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
+    case LT_MAP_SHEAR: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_SHEAR, FORM, UNIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
+    case LT_MAP_MASS: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_MASS, FORM, UNIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
+    default: hipLaunchKernelGGL((k_hessian32<PX, LT_MAP_HESSIAN, FORM, UNIT>), grd, blk, 0, s, h64, h32, runs, nruns, g, o); break;
     }
     return hipGetLastError();
 }
@@ -690,14 +728,22 @@ static hipError_t launch_hessian32h(const HaloRec* h64, const HaloRec32* h32, co
 }
 
 hipError_t launch_hessian32(const HaloRec* h64, const HaloRec32* h32, const Run* runs, int nruns, const GridDesc& g,
-                            const OutDesc& o, int px, hipStream_t s)
+                            const OutDesc& o, int px, bool unit, hipStream_t s)
 {
     switch (px) {
-    case kPxSplit: return launch_hessian32_px<1, kSplit>(h64, h32, runs, nruns, g, o, s);
-    case 1: return launch_hessian32_px<1, 1>(h64, h32, runs, nruns, g, o, s);
-    case 4: return launch_hessian32_px<4, 1>(h64, h32, runs, nruns, g, o, s);
+    case kPxSplit:
+        return unit ? launch_hessian32_px<1, SUM_WAVES, true>(h64, h32, runs, nruns, g, o, s)
+                    : launch_hessian32_px<1, SUM_WAVES>(h64, h32, runs, nruns, g, o, s);
+    case kPxParts:
+        if (parts_px(g, 1.45) == 1)
+            return unit ? launch_hessian32_px<1, SUM_PARTS, true>(h64, h32, runs, nruns, g, o, s)
+                        : launch_hessian32_px<1, SUM_PARTS>(h64, h32, runs, nruns, g, o, s);
+        return unit ? launch_hessian32_px<2, SUM_PARTS, true>(h64, h32, runs, nruns, g, o, s)
+                    : launch_hessian32_px<2, SUM_PARTS>(h64, h32, runs, nruns, g, o, s);
+    case 1: return launch_hessian32_px<1, SUM_PLAIN>(h64, h32, runs, nruns, g, o, s);
+    case 4: return launch_hessian32_px<4, SUM_PLAIN>(h64, h32, runs, nruns, g, o, s);
     case LT_PX_HALO_LANES: return launch_hessian32h(h64, h32, runs, nruns, g, o, s);
-    default: return launch_hessian32_px<2, 1>(h64, h32, runs, nruns, g, o, s);
+    default: return launch_hessian32_px<2, SUM_PLAIN>(h64, h32, runs, nruns, g, o, s);
     }
 }
 
@@ -788,75 +834,118 @@ __device__ __forceinline__ void grad_sis32_circ(const GradRec32& h, float tx, fl
     gy = __builtin_fmaf(s, ty, gy);
 }
 
-// Halos [t0, t1) of a run, their FP32 records in tile[0 .. t1 - t0): FP32 terms summed per chunk of
-// CHUNK halos, FP64 terms (near lanes) straight into the FP64 run sums
-template <int TYPE, int PX, int SPLIT>
-__device__ __forceinline__ void tileg32(const HaloRec* __restrict__ h64, const GradRec32* __restrict__ tile, int first,
-                                        int t0, int t1, const double* px, double py, double* sx, double* sy)
+// A chunk [c0, c1) of a run, its FP32 records in recs[0 .. c1 - c0): FP32 terms summed over the chunk, FP64 terms (near
+// lanes) straight into the FP64 run sums
+template <int TYPE, int PX>
+__device__ __forceinline__ void chunkg32(const HaloRec* __restrict__ h64, const GradRec32* __restrict__ recs, int c0,
+                                         int c1, const double* px, double py, double* sx, double* sy)
 {
-    for (int c0 = t0 + first; c0 < t1; c0 += CHUNK * SPLIT) {
-        const int c1 = min(c0 + CHUNK, t1);
-        float fx[PX], fy[PX];
+    float fx[PX], fy[PX];
 #pragma unroll
-        for (int k = 0; k < PX; ++k) fx[k] = fy[k] = 0.f;
-        for (int i = c0; i < c1; ++i) {
-            const GradRec32 h = hot_fields<5>(tile, i - t0);  // cs .. circ
-            const double xh = h64[i].xh;
-            const float ty = (float)(py - h64[i].yh);
-            const float ty2 = ty * ty;
-#pragma unroll
-            for (int k = 0; k < PX; ++k) {
-                const float tx = offset_x(xh, px[k]);
-                if (__builtin_fmaf(tx, tx, ty2) < h.near2) {
-                    const HaloRec& hd = h64[i];
-                    if constexpr (TYPE == TYPE_DPIE) grad_piemd<true>(hd, px[k], py, sx[k], sy[k]);
-                    else if constexpr (TYPE == TYPE_PIEMD) grad_piemd<false>(hd, px[k], py, sx[k], sy[k]);
-                    else if constexpr (TYPE == TYPE_SIS_CIRC) grad_sis_circ(hd, px[k], py, sx[k], sy[k]);
-                    else grad_sis(hd, px[k], py, sx[k], sy[k]);
-                } else {
-                    if constexpr (TYPE == TYPE_DPIE) grad_piemd32<true>(h, tx, ty, fx[k], fy[k]);
-                    else if constexpr (TYPE == TYPE_PIEMD) grad_piemd32<false>(h, tx, ty, fx[k], fy[k]);
-                    else if constexpr (TYPE == TYPE_SIS_CIRC) grad_sis32_circ(h, tx, ty, fx[k], fy[k]);
-                    else grad_sis32(h, tx, ty, fx[k], fy[k]);
-                }
-            }
-        }
+    for (int k = 0; k < PX; ++k) fx[k] = fy[k] = 0.f;
+    for (int i = c0; i < c1; ++i) {
+        const GradRec32 h = hot_fields<5>(recs, i - c0);  // cs .. circ
+        const double xh = h64[i].xh;
+        const float ty = (float)(py - h64[i].yh);
+        const float ty2 = ty * ty;
 #pragma unroll
         for (int k = 0; k < PX; ++k) {
-            sx[k] += (double)fx[k];
-            sy[k] += (double)fy[k];
+            const float tx = offset_x(xh, px[k]);
+            if (__builtin_fmaf(tx, tx, ty2) < h.near2) {
+                const HaloRec& hd = h64[i];
+                if constexpr (TYPE == TYPE_DPIE) grad_piemd<true>(hd, px[k], py, sx[k], sy[k]);
+                else if constexpr (TYPE == TYPE_PIEMD) grad_piemd<false>(hd, px[k], py, sx[k], sy[k]);
+                else if constexpr (TYPE == TYPE_SIS_CIRC) grad_sis_circ(hd, px[k], py, sx[k], sy[k]);
+                else grad_sis(hd, px[k], py, sx[k], sy[k]);
+            } else {
+                if constexpr (TYPE == TYPE_DPIE) grad_piemd32<true>(h, tx, ty, fx[k], fy[k]);
+                else if constexpr (TYPE == TYPE_PIEMD) grad_piemd32<false>(h, tx, ty, fx[k], fy[k]);
+                else if constexpr (TYPE == TYPE_SIS_CIRC) grad_sis32_circ(h, tx, ty, fx[k], fy[k]);
+                else grad_sis32(h, tx, ty, fx[k], fy[k]);
+            }
         }
+    }
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+        sx[k] += (double)fx[k];
+        sy[k] += (double)fy[k];
     }
 }
 
 // One run of halos of one type, its FP32 records staged tile by tile (staged: 12.9 ms on the
 // 503-halo 4096^2 map, scalar loads: 13.9 ms). Called by every thread of the work-group with the
-// same run (the barriers need all of them).
-template <int TYPE, int PX, int SPLIT>
+// same run (the barriers need all of them). SUM_PARTS: a part's chunks alone, eight to a tile.
+template <int TYPE, int PX, int FORM>
 __device__ __forceinline__ void rung32(const HaloRec* __restrict__ h64, const GradRec32* __restrict__ g32,
                                        GradRec32* __restrict__ tile, int wave, int start, int end, const double* px, double py,
                                        double* sx, double* sy)
 {
+    constexpr int threads = WAVE * rows_of(FORM);
+    if constexpr (FORM == SUM_PARTS) {
+        constexpr int step = CHUNK * kSplit;  // from a chunk of the part to the next
+        for (int t0 = first_chunk<kSplit>(start, wave); t0 < end; t0 += TILE / CHUNK * step) {
+            const int n = min(TILE / CHUNK, (end - t0 + step - 1) / step);
+            __syncthreads();  // every wave is done with the previous tile
+            stage_chunks<threads, step>(tile, g32, t0, n, end);
+            __syncthreads();
+            for (int c = 0; c < n; ++c) {
+                const int c0 = t0 + c * step;
+                chunkg32<TYPE, PX>(h64, tile + c * CHUNK, c0, min(c0 + CHUNK, end), px, py, sx, sy);
+            }
+        }
+        return;
+    }
+    constexpr int SPLIT = parts_of(FORM);
+    // a tile is TILE / CHUNK = kSplit chunks, so a wave's first chunk is the same in every tile of the run
+    const int first = first_chunk<SPLIT>(start, wave) - start;
     for (int t0 = start; t0 < end; t0 += TILE) {
         const int t1 = min(t0 + TILE, end);
         __syncthreads();  // every wave is done with the previous tile
-        stage_tile<WAVE*(SPLIT == 1 ? ROWS : SPLIT)>(tile, g32, t0, t1 - t0);
+        stage_tile<threads>(tile, g32, t0, t1 - t0);
         __syncthreads();
-        // a tile is TILE / CHUNK = SPLIT chunks, so a wave's first chunk is the same in every tile of the run
-        tileg32<TYPE, PX, SPLIT>(h64, tile, first_chunk<SPLIT>(start, wave) - start, t0, t1, px, py, sx, sy);
+        for (int c0 = t0 + first; c0 < t1; c0 += CHUNK * SPLIT)
+            chunkg32<TYPE, PX>(h64, tile + (c0 - t0), c0, min(c0 + CHUNK, t1), px, py, sx, sy);
     }
 }
 
-template <int PX, int SPLIT>
-__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_gradient32(const HaloRec* __restrict__ h64,
-                                                           const GradRec32* __restrict__ g32,
-                                                           const Run* __restrict__ runs, int nruns, GridDesc g,
-                                                           OutDesc o)
+// part `wave` of the gradient sums at PX pixels of a row, run by run
+template <int PX, int FORM>
+__device__ __forceinline__ void gradient_sums32(const HaloRec* __restrict__ h64, const GradRec32* __restrict__ g32,
+                                                GradRec32* __restrict__ tile, const Run* __restrict__ runs, int nruns,
+                                                int wave, const double* px, double py, double* tx, double* ty)
+{
+#pragma unroll
+    for (int k = 0; k < PX; ++k) tx[k] = ty[k] = 0.;
+    for (int r = 0; r < nruns; ++r) {
+        const Run run = runs[r];
+        double rx[PX], ry[PX];  // a part's terms are added to its sums as they come
+        double *const sx = FORM == SUM_PLAIN ? rx : tx, *const sy = FORM == SUM_PLAIN ? ry : ty;
+#pragma unroll
+        for (int k = 0; k < PX; ++k) rx[k] = ry[k] = 0.;
+        const int end = run.start + run.count;
+        if (run.type == TYPE_DPIE) rung32<TYPE_DPIE, PX, FORM>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
+        else if (run.type == TYPE_PIEMD) rung32<TYPE_PIEMD, PX, FORM>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
+        else if (run.circ) rung32<TYPE_SIS_CIRC, PX, FORM>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
+        else rung32<TYPE_SIS, PX, FORM>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
+        if (FORM != SUM_PLAIN) continue;
+#pragma unroll
+        for (int k = 0; k < PX; ++k) {
+            tx[k] += sx[k];
+            ty[k] += sy[k];
+        }
+    }
+}
+
+template <int PX, int FORM>
+__global__ __launch_bounds__(WAVE* rows_of(FORM)) void k_gradient32(const HaloRec* __restrict__ h64,
+                                                                    const GradRec32* __restrict__ g32,
+                                                                    const Run* __restrict__ runs, int nruns, GridDesc g,
+                                                                    OutDesc o)
 {
     // rows past the grid walk the runs too (the tile barriers need every thread) and store nothing
     __shared__ GradRec32 tile[TILE];
-    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
+    const int wave = FORM == SUM_WAVES ? __builtin_amdgcn_readfirstlane(threadIdx.y) : 0;
+    const int row = FORM == SUM_WAVES ? blockIdx.y : blockIdx.y * ROWS + threadIdx.y;
     const bool live = row < g.ny;
     h64 = select_sample(g, h64, o);
     g32 += (int64_t)blockIdx.z * g.halo_stride;
@@ -864,29 +953,23 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_gradient32
     const double py = pixel_coord(g.ymin, row + g.jstart, g.dy);
     double px[PX], tx[PX], ty[PX];
 #pragma unroll
-    for (int k = 0; k < PX; ++k) {
-        px[k] = pixel_coord(g.xmin, col0 + k * WAVE + g.istart, g.dx);
-        tx[k] = ty[k] = 0.;
-    }
-    for (int r = 0; r < nruns; ++r) {
-        const Run run = runs[r];
-        double sx[PX], sy[PX];
+    for (int k = 0; k < PX; ++k) px[k] = pixel_coord(g.xmin, col0 + k * WAVE + g.istart, g.dx);
+    if constexpr (FORM == SUM_PARTS) {
 #pragma unroll
-        for (int k = 0; k < PX; ++k) sx[k] = sy[k] = 0.;
-        const int end = run.start + run.count;
-        if (run.type == TYPE_DPIE) rung32<TYPE_DPIE, PX, SPLIT>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
-        else if (run.type == TYPE_PIEMD) rung32<TYPE_PIEMD, PX, SPLIT>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
-        else if (run.circ) rung32<TYPE_SIS_CIRC, PX, SPLIT>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
-        else rung32<TYPE_SIS, PX, SPLIT>(h64, g32, tile, wave, run.start, end, px, py, sx, sy);
-#pragma unroll
-        for (int k = 0; k < PX; ++k) {
-            tx[k] += sx[k];
-            ty[k] += sy[k];
+        for (int k = 0; k < PX; ++k) tx[k] = ty[k] = 0.;
+#pragma unroll 1
+        for (int m = g.parts; m; m &= m - 1) {
+            double sx[PX], sy[PX];
+            gradient_sums32<PX, FORM>(h64, g32, tile, runs, nruns, __builtin_ctz(m), px, py, sx, sy);
+            add_part<PX>(tx, sx);
+            add_part<PX>(ty, sy);
         }
+    } else {
+        gradient_sums32<PX, FORM>(h64, g32, tile, runs, nruns, wave, px, py, tx, ty);
     }
     const double m = o.kind == LT_MAP_DPL ? o.r : 1.0;
-    if constexpr (SPLIT > 1) {
-        if (!split_sum<PX, SPLIT>(wave, tx, ty)) return;
+    if constexpr (FORM == SUM_WAVES) {
+        if (!split_sum<PX, kSplit>(wave, tx, ty)) return;
         const int col = col0 + wave * WAVE;
         if (live && col < g.nx) {
             const int64_t idx = (int64_t)row * g.pitch + col;
@@ -906,13 +989,13 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_gradient32
     }
 }
 
-template <int PX, int SPLIT>
+template <int PX, int FORM>
 static void launch_gradient32_px(const HaloRec* h64, const GradRec32* g32, const Run* runs, int nruns,
                                  const GridDesc& g, const OutDesc& o, hipStream_t s)
 {
     dim3 blk, grd;
-    geometry<PX, SPLIT>(g, grd, blk);
-    hipLaunchKernelGGL((k_gradient32<PX, SPLIT>), grd, blk, 0, s, h64, g32, runs, nruns, g, o);
+    geometry<PX, FORM>(g, grd, blk);
+    hipLaunchKernelGGL((k_gradient32<PX, FORM>), grd, blk, 0, s, h64, g32, runs, nruns, g, o);
 }
 
 hipError_t launch_gradient32(const HaloRec* h64, const HaloRec32* recs32, const Run* runs, int nruns,
@@ -920,10 +1003,14 @@ hipError_t launch_gradient32(const HaloRec* h64, const HaloRec32* recs32, const 
 {
     const GradRec32* g32 = reinterpret_cast<const GradRec32*>(recs32);
     switch (px) {
-    case kPxSplit: launch_gradient32_px<1, kSplit>(h64, g32, runs, nruns, g, o, s); break;
-    case 1: launch_gradient32_px<1, 1>(h64, g32, runs, nruns, g, o, s); break;
-    case 4: launch_gradient32_px<4, 1>(h64, g32, runs, nruns, g, o, s); break;
-    default: launch_gradient32_px<2, 1>(h64, g32, runs, nruns, g, o, s); break;
+    case kPxSplit: launch_gradient32_px<1, SUM_WAVES>(h64, g32, runs, nruns, g, o, s); break;
+    case kPxParts:
+        if (parts_px(g, 1.2) == 1) launch_gradient32_px<1, SUM_PARTS>(h64, g32, runs, nruns, g, o, s);
+        else launch_gradient32_px<2, SUM_PARTS>(h64, g32, runs, nruns, g, o, s);
+        break;
+    case 1: launch_gradient32_px<1, SUM_PLAIN>(h64, g32, runs, nruns, g, o, s); break;
+    case 4: launch_gradient32_px<4, SUM_PLAIN>(h64, g32, runs, nruns, g, o, s); break;
+    default: launch_gradient32_px<2, SUM_PLAIN>(h64, g32, runs, nruns, g, o, s); break;
     }
     return hipGetLastError();
 }
@@ -1050,14 +1137,39 @@ __device__ __forceinline__ void runp32(const HaloRec* __restrict__ h64, const Po
     }
 }
 
+// part `wave` of SPLIT of the potential at PX pixels of a row, run by run
 template <int PX, int SPLIT>
-__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_potential32(const HaloRec* __restrict__ h64,
-                                                            const PotRec32* __restrict__ p32,
-                                                            const Run* __restrict__ runs, int nruns, GridDesc g,
-                                                            OutDesc o)
+__device__ __forceinline__ void potential_sums32(const HaloRec* __restrict__ h64, const PotRec32* __restrict__ p32,
+                                                 const Run* __restrict__ runs, int nruns, int wave, const double* px,
+                                                 double py, double* tot, float* mn)
 {
-    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
+#pragma unroll
+    for (int k = 0; k < PX; ++k) tot[k] = 0.;
+    for (int r = 0; r < nruns; ++r) {
+        const Run run = runs[r];
+        if (SPLIT > 1 && first_chunk<SPLIT>(run.start, wave) >= run.start + run.count) continue;
+        double rs[PX];
+        double* const s = SPLIT > 1 ? tot : rs;
+#pragma unroll
+        for (int k = 0; k < PX; ++k) rs[k] = 0.;
+        const int end = run.start + run.count;
+        if (run.type == TYPE_DPIE) runp32<TYPE_DPIE, PX, SPLIT>(h64, p32, wave, run.start, end, px, py, s, mn);
+        else if (run.type == TYPE_PIEMD) runp32<TYPE_PIEMD, PX, SPLIT>(h64, p32, wave, run.start, end, px, py, s, mn);
+        else runp32<TYPE_SIS, PX, SPLIT>(h64, p32, wave, run.start, end, px, py, s, mn);
+        if (SPLIT > 1) continue;
+#pragma unroll
+        for (int k = 0; k < PX; ++k) tot[k] += s[k];
+    }
+}
+
+template <int PX, int FORM>
+__global__ __launch_bounds__(WAVE* rows_of(FORM)) void k_potential32(const HaloRec* __restrict__ h64,
+                                                                     const PotRec32* __restrict__ p32,
+                                                                     const Run* __restrict__ runs, int nruns, GridDesc g,
+                                                                     OutDesc o)
+{
+    const int wave = FORM == SUM_WAVES ? __builtin_amdgcn_readfirstlane(threadIdx.y) : 0;
+    const int row = FORM == SUM_WAVES ? blockIdx.y : blockIdx.y * ROWS + threadIdx.y;
     if (row >= g.ny) return;
     h64 = select_sample(g, h64, o);
     p32 += (int64_t)blockIdx.z * g.halo_stride;
@@ -1068,27 +1180,26 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_potential3
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
         px[k] = pixel_coord(g.xmin, col0 + k * WAVE + g.istart, g.dx);
-        tot[k] = 0.;
         mn[k] = 1.f;
     }
-    for (int r = 0; r < nruns; ++r) {
-        const Run run = runs[r];
-        double s[PX];
+    if constexpr (FORM == SUM_PARTS) {
 #pragma unroll
-        for (int k = 0; k < PX; ++k) s[k] = 0.;
-        const int end = run.start + run.count;
-        if (run.type == TYPE_DPIE) runp32<TYPE_DPIE, PX, SPLIT>(h64, p32, wave, run.start, end, px, py, s, mn);
-        else if (run.type == TYPE_PIEMD) runp32<TYPE_PIEMD, PX, SPLIT>(h64, p32, wave, run.start, end, px, py, s, mn);
-        else runp32<TYPE_SIS, PX, SPLIT>(h64, p32, wave, run.start, end, px, py, s, mn);
-#pragma unroll
-        for (int k = 0; k < PX; ++k) tot[k] += s[k];
+        for (int k = 0; k < PX; ++k) tot[k] = 0.;
+#pragma unroll 1
+        for (int m = g.parts; m; m &= m - 1) {
+            double s[PX];
+            potential_sums32<PX, kSplit>(h64, p32, runs, nruns, __builtin_ctz(m), px, py, s, mn);
+            add_part<PX>(tot, s);
+        }
+    } else {
+        potential_sums32<PX, parts_of(FORM)>(h64, p32, runs, nruns, wave, px, py, tot, mn);
     }
-    if constexpr (SPLIT > 1) {
+    if constexpr (FORM == SUM_WAVES) {
         // a wave that met a PIEMD centre makes the sum NaN
 #pragma unroll
         for (int k = 0; k < PX; ++k)
             if (mn[k] == 0.f) tot[k] = __builtin_nan("");
-        if (!split_sum<PX, SPLIT>(wave, tot)) return;
+        if (!split_sum<PX, kSplit>(wave, tot)) return;
         const int col = col0 + wave * WAVE;
         if (col < g.nx) o.p0[(int64_t)row * g.pitch + col] = tot[0] * o.mult;
         return;
@@ -1102,13 +1213,13 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_potential3
     }
 }
 
-template <int PX, int SPLIT>
+template <int PX, int FORM>
 static void launch_potential32_px(const HaloRec* h64, const PotRec32* p32, const Run* runs, int nruns,
                                   const GridDesc& g, const OutDesc& o, hipStream_t s)
 {
     dim3 blk, grd;
-    geometry<PX, SPLIT>(g, grd, blk);
-    hipLaunchKernelGGL((k_potential32<PX, SPLIT>), grd, blk, 0, s, h64, p32, runs, nruns, g, o);
+    geometry<PX, FORM>(g, grd, blk);
+    hipLaunchKernelGGL((k_potential32<PX, FORM>), grd, blk, 0, s, h64, p32, runs, nruns, g, o);
 }
 
 hipError_t launch_potential32(const HaloRec* h64, const HaloRec32* recs32, const Run* runs, int nruns,
@@ -1116,10 +1227,14 @@ hipError_t launch_potential32(const HaloRec* h64, const HaloRec32* recs32, const
 {
     const PotRec32* p32 = reinterpret_cast<const PotRec32*>(recs32);
     switch (px) {
-    case kPxSplit: launch_potential32_px<1, kSplit>(h64, p32, runs, nruns, g, o, s); break;
-    case 1: launch_potential32_px<1, 1>(h64, p32, runs, nruns, g, o, s); break;
-    case 4: launch_potential32_px<4, 1>(h64, p32, runs, nruns, g, o, s); break;
-    default: launch_potential32_px<2, 1>(h64, p32, runs, nruns, g, o, s); break;
+    case kPxSplit: launch_potential32_px<1, SUM_WAVES>(h64, p32, runs, nruns, g, o, s); break;
+    case kPxParts:
+        if (parts_px(g, 1.1) == 1) launch_potential32_px<1, SUM_PARTS>(h64, p32, runs, nruns, g, o, s);
+        else launch_potential32_px<2, SUM_PARTS>(h64, p32, runs, nruns, g, o, s);
+        break;
+    case 1: launch_potential32_px<1, SUM_PLAIN>(h64, p32, runs, nruns, g, o, s); break;
+    case 4: launch_potential32_px<4, SUM_PLAIN>(h64, p32, runs, nruns, g, o, s); break;
+    default: launch_potential32_px<2, SUM_PLAIN>(h64, p32, runs, nruns, g, o, s); break;
     }
     return hipGetLastError();
 }

@@ -3,9 +3,10 @@
 // covers 64*PX columns of 4 rows. Halo records are walked in wavefront-uniform order, run by run.
 //
 // Small maps leave most of the chip idle that way: 200 x 200 pixels are 313 waves of two pixels a lane for
-// 1024 SIMDs, each walking every halo one record load after another. The split form (SPLIT > 1) gives a
-// row segment of 64 PX pixels to SPLIT waves, wave s taking halos s, s + SPLIT, .. of the model (so that every
-// wave has its share of each type), and adds their sums through LDS in the order of the waves.
+// 1024 SIMDs, each walking every halo one record load after another. The split form (SUM_WAVES) gives a
+// row segment of 64 PX pixels to kSplit waves, wave s taking halos s, s + kSplit, .. of the model (so that every
+// wave has its share of each type), and adds their sums through LDS in the order of the waves. A batch of small
+// maps fills the chip with a wave per segment: SUM_PARTS forms the same parts and sums one after another.
 //
 // Formulas (restated from the mathematics; reference equivalents cited):
 //   SIS gradient  src/gradient.cpp:260-299      PIEMD gradient  src/gradient.hpp:64-76,
@@ -21,28 +22,21 @@
 
 namespace lt {
 
-template <int PX, int KIND, int SPLIT>
-__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_hessian64(const HaloRec* __restrict__ halos,
-                                                          const Run* __restrict__ runs, int nruns,
-                                                          GridDesc g, OutDesc o)
+// part `wave` of SPLIT of the Hessian sums at PX pixels of a row, run by run. UNIT: every run's weight is 1 and its terms
+// are added to the part's sums as they come, with no sums of the run's own.
+template <int PX, int SPLIT, bool UNIT>
+__device__ __forceinline__ void hessian_sums(const HaloRec* __restrict__ halos, const Run* __restrict__ runs, int nruns,
+                                             int wave, const double* px, double py, double* tT, double* tD, double* tB)
 {
-    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
-    if (row >= g.ny) return;
-    halos = select_sample(g, halos, o);
-    const int col0 = blockIdx.x * (WAVE * PX) + threadIdx.x;
-    const double py = pixel_coord(g.ymin, row + g.jstart, g.dy);
-    double px[PX];
-#pragma unroll
-    for (int k = 0; k < PX; ++k) px[k] = pixel_coord(g.xmin, col0 + k * WAVE + g.istart, g.dx);
-    double tT[PX], tD[PX], tB[PX];
 #pragma unroll
     for (int k = 0; k < PX; ++k) tT[k] = tD[k] = tB[k] = 0.;
     for (int r = 0; r < nruns; ++r) {
         const Run run = runs[r];
-        double sT[PX], sD[PX], sB[PX];
+        if (SPLIT > 1 && first_halo<SPLIT>(run.start, wave) >= run.start + run.count) continue;
+        double rT[PX], rD[PX], rB[PX];
+        double *const sT = UNIT ? tT : rT, *const sD = UNIT ? tD : rD, *const sB = UNIT ? tB : rB;
 #pragma unroll
-        for (int k = 0; k < PX; ++k) sT[k] = sD[k] = sB[k] = 0.;
+        for (int k = 0; k < PX; ++k) rT[k] = rD[k] = rB[k] = 0.;
         const int end = run.start + run.count;
         switch (run.type) {
         case TYPE_DPIE:
@@ -88,6 +82,7 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_hessian64(
             }
             break;
         }
+        if (UNIT) continue;
         const double w = run.weight;
 #pragma unroll
         for (int k = 0; k < PX; ++k) {
@@ -96,11 +91,42 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_hessian64(
             tB[k] = __builtin_fma(w, sB[k], tB[k]);
         }
     }
-    if constexpr (SPLIT > 1) {
+}
+
+template <int PX, int KIND, int FORM, bool UNIT>
+__global__ __launch_bounds__(WAVE* rows_of(FORM), FORM == SUM_PARTS && PX == 2 ? 5 : 1) void k_hessian64(const HaloRec* __restrict__ halos,
+                                                                   const Run* __restrict__ runs, int nruns, GridDesc g,
+                                                                   OutDesc o)
+{
+    const int wave = FORM == SUM_WAVES ? __builtin_amdgcn_readfirstlane(threadIdx.y) : 0;
+    const int row = FORM == SUM_WAVES ? blockIdx.y : blockIdx.y * ROWS + threadIdx.y;
+    if (row >= g.ny) return;
+    halos = select_sample(g, halos, o);
+    const int col0 = blockIdx.x * (WAVE * PX) + threadIdx.x;
+    const double py = pixel_coord(g.ymin, row + g.jstart, g.dy);
+    double px[PX];
+#pragma unroll
+    for (int k = 0; k < PX; ++k) px[k] = pixel_coord(g.xmin, col0 + k * WAVE + g.istart, g.dx);
+    double tT[PX], tD[PX], tB[PX];
+    if constexpr (FORM == SUM_PARTS) {
+#pragma unroll
+        for (int k = 0; k < PX; ++k) tT[k] = tD[k] = tB[k] = 0.;
+#pragma unroll 1
+        for (int m = g.parts; m; m &= m - 1) {
+            double sT[PX], sD[PX], sB[PX];
+            hessian_sums<PX, kSplit, UNIT>(halos, runs, nruns, __builtin_ctz(m), px, py, sT, sD, sB);
+            add_part<PX>(tT, sT);
+            add_part<PX>(tD, sD);
+            add_part<PX>(tB, sB);
+        }
+    } else {
+        hessian_sums<PX, parts_of(FORM), UNIT>(halos, runs, nruns, wave, px, py, tT, tD, tB);
+    }
+    if constexpr (FORM == SUM_WAVES) {
         if constexpr (KIND == LT_MAP_MASS) {
-            if (!split_sum<PX, SPLIT>(wave, tT)) return;
+            if (!split_sum<PX, kSplit>(wave, tT)) return;
         } else {
-            if (!split_sum<PX, SPLIT>(wave, tT, tD, tB)) return;
+            if (!split_sum<PX, kSplit>(wave, tT, tD, tB)) return;
         }
         const int col = col0 + wave * WAVE;
         if (col < g.nx) hess_epilogue<KIND>(o, (int64_t)row * g.pitch + col, tT[0], tD[0], tB[0]);
@@ -113,28 +139,20 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_hessian64(
     }
 }
 
+// the same of the gradient sums
 template <int PX, int SPLIT>
-__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_gradient64(const HaloRec* __restrict__ halos,
-                                                           const Run* __restrict__ runs, int nruns,
-                                                           GridDesc g, OutDesc o)
+__device__ __forceinline__ void gradient_sums(const HaloRec* __restrict__ halos, const Run* __restrict__ runs, int nruns,
+                                              int wave, const double* px, double py, double* tx, double* ty)
 {
-    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
-    if (row >= g.ny) return;
-    halos = select_sample(g, halos, o);
-    const int col0 = blockIdx.x * (WAVE * PX) + threadIdx.x;
-    const double py = pixel_coord(g.ymin, row + g.jstart, g.dy);
-    double px[PX], tx[PX], ty[PX];
 #pragma unroll
-    for (int k = 0; k < PX; ++k) {
-        px[k] = pixel_coord(g.xmin, col0 + k * WAVE + g.istart, g.dx);
-        tx[k] = ty[k] = 0.;
-    }
+    for (int k = 0; k < PX; ++k) tx[k] = ty[k] = 0.;
     for (int r = 0; r < nruns; ++r) {
         const Run run = runs[r];
-        double sx[PX], sy[PX];
+        if (SPLIT > 1 && first_halo<SPLIT>(run.start, wave) >= run.start + run.count) continue;
+        double rx[PX], ry[PX];  // a part's terms are added to its sums as they come
+        double *const sx = SPLIT > 1 ? tx : rx, *const sy = SPLIT > 1 ? ty : ry;
 #pragma unroll
-        for (int k = 0; k < PX; ++k) sx[k] = sy[k] = 0.;
+        for (int k = 0; k < PX; ++k) rx[k] = ry[k] = 0.;
         const int end = run.start + run.count;
         switch (run.type) {
         case TYPE_DPIE:
@@ -169,15 +187,45 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_gradient64
             }
             break;
         }
+        if (SPLIT > 1) continue;
 #pragma unroll
         for (int k = 0; k < PX; ++k) {
             tx[k] += sx[k];
             ty[k] += sy[k];
         }
     }
+}
+
+template <int PX, int FORM>
+__global__ __launch_bounds__(WAVE* rows_of(FORM)) void k_gradient64(const HaloRec* __restrict__ halos,
+                                                                    const Run* __restrict__ runs, int nruns, GridDesc g,
+                                                                    OutDesc o)
+{
+    const int wave = FORM == SUM_WAVES ? __builtin_amdgcn_readfirstlane(threadIdx.y) : 0;
+    const int row = FORM == SUM_WAVES ? blockIdx.y : blockIdx.y * ROWS + threadIdx.y;
+    if (row >= g.ny) return;
+    halos = select_sample(g, halos, o);
+    const int col0 = blockIdx.x * (WAVE * PX) + threadIdx.x;
+    const double py = pixel_coord(g.ymin, row + g.jstart, g.dy);
+    double px[PX], tx[PX], ty[PX];
+#pragma unroll
+    for (int k = 0; k < PX; ++k) px[k] = pixel_coord(g.xmin, col0 + k * WAVE + g.istart, g.dx);
+    if constexpr (FORM == SUM_PARTS) {
+#pragma unroll
+        for (int k = 0; k < PX; ++k) tx[k] = ty[k] = 0.;
+#pragma unroll 1
+        for (int m = g.parts; m; m &= m - 1) {
+            double sx[PX], sy[PX];
+            gradient_sums<PX, kSplit>(halos, runs, nruns, __builtin_ctz(m), px, py, sx, sy);
+            add_part<PX>(tx, sx);
+            add_part<PX>(ty, sy);
+        }
+    } else {
+        gradient_sums<PX, parts_of(FORM)>(halos, runs, nruns, wave, px, py, tx, ty);
+    }
     const double m = o.kind == LT_MAP_DPL ? o.r : 1.0;
-    if constexpr (SPLIT > 1) {
-        if (!split_sum<PX, SPLIT>(wave, tx, ty)) return;
+    if constexpr (FORM == SUM_WAVES) {
+        if (!split_sum<PX, kSplit>(wave, tx, ty)) return;
         const int col = col0 + wave * WAVE;
         if (col < g.nx) {
             const int64_t idx = (int64_t)row * g.pitch + col;
@@ -197,13 +245,38 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_gradient64
     }
 }
 
+// the same of the potential; mn = min(mn, rem^2) over the part's PIEMD and dPIE halos
 template <int PX, int SPLIT>
-__global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_potential64(const HaloRec* __restrict__ halos,
-                                                            const Run* __restrict__ runs, int nruns,
-                                                            GridDesc g, OutDesc o)
+__device__ __forceinline__ void potential_sums(const HaloRec* __restrict__ halos, const Run* __restrict__ runs, int nruns,
+                                               int wave, const double* px, double py, double* tot, double* mn)
 {
-    const int wave = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int row = SPLIT == 1 ? blockIdx.y * ROWS + threadIdx.y : blockIdx.y;
+#pragma unroll
+    for (int k = 0; k < PX; ++k) tot[k] = 0.;
+    for (int r = 0; r < nruns; ++r) {
+        const Run run = runs[r];
+        if (SPLIT > 1 && first_halo<SPLIT>(run.start, wave) >= run.start + run.count) continue;
+        double rs[PX];
+        double* const s = SPLIT > 1 ? tot : rs;
+#pragma unroll
+        for (int k = 0; k < PX; ++k) rs[k] = 0.;
+        for (int i = first_halo<SPLIT>(run.start, wave); i < run.start + run.count; i += SPLIT) {
+            const HaloRec& h = halos[i];
+#pragma unroll
+            for (int k = 0; k < PX; ++k) s[k] += pot_halo(h, run.type, px[k], py, mn[k]);
+        }
+        if (SPLIT > 1) continue;
+#pragma unroll
+        for (int k = 0; k < PX; ++k) tot[k] += s[k];
+    }
+}
+
+template <int PX, int FORM>
+__global__ __launch_bounds__(WAVE* rows_of(FORM)) void k_potential64(const HaloRec* __restrict__ halos,
+                                                                     const Run* __restrict__ runs, int nruns, GridDesc g,
+                                                                     OutDesc o)
+{
+    const int wave = FORM == SUM_WAVES ? __builtin_amdgcn_readfirstlane(threadIdx.y) : 0;
+    const int row = FORM == SUM_WAVES ? blockIdx.y : blockIdx.y * ROWS + threadIdx.y;
     if (row >= g.ny) return;
     halos = select_sample(g, halos, o);
     const int col0 = blockIdx.x * (WAVE * PX) + threadIdx.x;
@@ -212,28 +285,26 @@ __global__ __launch_bounds__(WAVE*(SPLIT == 1 ? ROWS : SPLIT)) void k_potential6
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
         px[k] = pixel_coord(g.xmin, col0 + k * WAVE + g.istart, g.dx);
-        tot[k] = 0.;
         mn[k] = 1.;
     }
-    for (int r = 0; r < nruns; ++r) {
-        const Run run = runs[r];
-        double s[PX];
+    if constexpr (FORM == SUM_PARTS) {
 #pragma unroll
-        for (int k = 0; k < PX; ++k) s[k] = 0.;
-        for (int i = first_halo<SPLIT>(run.start, wave); i < run.start + run.count; i += SPLIT) {
-            const HaloRec& h = halos[i];
-#pragma unroll
-            for (int k = 0; k < PX; ++k) s[k] += pot_halo(h, run.type, px[k], py, mn[k]);
+        for (int k = 0; k < PX; ++k) tot[k] = 0.;
+#pragma unroll 1
+        for (int m = g.parts; m; m &= m - 1) {
+            double s[PX];
+            potential_sums<PX, kSplit>(halos, runs, nruns, __builtin_ctz(m), px, py, s, mn);
+            add_part<PX>(tot, s);
         }
-#pragma unroll
-        for (int k = 0; k < PX; ++k) tot[k] += s[k];
+    } else {
+        potential_sums<PX, parts_of(FORM)>(halos, runs, nruns, wave, px, py, tot, mn);
     }
-    if constexpr (SPLIT > 1) {
+    if constexpr (FORM == SUM_WAVES) {
         // a wave that met a PIEMD centre makes the sum NaN
 #pragma unroll
         for (int k = 0; k < PX; ++k)
             if (mn[k] == 0.) tot[k] = __builtin_nan("");
-        if (!split_sum<PX, SPLIT>(wave, tot)) return;
+        if (!split_sum<PX, kSplit>(wave, tot)) return;
         const int col = col0 + wave * WAVE;
         if (col < g.nx) o.p0[(int64_t)row * g.pitch + col] = tot[0] * o.mult;
         return;
@@ -311,30 +382,38 @@ __global__ __launch_bounds__(256) void k_epilogue(const double* __restrict__ a, 
 // ------------------------------------------------------------------------------------------------
 // launchers
 // ------------------------------------------------------------------------------------------------
-template <int PX, int SPLIT>
+template <int PX, int FORM, bool UNIT = false>
 static hipError_t launch_hessian64_px(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
                                       const OutDesc& o, hipStream_t s)
 {
     dim3 blk, grd;
-    geometry<PX, SPLIT>(g, grd, blk);
+    geometry<PX, FORM>(g, grd, blk);
     switch (o.kind) {
-    case LT_MAP_FIELDS: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_FIELDS, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
-    case LT_MAP_AMPLI: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_AMPLI, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
-    case LT_MAP_SHEAR: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_SHEAR, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
-    case LT_MAP_MASS: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_MASS, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
-    default: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_HESSIAN, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
+    case LT_MAP_FIELDS: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_FIELDS, FORM, UNIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
+    case LT_MAP_AMPLI: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_AMPLI, FORM, UNIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
+    case LT_MAP_SHEAR: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_SHEAR, FORM, UNIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
+    case LT_MAP_MASS: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_MASS, FORM, UNIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
+    default: hipLaunchKernelGGL((k_hessian64<PX, LT_MAP_HESSIAN, FORM, UNIT>), grd, blk, 0, s, halos, runs, nruns, g, o); break;
     }
     return hipGetLastError();
 }
 
 hipError_t launch_hessian64(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
-                            const OutDesc& o, int px, hipStream_t s)
+                            const OutDesc& o, int px, bool unit, hipStream_t s)
 {
     switch (px) {
-    case kPxSplit: return launch_hessian64_px<1, kSplit>(halos, runs, nruns, g, o, s);
-    case 1: return launch_hessian64_px<1, 1>(halos, runs, nruns, g, o, s);
-    case 4: return launch_hessian64_px<4, 1>(halos, runs, nruns, g, o, s);
-    default: return launch_hessian64_px<2, 1>(halos, runs, nruns, g, o, s);
+    case kPxSplit:
+        return unit ? launch_hessian64_px<1, SUM_WAVES, true>(halos, runs, nruns, g, o, s)
+                    : launch_hessian64_px<1, SUM_WAVES>(halos, runs, nruns, g, o, s);
+    case kPxParts:
+        if (parts_px(g, 1.15) == 1)
+            return unit ? launch_hessian64_px<1, SUM_PARTS, true>(halos, runs, nruns, g, o, s)
+                        : launch_hessian64_px<1, SUM_PARTS>(halos, runs, nruns, g, o, s);
+        return unit ? launch_hessian64_px<2, SUM_PARTS, true>(halos, runs, nruns, g, o, s)
+                    : launch_hessian64_px<2, SUM_PARTS>(halos, runs, nruns, g, o, s);
+    case 1: return launch_hessian64_px<1, SUM_PLAIN>(halos, runs, nruns, g, o, s);
+    case 4: return launch_hessian64_px<4, SUM_PLAIN>(halos, runs, nruns, g, o, s);
+    default: return launch_hessian64_px<2, SUM_PLAIN>(halos, runs, nruns, g, o, s);
     }
 }
 
@@ -363,44 +442,52 @@ hipError_t launch_points_gradient64(const HaloRec* halos, const Run* runs, int n
     return hipGetLastError();
 }
 
-template <int PX, int SPLIT>
+template <int PX, int FORM>
 static void launch_gradient64_px(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g, const OutDesc& o,
                            hipStream_t s)
 {
     dim3 blk, grd;
-    geometry<PX, SPLIT>(g, grd, blk);
-    hipLaunchKernelGGL((k_gradient64<PX, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o);
+    geometry<PX, FORM>(g, grd, blk);
+    hipLaunchKernelGGL((k_gradient64<PX, FORM>), grd, blk, 0, s, halos, runs, nruns, g, o);
 }
 
 hipError_t launch_gradient64(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
                              const OutDesc& o, int px, hipStream_t s)
 {
     switch (px) {
-    case kPxSplit: launch_gradient64_px<1, kSplit>(halos, runs, nruns, g, o, s); break;
-    case 1: launch_gradient64_px<1, 1>(halos, runs, nruns, g, o, s); break;
-    case 4: launch_gradient64_px<4, 1>(halos, runs, nruns, g, o, s); break;
-    default: launch_gradient64_px<2, 1>(halos, runs, nruns, g, o, s); break;
+    case kPxSplit: launch_gradient64_px<1, SUM_WAVES>(halos, runs, nruns, g, o, s); break;
+    case kPxParts:
+        if (parts_px(g, 1.0) == 1) launch_gradient64_px<1, SUM_PARTS>(halos, runs, nruns, g, o, s);
+        else launch_gradient64_px<2, SUM_PARTS>(halos, runs, nruns, g, o, s);
+        break;
+    case 1: launch_gradient64_px<1, SUM_PLAIN>(halos, runs, nruns, g, o, s); break;
+    case 4: launch_gradient64_px<4, SUM_PLAIN>(halos, runs, nruns, g, o, s); break;
+    default: launch_gradient64_px<2, SUM_PLAIN>(halos, runs, nruns, g, o, s); break;
     }
     return hipGetLastError();
 }
 
-template <int PX, int SPLIT>
+template <int PX, int FORM>
 static void launch_potential64_px(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g, const OutDesc& o,
                            hipStream_t s)
 {
     dim3 blk, grd;
-    geometry<PX, SPLIT>(g, grd, blk);
-    hipLaunchKernelGGL((k_potential64<PX, SPLIT>), grd, blk, 0, s, halos, runs, nruns, g, o);
+    geometry<PX, FORM>(g, grd, blk);
+    hipLaunchKernelGGL((k_potential64<PX, FORM>), grd, blk, 0, s, halos, runs, nruns, g, o);
 }
 
 hipError_t launch_potential64(const HaloRec* halos, const Run* runs, int nruns, const GridDesc& g,
                               const OutDesc& o, int px, hipStream_t s)
 {
     switch (px) {
-    case kPxSplit: launch_potential64_px<1, kSplit>(halos, runs, nruns, g, o, s); break;
-    case 1: launch_potential64_px<1, 1>(halos, runs, nruns, g, o, s); break;
-    case 4: launch_potential64_px<4, 1>(halos, runs, nruns, g, o, s); break;
-    default: launch_potential64_px<2, 1>(halos, runs, nruns, g, o, s); break;
+    case kPxSplit: launch_potential64_px<1, SUM_WAVES>(halos, runs, nruns, g, o, s); break;
+    case kPxParts:
+        if (parts_px(g, 1.0) == 1) launch_potential64_px<1, SUM_PARTS>(halos, runs, nruns, g, o, s);
+        else launch_potential64_px<2, SUM_PARTS>(halos, runs, nruns, g, o, s);
+        break;
+    case 1: launch_potential64_px<1, SUM_PLAIN>(halos, runs, nruns, g, o, s); break;
+    case 4: launch_potential64_px<4, SUM_PLAIN>(halos, runs, nruns, g, o, s); break;
+    default: launch_potential64_px<2, SUM_PLAIN>(halos, runs, nruns, g, o, s); break;
     }
     return hipGetLastError();
 }

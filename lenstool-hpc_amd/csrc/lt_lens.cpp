@@ -1,6 +1,7 @@
 // lt_lens.cpp -- packs a caller's SOA lens model (the reference's Potential_SOA layout) into the
 // device halo records and runs. All per-halo constants of the closed forms are formed here, once
 // per model, in double precision.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <cstdio>
@@ -311,12 +312,19 @@ ModelCost model_cost(const std::vector<Run>& runs)
     static const double kDpie[4] = {126., 55., 228., 24.}, kPiemd[4] = {85., 34., 140., 15.},
                         kSis[4] = {34., 34., 40., 20.}, kCirc[4] = {17., 21., 40., 11.};
     ModelCost c;
-    for (const Run& r : runs)
+    for (const Run& r : runs) {
         for (int f = 0; f < 4; ++f)
             c.px[f] += r.count * (r.type == TYPE_DPIE    ? kDpie[f]
                                   : r.type == TYPE_PIEMD ? kPiemd[f]
                                   : r.type == TYPE_SIS   ? (r.circ ? kCirc[f] : kSis[f])
                                                          : 3.);
+        for (int prec = 0; prec < 2; ++prec) {
+            const int unit = prec && r.type != TYPE_SHEAR ? kChunk32 : 1;
+            const int n = std::min((r.count + unit - 1) / unit, kSplit);
+            for (int k = 0; k < n; ++k) c.parts[prec] |= 1 << ((r.start + k) & (kSplit - 1));
+            c.nparts[prec] += n;
+        }
+    }
     return c;
 }
 

@@ -12,6 +12,7 @@
 
 #include "lenstool_hip/lt_status.h"
 #include "lt_device.h"
+#include "lt_kernels.h"
 #include "lt_math.h"
 
 namespace lt {
@@ -488,7 +489,16 @@ __device__ __forceinline__ const HaloRec* select_sample(const GridDesc& g, const
     return halos + s * g.halo_stride;
 }
 
-// this wave's halos of a run: first, first + SPLIT, ..
+// How the halos of a pixel are summed: one after another by a wave; in kSplit parts (part p takes halos p, p + kSplit, ..
+// of the model) by as many waves, whose sums are then added in the order of the parts; or the same parts one after
+// another by one wave. The last two give the same bits: waves where a launch leaves the chip idle, one wave
+// where it does not (a batch of small maps).
+enum : int { SUM_PLAIN = 0, SUM_WAVES = 1, SUM_PARTS = 2 };
+
+constexpr int parts_of(int form) { return form == SUM_PLAIN ? 1 : kSplit; }
+constexpr int rows_of(int form) { return form == SUM_WAVES ? kSplit : ROWS; }  // waves of a work-group
+
+// the halos of a run that belong to part `wave`: first, first + SPLIT, ..
 template <int SPLIT>
 __device__ __forceinline__ int first_halo(int start, int wave)
 {
@@ -523,6 +533,15 @@ __device__ __forceinline__ bool split_sum(int wave, V&... v)
     return true;
 }
 
+// the sums t of a part, of PX pixels, added to those of the parts before it, in the order of split_sum() (a part without
+// halos is left out: it is +0 there)
+template <int PX>
+__device__ __forceinline__ void add_part(double* sum, const double* t)
+{
+#pragma unroll
+    for (int k = 0; k < PX; ++k) sum[k] += t[k];
+}
+
 // Launch geometry: a 64 x 4 work-group, PX pixels per thread along a row, blockIdx.z = sample.
 inline dim3 grid_for(const GridDesc& g, int px)
 {
@@ -530,16 +549,21 @@ inline dim3 grid_for(const GridDesc& g, int px)
                 (unsigned)(g.nsamples > 0 ? g.nsamples : 1));
 }
 
-// waves of a row segment in the split form
-constexpr int kSplit = 8;
-
-// launch geometry: SPLIT 1 as grid_for(); else a work-group per row and 64 PX columns
-template <int PX, int SPLIT>
+// launch geometry: as grid_for(); for SUM_WAVES a work-group per row and 64 PX columns
+template <int PX, int FORM>
 inline void geometry(const GridDesc& g, dim3& grd, dim3& blk)
 {
     grd = grid_for(g, PX);
-    blk = dim3(WAVE, SPLIT == 1 ? ROWS : SPLIT, 1);
-    if (SPLIT > 1) grd.y = (unsigned)g.ny;
+    blk = dim3(WAVE, rows_of(FORM), 1);
+    if (FORM == SUM_WAVES) grd.y = (unsigned)g.ny;
+}
+
+// pixels per thread of a SUM_PARTS launch: two, or one where the columns past the grid of two (whole segments of 128)
+// cost more than the record loads that two pixels share (`share`: times of one pixel a thread to two, measured)
+inline int parts_px(const GridDesc& g, double share)
+{
+    const auto cover = [&](int seg) { return (double)((g.nx + seg - 1) / seg * seg); };
+    return cover(WAVE) * share < cover(2 * WAVE) ? 1 : 2;
 }
 
 }  // namespace lt
