@@ -167,6 +167,23 @@ int lt_map_device(lt_model model, int kind, int mode, double* out0, double* out1
                   double* out4, double r, double mult, const lt_grid_desc* grid, int precision, int px,
                   void* stream);
 
+/* The form in which lt_map_device sums the map of `sample` of the model: from its types, halo count and run
+ * structure, the sample's own parameters and the grid, by estimated time. Maps of one lens in one form
+ * are equal bit for bit, in a batch or alone, updated or new; forms differ by rounding. The LT_FORM_TILES forms
+ * sum halos far from a tile of pixels at nodes of the tile, in FP64 also where FP32C is asked for; models of more than
+ * 2048 halos or 16 runs (of equal type, and dlsds for LT_MAP_MASS) do not take them. A captured launch
+ * sequence keeps the form of its capture: its replays with parameters staged later are maps of that form. */
+#define LT_FORM_PIXELS            0 /* every halo at every pixel                                           */
+#define LT_FORM_PARTS             1 /* the same in eight parts of the halos (small maps)                   */
+#define LT_FORM_TILES_64          2 /* tiles of 64 pixels, four waves                                      */
+#define LT_FORM_TILES_64_WIDE     3 /* 16 waves                                                            */
+#define LT_FORM_TILES_64_HALVES   4 /* two work-groups of 8                                                */
+#define LT_FORM_TILES_64_QUARTERS 5 /* four work-groups of 4                                               */
+#define LT_FORM_TILES_128         6
+#define LT_FORM_TILES_256         7
+#define LT_FORM_HALO_LANES        8 /* px = LT_PX_HALO_LANES                                               */
+int lt_map_form(lt_model model, int sample, int kind, const lt_grid_desc* grid, int precision, int px, int* form);
+
 /* Time the map with 1, 2 and 4 pixels per thread (one warm-up and two timed launches each, into
  * scratch planes) and make the fastest the default (px = 0) for maps of this family, precision,
  * halo-count octave and pixel-count octave in this process. ms[3] (optional) gets the per-launch

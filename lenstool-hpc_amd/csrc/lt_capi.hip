@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <map>
+#include <memory>
 #include <tuple>
 #include <cmath>
 #include <cstdio>
@@ -105,7 +106,12 @@ struct DevModel {
     Run* runs = nullptr;
     int nruns = 0;
     bool unit = true;  // every run's weight is 1
-    FarStats far;  // of the model (of a batch's first sample) as it was created
+};
+
+// What the forms of a model's maps go by (lt_far.h): of the model, and of each sample.
+struct LensStats {
+    FarStats far;
+    std::vector<double> density;
 };
 
 bool unit_weights(const std::vector<Run>& runs)
@@ -138,65 +144,108 @@ double split_pixels(const ModelCost& model, int kind, int precision)
     return std::min(1e6, 52. * cost);
 }
 
-// Launch the kernel that produces map `kind` from a device model. `whole`: the grid that g is rows of.
-int launch_map(const DevModel& m, int kind, int mode, double* const outs[5], double r, double mult,
+// The form in which a lens's map is summed. It depends on the model, the lens and the whole map alone, not on
+// the launch (a batch, rows of the map, pixels per thread) nor on what the model held before: equal forms of equal
+// lenses are equal bit for bit.
+struct Form {
+    FarShape shape = FarShape::Direct;
+    bool split = false;  // direct, in parts
+
+    bool operator==(const Form& o) const { return shape == o.shape && split == o.split; }
+};
+
+Form map_form(const FarStats& far, double density, int kind, int precision, const GridDesc& whole, int px)
+{
+    Form f;
+    if (px == LT_PX_HALO_LANES) return f;
+    // Large grids: the halo sums by tile expansions (lt_far.hip), in FP64 whatever precision is asked for
+    // (both cost less than the FP32C direct sum there, and the result is the FP64 map).
+    f.shape = far_shape(far, density, kind, precision, whole, nullptr);
+    if (f.shape != FarShape::Direct) return f;
+    // (a work-group per row in SUM_WAVES, in a dimension of the grid that may hold no more than 65535)
+    f.split = whole.ny <= 65535 && (double)whole.nx * (double)whole.ny <= split_pixels(far.cost, kind, precision);
+    return f;
+}
+
+// Launch the kernel that produces map `kind` of samples [s0, s0 + n) of a device model in form f; o's planes are those of
+// sample s0. `whole`: the grid that g is rows of.
+hipError_t launch_form(const DevModel& m, const ModelCost& cost, const Form& f, int s0, int n, OutDesc o, int mode, GridDesc g,
+                       const GridDesc& whole, int precision, int px, int nhalos, hipStream_t s)
+{
+    const int64_t at = (int64_t)s0 * g.halo_stride;
+    const HaloRec* const recs = m.recs + at;
+    const HaloRec32* const recs32 = m.recs32 + at;
+    g.nsamples = n;
+    if (f.shape != FarShape::Direct) {
+        if (o.kind == LT_MAP_AMPLI && mode == 5) {  // kappa: the Hessian's trace alone
+            o.kind = LT_MAP_MASS;
+            o.mult = 1.0;
+        }
+        return launch_far(recs, m.frecs + at, m.runs, m.nruns, nhalos, g, o, f.shape, s);
+    }
+    if (f.split) {
+        const double npix = (double)whole.nx * (double)whole.ny * n;
+        px = npix <= split_pixels(cost, o.kind, precision) ? kPxSplit : kPxParts;
+        g.parts = cost.parts[precision == LT_PREC_FP32C];
+    }
+    switch (o.kind) {
+    case LT_MAP_GRADIENT:
+    case LT_MAP_DPL:
+        return precision == LT_PREC_FP32C ? launch_gradient32(recs, recs32, m.runs, m.nruns, g, o, px, s)
+                                          : launch_gradient64(recs, m.runs, m.nruns, g, o, px, s);
+    case LT_MAP_POT:
+        return precision == LT_PREC_FP32C ? launch_potential32(recs, recs32, m.runs, m.nruns, g, o, px, s)
+                                          : launch_potential64(recs, m.runs, m.nruns, g, o, px, s);
+    default:
+        // FP32C covers the Hessian-derived and the gradient maps
+        return precision == LT_PREC_FP32C ? launch_hessian32(recs, recs32, m.runs, m.nruns, g, o, px, m.unit, s)
+                                          : launch_hessian64(recs, m.runs, m.nruns, g, o, px, m.unit, s);
+    }
+}
+
+// px as asked for (0: the default) and precision of a map of `kind`
+int check_launch(int kind, int precision, int px)
+{
+    // LT_PX_HALO_LANES exists for FP32C Hessian-derived maps (lanes over halos, lt_kernels32.hip)
+    const bool hessian_family = kind != LT_MAP_GRADIENT && kind != LT_MAP_DPL && kind != LT_MAP_POT;
+    if (px == LT_PX_HALO_LANES && !(hessian_family && precision == LT_PREC_FP32C))
+        return fail(LT_ERR_INVALID, "px = LT_PX_HALO_LANES applies to FP32C Hessian-derived maps only");
+    if (px != 0 && px != 1 && px != 2 && px != 4 && px != LT_PX_HALO_LANES)
+        return fail(LT_ERR_INVALID, "px must be 0, 1, 2, 4 or LT_PX_HALO_LANES");
+    if (precision != LT_PREC_FP64 && precision != LT_PREC_FP32C)
+        return fail(LT_ERR_INVALID, "precision must be LT_PREC_FP64 or LT_PREC_FP32C");
+    return LT_OK;
+}
+
+// Launch the kernels that produce map `kind` from a device model: one launch, or one for each sequence of samples of the
+// same form.
+int launch_map(const DevModel& m, const LensStats& lens, int kind, int mode, double* const outs[5], double r, double mult,
                const GridDesc& g, const GridDesc& whole, int precision, int px, hipStream_t s, int nhalos)
 {
     OutDesc o{};
-    o.p0 = outs[0];
-    o.p1 = outs[1];
-    o.p2 = outs[2];
-    o.p3 = outs[3];
-    o.p4 = outs[4];
+    double** const planes[5] = {&o.p0, &o.p1, &o.p2, &o.p3, &o.p4};
+    for (int k = 0; k < 5; ++k) *planes[k] = outs[k];
     o.kind = kind;
     o.mode = mode;
     o.r = r;
     o.mult = mult;
-    if (px <= 0) px = default_px(kind, precision, nhalos, (long long)g.nx * g.ny);
-    const bool hessian_family = kind != LT_MAP_GRADIENT && kind != LT_MAP_DPL && kind != LT_MAP_POT;
-    if (px == LT_PX_HALO_LANES && !(hessian_family && precision == LT_PREC_FP32C))
-        return fail(LT_ERR_INVALID, "px = LT_PX_HALO_LANES applies to FP32C Hessian-derived maps only");
-    if (px != 1 && px != 2 && px != 4 && px != LT_PX_HALO_LANES)
-        return fail(LT_ERR_INVALID, "px must be 0, 1, 2, 4 or LT_PX_HALO_LANES");
-    if (precision != LT_PREC_FP64 && precision != LT_PREC_FP32C)
-        return fail(LT_ERR_INVALID, "precision must be LT_PREC_FP64 or LT_PREC_FP32C");
-    hipError_t e;
-    // Large grids: the halo sums by tile expansions (lt_far.hip), in FP64 whatever precision is asked for
-    // (both cost less than the FP32C direct sum there, and the result is the FP64 map).
-    const FarShape shape = px == LT_PX_HALO_LANES ? FarShape::Direct : far_shape(m.far, kind, precision, whole, nullptr);
-    const bool tiled = shape != FarShape::Direct;
-    if (tiled) {
-        if (kind == LT_MAP_AMPLI && mode == 5) {  // kappa: the Hessian's trace alone
-            o.kind = LT_MAP_MASS;
-            o.mult = 1.0;
+    if (int st = check_launch(kind, precision, px)) return st;
+    if (px == 0) px = default_px(kind, precision, nhalos, (long long)g.nx * g.ny);
+    const int S = std::max(g.nsamples, 1);
+    const std::vector<double>& density = lens.density;
+    Form form = map_form(lens.far, density[0], kind, precision, whole, px);
+    for (int s0 = 0, s1; s0 < S; s0 = s1) {
+        Form next = form;
+        for (s1 = s0 + 1; s1 < S; ++s1) {
+            if (density[s1] != density[s1 - 1]) next = map_form(lens.far, density[s1], kind, precision, whole, px);
+            if (!(next == form)) break;
         }
-        e = launch_far(m.recs, m.frecs, m.runs, m.nruns, nhalos, g, o, shape, s);
+        const hipError_t e = launch_form(m, lens.far.cost, form, s0, s1 - s0, o, mode, g, whole, precision, px, nhalos, s);
         if (e != hipSuccess) return hip_fail(e, "kernel launch");
-        return LT_OK;
+        for (int k = 0; k < 5; ++k)
+            if (*planes[k]) *planes[k] += (size_t)(s1 - s0) * g.plane_stride;
+        form = next;
     }
-    // (a work-group per row in SUM_WAVES, in a dimension of the grid that may hold no more than 65535)
-    const double npix = (double)whole.nx * (double)whole.ny, most = split_pixels(m.far.cost, kind, precision);
-    if (px != LT_PX_HALO_LANES && whole.ny <= 65535 && npix <= most)
-        px = npix * std::max(g.nsamples, 1) <= most ? kPxSplit : kPxParts;
-    GridDesc gp = g;
-    gp.parts = m.far.cost.parts[precision == LT_PREC_FP32C];
-    switch (kind) {
-    case LT_MAP_GRADIENT:
-    case LT_MAP_DPL:
-        if (precision == LT_PREC_FP32C) e = launch_gradient32(m.recs, m.recs32, m.runs, m.nruns, gp, o, px, s);
-        else e = launch_gradient64(m.recs, m.runs, m.nruns, gp, o, px, s);
-        break;
-    case LT_MAP_POT:
-        if (precision == LT_PREC_FP32C) e = launch_potential32(m.recs, m.recs32, m.runs, m.nruns, gp, o, px, s);
-        else e = launch_potential64(m.recs, m.runs, m.nruns, gp, o, px, s);
-        break;
-    default:
-        // FP32C covers the Hessian-derived and the gradient maps
-        if (precision == LT_PREC_FP32C) e = launch_hessian32(m.recs, m.recs32, m.runs, m.nruns, gp, o, px, m.unit, s);
-        else e = launch_hessian64(m.recs, m.runs, m.nruns, gp, o, px, m.unit, s);
-        break;
-    }
-    if (e != hipSuccess) return hip_fail(e, "kernel launch");
     return LT_OK;
 }
 
@@ -307,8 +356,8 @@ int host_map(int kind, int mode, Use use, double* const host_out[5], const lt_gr
     g.jstart = jstart;
     g.pitch = nx;
     g.nsamples = 1;
-    m.far = far_stats(recs.data(), nhalos, runs);
-    if ((st = launch_map(m, kind, mode, dev_out, r, mult, g, g, precision, 0, S.stream, nhalos))) {
+    const LensStats lens_stats{far_stats(nhalos, runs), {halo_density(recs.data(), runs)}};
+    if ((st = launch_map(m, lens_stats, kind, mode, dev_out, r, mult, g, g, precision, 0, S.stream, nhalos))) {
         (void)hipStreamSynchronize(S.stream);  // the upload reads the pinned area
         return st;
     }
@@ -599,6 +648,9 @@ struct lt_model_s {
     std::vector<Run> runs_host;
     std::vector<int> types;
     DevModel dm;
+    // of the samples on the device, and of those in `staging`; a map takes `stats` as it finds it, whatever another
+    // thread stages or uploads meanwhile
+    std::shared_ptr<const LensStats> stats, staged_stats;
     size_t bytes = 0;
     size_t rec_bytes = 0, rec32_bytes = 0;  // all samples
     void* base = nullptr;                   // device: records [S*H], fp32 records [S*H], far records [S*H], runs
@@ -646,6 +698,8 @@ static int stage_samples(lt_model_s* m, const lt_potential_soa* lenses, int nsam
     std::string err;
     char* st = (char*)m->staging;
     std::vector<Run> batch_runs = m->runs_host;
+    auto stats = std::make_shared<LensStats>();
+    stats->density.resize(nsamples);
     for (int s = 0; s < nsamples; ++s) {
         const lt_potential_soa& L = lenses[s];
         for (int i = 0; i < H; ++i)
@@ -662,7 +716,10 @@ static int stage_samples(lt_model_s* m, const lt_potential_soa* lenses, int nsam
                         (size_t)H * sizeof(HaloRec32));
             far_records(recs.data(), H, (FarRec*)(st + m->rec_bytes + m->rec32_bytes) + (size_t)s * H);
         }
+        stats->density[s] = halo_density(recs.data(), runs);
     }
+    stats->far = far_stats(H, batch_runs);
+    m->staged_stats = stats;
     if (!batch_runs.empty()) std::memcpy(st + m->off_runs, batch_runs.data(), batch_runs.size() * sizeof(Run));
     return LT_OK;
 }
@@ -673,6 +730,7 @@ static int upload_staged(lt_model_s* m, hipStream_t s)
     const size_t n = m->off_runs + m->runs_host.size() * sizeof(Run);
     if (!n) return LT_OK;
     HIP_TRY(hipMemcpyAsync(m->base, m->staging, n, hipMemcpyHostToDevice, s));
+    std::atomic_store(&m->stats, m->staged_stats);
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing(s, &cs));
     if (cs == hipStreamCaptureStatusNone) {
@@ -715,7 +773,6 @@ int lt_model_create_batch(lt_model* out, const lt_potential_soa* lenses, int nsa
     m->nhalos = nhalos;
     m->nsamples = nsamples;
     m->runs_host = runs;
-    m->dm.far = far_stats(recs.data(), nhalos, runs);  // kept when samples change: only speed depends on it
     for (int i = 0; i < nhalos; ++i) m->types.push_back(lenses[0].type[i]);
     m->rec_bytes = (size_t)nsamples * nhalos * sizeof(HaloRec);
     m->rec32_bytes = (size_t)nsamples * nhalos * sizeof(HaloRec32);
@@ -742,6 +799,7 @@ int lt_model_create_batch(lt_model* out, const lt_potential_soa* lenses, int nsa
         free_model(m);
         return st;
     }
+    m->stats = m->staged_stats;
     e = hipMemcpy(m->base, m->staging, off_runs + runs.size() * sizeof(Run), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         free_model(m);
@@ -826,8 +884,19 @@ static GridDesc grid_desc(const lt_model_s* m, const lt_grid_desc* grid)
 double lt::map_rows_cost(lt_model m, int kind, int precision, const lt_grid_desc* whole, bool* tiled)
 {
     double cost = 0;
-    *tiled = far_shape(m->dm.far, kind, precision, grid_desc(m, whole), &cost) != FarShape::Direct;
+    const auto stats = std::atomic_load(&m->stats);
+    *tiled = far_shape(stats->far, stats->density[0], kind, precision, grid_desc(m, whole), &cost) != FarShape::Direct;
     return cost;
+}
+
+static int check_use(const lt_model_s* m, int kind)
+{
+    Use need = kind == LT_MAP_DPL || kind == LT_MAP_GRADIENT ? Use::Gradient
+               : kind == LT_MAP_POT ? Use::Potential
+               : kind == LT_MAP_MASS ? Use::Kmap : Use::Hessian;
+    if (need != m->use && !(need == Use::Hessian && m->use == Use::Kmap))
+        return fail(LT_ERR_INVALID, "model was created for another kind of map");
+    return LT_OK;
 }
 
 int lt::map_device_rows(lt_model m, int kind, int mode, double* const outs[5], double r, double mult,
@@ -837,17 +906,13 @@ int lt::map_device_rows(lt_model m, int kind, int mode, double* const outs[5], d
     if (!grid) return fail(LT_ERR_INVALID, "grid is NULL");
     int st = check_kind_mode(kind, mode);
     if (st) return st;
-    Use need = kind == LT_MAP_DPL || kind == LT_MAP_GRADIENT ? Use::Gradient
-               : kind == LT_MAP_POT ? Use::Potential
-               : kind == LT_MAP_MASS ? Use::Kmap : Use::Hessian;
-    if (need != m->use && !(need == Use::Hessian && m->use == Use::Kmap))
-        return fail(LT_ERR_INVALID, "model was created for another kind of map");
+    if ((st = check_use(m, kind))) return st;
     if (grid->nx <= 0 || grid->ny <= 0 || grid->pitch < grid->nx) return fail(LT_ERR_INVALID, "bad grid");
     if ((kind == LT_MAP_GRADIENT || kind == LT_MAP_DPL) && (!outs[0] || !outs[1]))
         return fail(LT_ERR_INVALID, "gradient output needs two planes");
     if (kind != LT_MAP_HESSIAN && kind != LT_MAP_FIELDS && !outs[0]) return fail(LT_ERR_INVALID, "out0 is NULL");
     HIP_TRY(hipSetDevice(m->device));
-    return launch_map(m->dm, kind, mode, outs, r, mult, grid_desc(m, grid), grid_desc(m, whole), precision, px,
+    return launch_map(m->dm, *std::atomic_load(&m->stats), kind, mode, outs, r, mult, grid_desc(m, grid), grid_desc(m, whole), precision, px,
                       (hipStream_t)stream, m->nhalos);
 }
 
@@ -858,6 +923,29 @@ int lt_map_device(lt_model m, int kind, int mode, double* out0, double* out1, do
 {
     double* outs[5] = {out0, out1, out2, out3, out4};
     return map_device_rows(m, kind, mode, outs, r, mult, grid, grid, precision, px, stream);
+}
+
+int lt_map_form(lt_model m, int sample, int kind, const lt_grid_desc* grid, int precision, int px, int* form)
+{
+    if (!m) return fail(LT_ERR_NOT_FOUND, "model is NULL");
+    if (!grid || !form) return fail(LT_ERR_INVALID, "NULL argument");
+    if (sample < 0 || sample >= m->nsamples) return fail(LT_ERR_INVALID, "sample out of range");
+    if (kind < LT_MAP_AMPLI || kind > LT_MAP_GRADIENT) return fail(LT_ERR_INVALID, "unknown map kind " + std::to_string(kind));
+    int st;
+    if ((st = check_use(m, kind)) || (st = check_launch(kind, precision, px))) return st;
+    if (grid->nx <= 0 || grid->ny <= 0 || grid->pitch < grid->nx) return fail(LT_ERR_INVALID, "bad grid");
+    const auto stats = std::atomic_load(&m->stats);
+    const Form f = map_form(stats->far, stats->density[sample], kind, precision, grid_desc(m, grid), px);
+    switch (f.shape) {
+    case FarShape::Root64: *form = LT_FORM_TILES_64; break;
+    case FarShape::Root64Wide: *form = LT_FORM_TILES_64_WIDE; break;
+    case FarShape::Root64Half: *form = LT_FORM_TILES_64_HALVES; break;
+    case FarShape::Root64Quarter: *form = LT_FORM_TILES_64_QUARTERS; break;
+    case FarShape::Root128: *form = LT_FORM_TILES_128; break;
+    case FarShape::Root256: *form = LT_FORM_TILES_256; break;
+    default: *form = px == LT_PX_HALO_LANES ? LT_FORM_HALO_LANES : f.split ? LT_FORM_PARTS : LT_FORM_PIXELS; break;
+    }
+    return LT_OK;
 }
 
 int lt_scale_device(double* x, double s, long long n, void* stream)

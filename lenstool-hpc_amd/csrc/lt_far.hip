@@ -572,12 +572,17 @@ __global__ __launch_bounds__(WAVE* far_waves(LV) / PARTS, LV == 3 && PARTS < 4 ?
 // ------------------------------------------------------------------------------------------------
 // the rule
 // ------------------------------------------------------------------------------------------------
-FarStats far_stats(const HaloRec* recs, int nhalos, const std::vector<Run>& runs)
+FarStats far_stats(int nhalos, const std::vector<Run>& runs)
 {
     FarStats st;
     st.nhalos = nhalos;
     st.nruns = (int)runs.size();
     st.cost = model_cost(runs);
+    return st;
+}
+
+double halo_density(const HaloRec* recs, const std::vector<Run>& runs)
+{
     double x0 = INFINITY, x1 = -INFINITY, y0 = INFINITY, y1 = -INFINITY, sum = 0;
     int n = 0;
     for (const Run& r : runs) {
@@ -593,11 +598,9 @@ FarStats far_stats(const HaloRec* recs, int nhalos, const std::vector<Run>& runs
             ++n;
         }
     }
-    if (n) {
-        st.area = (x1 - x0) * (y1 - y0);
-        st.near_area = sum / n;
-    }
-    return st;
+    if (!n) return 0.;
+    const double area = (x1 - x0) * (y1 - y0);
+    return area > 0. ? std::exp2(0.25 * std::rint(4. * std::log2(sum / n / area))) : INFINITY;
 }
 
 void far_records(const HaloRec* recs, int nhalos, FarRec* out)
@@ -636,7 +639,7 @@ static unsigned tiles_over(int start, int n, int side);
 // so that a part of a map takes the same form as the whole; roots of 256 again have to halve the count of 128: their
 // work-groups are few and uneven (a 300 x 200 part of the 4096^2 map: 271 us, 111 with 128, 183 directly).
 // Elsewhere the quickest shape is taken, or the direct sum.
-FarShape far_shape(const FarStats& st, int kind, int precision, const GridDesc& g, double* cost)
+FarShape far_shape(const FarStats& st, double density, int kind, int precision, const GridDesc& g, double* cost)
 {
     const int fam = family_of(kind);
     const double d = st.cost.px[fam], direct = direct_cost(st.cost, kind, precision);
@@ -651,7 +654,7 @@ FarShape far_shape(const FarStats& st, int kind, int precision, const GridDesc& 
     // share of the halos near a square of n pixels a side
     auto near = [&](double n) {
         const double h = 0.5 * n * std::fmax(dx, dy);
-        return st.area > 0. ? std::fmin(1., st.near_area * h * h / st.area) : st.near_area > 0. ? 1. : 0.;
+        return std::fmin(1., density * h * h);
     };
     auto per_px = [&](int side) {
         double nodes = 0., above = 1.;  // the halos not yet expanded

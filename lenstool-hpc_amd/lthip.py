@@ -22,6 +22,9 @@ PREC_FP64 = 0
 PREC_FP32C = 1
 PX_HALO_LANES = 16
 MAP_AMPLI, MAP_SHEAR, MAP_MASS, MAP_POT, MAP_DPL, MAP_FIELDS, MAP_HESSIAN, MAP_GRADIENT = range(1, 9)
+# LT_FORM_*: how lt_map_device sums a map
+FORMS = ("pixels", "parts", "tiles_64", "tiles_64_wide", "tiles_64_halves", "tiles_64_quarters", "tiles_128", "tiles_256",
+         "halo_lanes")
 
 _lib = None
 
@@ -121,6 +124,7 @@ SIGNATURES = {
     "lt_server_get_stats": ([C.c_void_p, C.POINTER(LtServerStats)], C.c_int),
     "lt_server_reset_stats": ([C.c_void_p], C.c_int),
     "lt_server_destroy": ([C.c_void_p], C.c_int),
+    "lt_map_form": ([C.c_void_p, C.c_int, C.c_int, C.POINTER(LtGridDesc), C.c_int, C.c_int, C.POINTER(C.c_int)], C.c_int),
     "lt_autotune": ([C.c_void_p, C.c_int, C.c_int, C.POINTER(LtGridDesc), C.c_int, C.c_void_p,
                      C.POINTER(C.c_int), C.POINTER(C.c_float)], C.c_int),
     "lt_par_load": ([C.POINTER(C.c_void_p), C.c_char_p], C.c_int),
@@ -727,6 +731,13 @@ class Model:
         ptrs = [C.c_void_p(p) if p else None for p in (list(outs) + [0] * 5)[:5]]
         check(lib().lt_map_device(self.h, kind, mode, *ptrs, r, mult, C.byref(g), precision, px,
                                   C.c_void_p(stream)))
+
+    def form(self, kind, grid: M.Grid, precision=PREC_FP64, px=0, sample=0, istart=0, jstart=0) -> str:
+        """The form in which map() sums a sample's map (FORMS)."""
+        g = LtGridDesc(grid.frame.xmin, grid.frame.ymin, grid.dx, grid.dy, grid.nx, grid.ny, istart, jstart, grid.nx)
+        form = C.c_int()
+        check(lib().lt_map_form(self.h, sample, kind, C.byref(g), precision, px, C.byref(form)))
+        return FORMS[form.value]
 
     def autotune(self, kind, mode, grid: M.Grid, precision=PREC_FP64, stream=0):
         """Pick the fastest pixels-per-thread for this map shape; returns (best_px, ms for px 1, 2, 4)."""

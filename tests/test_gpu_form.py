@@ -1,0 +1,139 @@
+"""The form of a halo sum (lt_map_form) follows the sample: two lenses of one model, spread over the map or crowded at
+its middle, take different forms, and each gives the same map bit for bit alone, in a batch at any place, after
+updates in either order, and as a model of its own; a captured sequence keeps the form of its capture."""
+import numpy as np
+import pytest
+
+import ltmodel as M
+from parity import print_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    import lthip
+    lthip.check(lthip.lib().lt_init(0))
+    return lthip
+
+
+def _mixed(n):
+    rng = np.random.default_rng(5)
+    halos = [dict(type=81, x=0.0, y=0.0, sigma=950.0, e=0.3, theta=0.4, rcore=9.0, rcut=900.0)]
+    for k in range(n - 1):
+        f = 10.0 ** (0.4 * (18 - rng.uniform(18, 24)))
+        halos.append(dict(type=(5, 8, 81)[k % 3], x=float(rng.uniform(-110, 110)), y=float(rng.uniform(-110, 110)),
+                          sigma=180.0 * f ** 0.25, e=float(rng.uniform(0.02, 0.6)), theta=float(rng.uniform(0, 3.1)),
+                          rcore=0.15 * f ** 0.5, rcut=40.0 * f ** 0.5))
+    return M.LensModel.from_halos(halos)
+
+
+def _pair():
+    """(spread, crowded): the same halos over 220 and over 18 arcseconds."""
+    spread = _mixed(160)
+    crowded = spread.subset(np.arange(spread.n))
+    crowded.x *= 0.08
+    crowded.y *= 0.08
+    crowded.refresh()
+    return spread, crowded
+
+
+GRID = M.Grid(M.grid_param(-110, 110, -110, 110), 673, 577)
+# (kind, use, planes, precisions, the crowded lens's form): FP32C mass and potential maps of this size stay direct for both
+KINDS = [("MAP_FIELDS", "MAP_HESSIAN", 5, (0, 1), "pixels"), ("MAP_DPL", "MAP_DPL", 2, (0, 1), "parts"),
+         ("MAP_MASS", "MAP_MASS", 1, (0,), "pixels"), ("MAP_POT", "MAP_POT", 1, (0,), "parts")]
+
+
+def _maps(hip, model, kind, planes, nsamples, precision):
+    outs = [hip.DeviceArray(nsamples * GRID.npix) for _ in range(planes)]
+    model.map(kind, 1, [o.ptr for o in outs], GRID, r=0.7, precision=precision)
+    hip.sync()
+    got = [o.download().reshape(nsamples, GRID.npix) for o in outs]
+    for o in outs:
+        o.close()
+    return got
+
+
+@pytest.mark.parametrize("name,use,planes,precisions,direct", KINDS)
+def test_form_follows_the_sample(hip, name, use, planes, precisions, direct):
+    kind, use = getattr(hip, name), getattr(hip, use)
+    lenses, forms = _pair(), ("tiles_64_halves", direct)
+    for precision in precisions:
+        print_case(f"{name} spread and crowded, precision={precision}", lenses[0], GRID)
+        alone = []
+        for lens, form in zip(lenses, forms):
+            m = hip.Model(lens, use)
+            assert m.form(kind, GRID, precision) == form
+            alone.append(_maps(hip, m, kind, planes, 1, precision))
+            m.close()
+        for first in (0, 1):  # a batch whose first sample takes one form or the other, then updated to the other order
+            order = [first, 1 - first, 1 - first, first]
+            m = hip.Model([lenses[k] for k in order], use)
+            for turn in range(2):
+                assert [m.form(kind, GRID, precision, sample=s) for s in range(4)] == [forms[k] for k in order]
+                got = _maps(hip, m, kind, planes, 4, precision)
+                for p in range(planes):
+                    for s, k in enumerate(order):
+                        np.testing.assert_array_equal(got[p][s], alone[k][p][0])
+                order = order[1:] + order[:1]
+                m.update_batch([lenses[k] for k in order])
+            m.close()
+        m = hip.Model(lenses[0], use)
+        for k in (1, 0, 1):
+            m.update(lenses[k])
+            for got, want in zip(_maps(hip, m, kind, planes, 1, precision), alone[k]):
+                np.testing.assert_array_equal(got, want)
+        m.close()
+
+
+def test_stage_alone_changes_nothing(hip):
+    """lt_model_stage is host work: until the upload, maps and their form are those of the samples on the device."""
+    spread, crowded = _pair()
+    print_case("stage without upload", spread, GRID)
+    m = hip.Model(spread, hip.MAP_HESSIAN)
+    want = _maps(hip, m, hip.MAP_FIELDS, 5, 1, 0)
+    m.stage(crowded)
+    assert m.form(hip.MAP_FIELDS, GRID) == "tiles_64_halves"
+    for a, b in zip(_maps(hip, m, hip.MAP_FIELDS, 5, 1, 0), want):
+        np.testing.assert_array_equal(a, b)
+    m.upload()
+    assert m.form(hip.MAP_FIELDS, GRID) == "pixels"
+    m.close()
+
+
+def test_capture_keeps_its_form(hip):
+    """Replays of a sequence captured with one lens, staged with the other and back: the captured lens bit for bit,
+    the other within rounding (1e-12 of the Hessian's scale at each pixel)."""
+    lenses = _pair()
+    print_case("captured upload and Hessian", lenses[0], GRID)
+    alone = []
+    for lens in lenses:
+        m = hip.Model(lens, hip.MAP_HESSIAN)
+        alone.append([p[0] for p in _maps(hip, m, hip.MAP_HESSIAN, 4, 1, 0)])
+        m.close()
+    s = hip.stream_create()
+    try:
+        m = hip.Model(lenses[0], hip.MAP_HESSIAN)
+        outs = [hip.DeviceArray(GRID.npix) for _ in range(4)]
+        g = hip.Graph(s)
+        m.upload(s)
+        m.map(hip.MAP_HESSIAN, 0, [o.ptr for o in outs], GRID, stream=s)
+        g.end()
+        for k in (0, 1, 0, 1):
+            m.stage(lenses[k])
+            g.launch()
+            hip.sync(s)
+            scale = sum(np.abs(p) for p in alone[k]) + 1.0
+            for o, want in zip(outs, alone[k]):
+                got = o.download()
+                if k == 0:
+                    np.testing.assert_array_equal(got, want)
+                else:
+                    assert (np.abs(got - want) <= 1e-12 * scale).all()
+            other = hip.Model(lenses[1 - k], hip.MAP_HESSIAN)  # eager work between the replays
+            _maps(hip, other, hip.MAP_HESSIAN, 4, 1, 0)
+            other.close()
+        g.close()
+        m.close()
+    finally:
+        hip.stream_destroy(s)
