@@ -118,7 +118,7 @@ __device__ __forceinline__ void add_halo(const HaloRec& h, double tx, const doub
             else if constexpr (CIRC) grad_sis_circ_at(h, tx, ty[k], acc[0][k], acc[1][k]);
             else grad_sis_at(h, tx, ty[k], acc[0][k], acc[1][k]);
         } else {
-            acc[0][k] += pot_halo_at<FULL>(h, TYPE, tx, ty[k], mn[k]);
+            add_pot_halo<FULL>(h, TYPE, tx, ty[k], acc[0][k], mn[k]);
         }
     }
 }

@@ -205,11 +205,10 @@ __device__ __forceinline__ void hess_sis32(const HaloRec32& h, const Frame32& f,
 __device__ __forceinline__ void hess_sis32_circ(const HaloRec32& h, float tx, float ty, float ty2, float& fT, float& fD,
                                                 float& fB)
 {
-    const float x2 = tx * tx;
-    const float iR = rsq32(x2 + ty2);
+    const float iR = rsq32(__builtin_fmaf(tx, tx, ty2));
     const float ga = h.hT * (iR * iR * iR);
     fT = __builtin_fmaf(h.hT, iR, fT);
-    fD = __builtin_fmaf(ga, ty2 - x2, fD);
+    fD = __builtin_fmaf(ga, __builtin_fmaf(-tx, tx, ty2), fD);
     fB = __builtin_fmaf(-ga, tx * ty, fB);
 }
 
@@ -518,11 +517,10 @@ __device__ __forceinline__ void add_term32(const HaloRec32& h, const Seg32& s, f
                                            float& aD, float& aB)
 {
     if constexpr (TYPE == TYPE_SIS_CIRC) {
-        const float x2 = X * X;
-        const float iR = far ? rsq32(x2 + s.ty2) : 0.f;
+        const float iR = far ? rsq32(__builtin_fmaf(X, X, s.ty2)) : 0.f;
         const float ga = h.hT * (iR * iR * iR);
         aT = __builtin_fmaf(h.hT, iR, aT);
-        aD = __builtin_fmaf(ga, s.ty2 - x2, aD);
+        aD = __builtin_fmaf(ga, __builtin_fmaf(-X, X, s.ty2), aD);
         aB = __builtin_fmaf(-ga, X * Y, aB);
     } else if constexpr (TYPE == TYPE_SIS) {
         const float x2 = X * X, y2 = Y * Y;
@@ -783,14 +781,14 @@ struct QS32 {
     float R, Q2, S;
 };
 
-__device__ __forceinline__ QS32 qs32(const GradRec32& h, float rem2, float I2, float vy, float r, float r2, float rc)
+__device__ __forceinline__ QS32 qs32(const GradRec32& h, float rem2, float I2, float y, float r, float r2, float rc)
 {
     const float q = r2 + rem2;
     const float w = q * rsq32(q);
     QS32 o;
     o.R = __builtin_fmaf(h.cx1, w, r);
     o.Q2 = __builtin_fmaf(o.R, o.R, I2);
-    o.S = w + (rc + vy);
+    o.S = w + __builtin_fmaf(h.kv, y, rc);
     return o;
 }
 
@@ -801,11 +799,10 @@ __device__ __forceinline__ void grad_piemd32(const GradRec32& h, float tx, float
     const float rem2 = __builtin_fmaf(f.x2, h.kx, f.y2 * h.ky);
     const float I = h.ki * f.x;
     const float I2 = I * I;
-    const float vy = h.kv * f.y;
-    const QS32 a = qs32(h, rem2, I2, vy, h.ra, h.ra2, h.rca);
+    const QS32 a = qs32(h, rem2, I2, f.y, h.ra, h.ra2, h.rca);
     float arg, ratio;
     if (CUT) {
-        const QS32 b = qs32(h, rem2, I2, vy, h.rb, h.rb2, h.rcb);
+        const QS32 b = qs32(h, rem2, I2, f.y, h.rb, h.rb2, h.rcb);
         arg = atan2f_lt(I * (b.R - a.R), __builtin_fmaf(a.R, b.R, I2));
         ratio = (a.Q2 * (b.S * b.S)) * rcp32(b.Q2 * (a.S * a.S));
     } else {

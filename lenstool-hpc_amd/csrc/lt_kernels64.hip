@@ -262,7 +262,7 @@ __device__ __forceinline__ void potential_sums(const HaloRec* __restrict__ halos
         for (int i = first_halo<SPLIT>(run.start, wave); i < run.start + run.count; i += SPLIT) {
             const HaloRec& h = halos[i];
 #pragma unroll
-            for (int k = 0; k < PX; ++k) s[k] += pot_halo(h, run.type, px[k], py, mn[k]);
+            for (int k = 0; k < PX; ++k) add_pot_halo<false>(h, run.type, px[k] - h.xh, py - h.yh, s[k], mn[k]);
         }
         if (SPLIT > 1) continue;
 #pragma unroll

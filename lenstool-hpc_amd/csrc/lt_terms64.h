@@ -15,6 +15,10 @@
 #include "lt_kernels.h"
 #include "lt_math.h"
 
+// Contraction is off from here to the end of every file that includes this: only the written FMAs are fused, so that
+// each instantiation (pixels per thread, parts, tiles) evaluates the same operations on the same inputs.
+#pragma clang fp contract(off)
+
 namespace lt {
 
 // ------------------------------------------------------------------------------------------------
@@ -178,11 +182,11 @@ template <bool FULL>
 __device__ __forceinline__ void hess_sis_circ_at(const HaloRec& h, double tx, double ty, double& aT, double& aD,
                                                  double& aB)
 {
-    const double x2 = tx * tx, y2 = ty * ty;
-    const double iR = rsq_c<FULL>(x2 + y2);
+    const double y2 = ty * ty;
+    const double iR = rsq_c<FULL>(__builtin_fma(tx, tx, y2));
     const double ga = h.amph * (iR * iR * iR);
     aT = __builtin_fma(h.amph, iR, aT);
-    aD = __builtin_fma(ga, y2 - x2, aD);
+    aD = __builtin_fma(ga, __builtin_fma(-tx, tx, y2), aD);
     aB = __builtin_fma(-ga, tx * ty, aB);
 }
 
@@ -210,7 +214,7 @@ struct QS64 {
 };
 
 template <bool FULL>
-__device__ __forceinline__ QS64 qs64(const HaloRec& h, double rem2, double I2, double vy, double r, double r2,
+__device__ __forceinline__ QS64 qs64(const HaloRec& h, double rem2, double I2, double y, double r, double r2,
                                      double rcx)
 {
     const double q = r2 + rem2;
@@ -218,7 +222,7 @@ __device__ __forceinline__ QS64 qs64(const HaloRec& h, double rem2, double I2, d
     QS64 o;
     o.R = __builtin_fma(h.cx1, w, r);
     o.Q2 = __builtin_fma(o.R, o.R, I2);
-    o.S = (w + rcx) + vy;
+    o.S = __builtin_fma(h.gkv, y, w + rcx);
     return o;
 }
 
@@ -233,11 +237,10 @@ __device__ __forceinline__ void grad_piemd_at(const HaloRec& h, double tx, doubl
     const double rem2 = __builtin_fma(f.x2, h.kx, f.y2 * h.ky);
     const double I = h.gki * f.x;
     const double I2 = I * I;
-    const double vy = h.gkv * f.y;
-    const QS64 a = qs64<FULL>(h, rem2, I2, vy, h.rc, h.ra2, h.rca);
+    const QS64 a = qs64<FULL>(h, rem2, I2, f.y, h.rc, h.ra2, h.rca);
     double arg, ratio;
     if (CUT) {
-        const QS64 b = qs64<FULL>(h, rem2, I2, vy, h.rcut, h.rb2, h.rcb);
+        const QS64 b = qs64<FULL>(h, rem2, I2, f.y, h.rcut, h.rb2, h.rcb);
         arg = atan2p_lt(I * (b.R - a.R), __builtin_fma(a.R, b.R, I2));
         ratio = (a.Q2 * (b.S * b.S)) * rcp_c<FULL>(b.Q2 * (a.S * a.S));
     } else {
@@ -368,19 +371,15 @@ __device__ __forceinline__ double pot_piemd(const HaloRec& h, const PixelFrame& 
     return __builtin_fma(f.x, arg, __builtin_fma(f.y, ay, -L));
 }
 
-// One halo's potential at (px, py) (SIS: b0 R, R^2 = (1-e) x^2 + (1+e) y^2).
+// One halo's potential at an offset from its centre added to acc (SIS: b0 R, R^2 = (1-e) x^2 + (1+e) y^2).
 template <bool FULL>
-__device__ __forceinline__ double pot_halo_at(const HaloRec& h, int type, double tx, double ty, double& mn)
+__device__ __forceinline__ void add_pot_halo(const HaloRec& h, int type, double tx, double ty, double& acc, double& mn)
 {
     const PixelFrame f = halo_frame_at(h, tx, ty);
-    if (type == TYPE_SIS) return h.ampg * sqrt(__builtin_fma(h.sa, f.x2, h.sb * f.y2));
-    const double v = (type == TYPE_PIEMD) ? pot_piemd<false, FULL>(h, f, mn) : pot_piemd<true, FULL>(h, f, mn);
-    return h.ampg * v;
-}
-
-__device__ __forceinline__ double pot_halo(const HaloRec& h, int type, double px, double py, double& mn)
-{
-    return pot_halo_at<false>(h, type, px - h.xh, py - h.yh, mn);
+    const double v = type == TYPE_SIS     ? sqrt(__builtin_fma(h.sa, f.x2, h.sb * f.y2))
+                     : type == TYPE_PIEMD ? pot_piemd<false, FULL>(h, f, mn)
+                                          : pot_piemd<true, FULL>(h, f, mn);
+    acc = __builtin_fma(h.ampg, v, acc);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -391,7 +390,7 @@ __device__ __forceinline__ double pot_halo(const HaloRec& h, int type, double px
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ void eigen(double A, double B, double C, double& lam, double& mu)
 {
-    double e = sqrt((A - C) * (A - C) + 4. * B * B);
+    double e = sqrt(__builtin_fma(A - C, A - C, 4. * B * B));
     lam = .5 * (A + C + e);
     mu = .5 * (A + C - e);
 }
@@ -416,7 +415,7 @@ __device__ __forceinline__ void hess_epilogue(const OutDesc& o, int64_t idx, dou
         if (o.p3) o.p3[idx] = b;
     } else if constexpr (KIND == LT_MAP_FIELDS) {
         double kappa = 0.5 * T * r, g1 = 0.5 * D * r, g2 = B * r;
-        double omk = 1. - kappa;
+        double omk = __builtin_fma(-0.5 * T, r, 1.);
         double det = __builtin_fma(omk, omk, -__builtin_fma(g1, g1, g2 * g2));
         if (o.p0) o.p0[idx] = kappa;
         if (o.p1) o.p1[idx] = g1;
@@ -430,29 +429,29 @@ __device__ __forceinline__ void hess_epilogue(const OutDesc& o, int64_t idx, dou
         double v;
         if (o.mode <= 3) {
             // det A, the product of the eigenvalues of 1 - r H, without their square root
-            const double omk = 1. - 0.5 * T * r, g1 = 0.5 * D * r, g2 = B * r;
+            const double omk = __builtin_fma(-0.5 * T, r, 1.), g1 = 0.5 * D * r, g2 = B * r;
             const double det = __builtin_fma(omk, omk, -__builtin_fma(g1, g1, g2 * g2));
             if (o.mode == 1) v = 1. / det;
             else if (o.mode == 2) v = 1. / fabs(det);
             else v = magnitudes(fabs(det));
         } else if (o.mode == 4) {
             const double kappa = (a + c) * r / 2., ga1 = (a - c) * r / 2., ga2 = b * r;
-            const double gp = sqrt(ga1 * ga1 + ga2 * ga2) / (1 - kappa);
-            v = (1 - kappa) * (1 + gp * gp) / (1 - gp * gp);
+            const double gp = sqrt(__builtin_fma(ga1, ga1, ga2 * ga2)) / (1 - kappa);
+            v = (1 - kappa) * __builtin_fma(gp, gp, 1.) / __builtin_fma(-gp, gp, 1.);
         } else if (o.mode == 5) {
             v = (a + c) / 2.;                                                   // kappa, no dlsds
         } else {
             const double h1 = (a - c) / 2.;
-            v = sqrt(h1 * h1 + b * b);                                          // 6: gamma, no dlsds
+            v = sqrt(__builtin_fma(h1, h1, b * b));                             // 6: gamma, no dlsds
         }
         o.p0[idx] = v;
     } else if constexpr (KIND == LT_MAP_SHEAR) {
         double v;
         if (o.mode <= 2) {
             double lam, mu;
-            eigen(1. - a * r, -b * r, 1. - c * r, lam, mu);
+            eigen(__builtin_fma(-a, r, 1.), -b * r, __builtin_fma(-c, r, 1.), lam, mu);
             const double q = lam / mu;
-            v = o.mode == 1 ? (lam - mu) / 2. : fabs((q * q - 1.) / (q * q + 1.));
+            v = o.mode == 1 ? (lam - mu) / 2. : fabs(__builtin_fma(q, q, -1.) / __builtin_fma(q, q, 1.));
         } else {
             v = o.mode == 3 ? (a - c) * r / 2. : b * r;                         // gamma1, gamma2
         }
