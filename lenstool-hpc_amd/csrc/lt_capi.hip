@@ -169,20 +169,14 @@ Form map_form(const FarStats& far, double density, int kind, int precision, cons
 
 // Launch the kernel that produces map `kind` of samples [s0, s0 + n) of a device model in form f; o's planes are those of
 // sample s0. `whole`: the grid that g is rows of.
-hipError_t launch_form(const DevModel& m, const ModelCost& cost, const Form& f, int s0, int n, OutDesc o, int mode, GridDesc g,
+hipError_t launch_form(const DevModel& m, const ModelCost& cost, const Form& f, int s0, int n, const OutDesc& o, GridDesc g,
                        const GridDesc& whole, int precision, int px, int nhalos, hipStream_t s)
 {
     const int64_t at = (int64_t)s0 * g.halo_stride;
     const HaloRec* const recs = m.recs + at;
     const HaloRec32* const recs32 = m.recs32 + at;
     g.nsamples = n;
-    if (f.shape != FarShape::Direct) {
-        if (o.kind == LT_MAP_AMPLI && mode == 5) {  // kappa: the Hessian's trace alone
-            o.kind = LT_MAP_MASS;
-            o.mult = 1.0;
-        }
-        return launch_far(recs, m.frecs + at, m.runs, m.nruns, nhalos, g, o, f.shape, s);
-    }
+    if (f.shape != FarShape::Direct) return launch_far(recs, m.frecs + at, m.runs, m.nruns, nhalos, g, o, f.shape, s);
     if (f.split) {
         const double npix = (double)whole.nx * (double)whole.ny * n;
         px = npix <= split_pixels(cost, o.kind, precision) ? kPxSplit : kPxParts;
@@ -240,7 +234,7 @@ int launch_map(const DevModel& m, const LensStats& lens, int kind, int mode, dou
             if (density[s1] != density[s1 - 1]) next = map_form(lens.far, density[s1], kind, precision, whole, px);
             if (!(next == form)) break;
         }
-        const hipError_t e = launch_form(m, lens.far.cost, form, s0, s1 - s0, o, mode, g, whole, precision, px, nhalos, s);
+        const hipError_t e = launch_form(m, lens.far.cost, form, s0, s1 - s0, o, g, whole, precision, px, nhalos, s);
         if (e != hipSuccess) return hip_fail(e, "kernel launch");
         for (int k = 0; k < 5; ++k)
             if (*planes[k]) *planes[k] += (size_t)(s1 - s0) * g.plane_stride;

@@ -137,3 +137,19 @@ def test_capture_keeps_its_form(hip):
         m.close()
     finally:
         hip.stream_destroy(s)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_kappa_is_half_the_trace(hip, precision):
+    """Amplification mode 5 (kappa) is (a + c) / 2 of the Hessian map bit for bit, expanded or direct. (Not so where the
+    FP32C kernel runs: its amplification maps take pixels of large kappa again in FP64, its Hessian maps do not.)"""
+    for lens, form in zip(_pair()[:2 - precision], ("tiles_64_halves", "pixels")):
+        print_case(f"kappa {form} precision={precision}", lens, GRID)
+        m = hip.Model(lens, hip.MAP_HESSIAN)
+        assert m.form(hip.MAP_AMPLI, GRID, precision) == m.form(hip.MAP_HESSIAN, GRID, precision) == form
+        a, _, c, _ = _maps(hip, m, hip.MAP_HESSIAN, 4, 1, precision)
+        out = hip.DeviceArray(GRID.npix)
+        m.map(hip.MAP_AMPLI, 5, [out.ptr], GRID, r=0.7, precision=precision)
+        hip.sync()
+        np.testing.assert_array_equal(out.download(), 0.5 * (a[0] + c[0]))
+        m.close()
