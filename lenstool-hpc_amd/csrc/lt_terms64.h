@@ -395,11 +395,10 @@ __device__ __forceinline__ void eigen(double A, double B, double C, double& lam,
     mu = .5 * (A + C - e);
 }
 
-// -2.5 log10(x), x >= 0: log_lt for a normal finite x, the library's for zero, infinity, NaN and the
-// smallest numbers
+// -2.5 log10(x), x >= 0: the library's log10 for zero, infinity, NaN and the largest and smallest numbers
 __device__ __forceinline__ double magnitudes(double x)
 {
-    if (x >= 0x1p-1000 && x <= 0x1p1000) return -1.0857362047581295 * log_lt(x);  // -2.5 / ln 10
+    if (x >= 0x1p-1000 && x <= 0x1p1000) return magnitudes_lt(x);
     return -2.5 * log10(x);
 }
 
