@@ -646,7 +646,8 @@ FarShape far_shape(const FarStats& st, double density, int kind, int precision, 
     if (cost) *cost = direct;
     if (st.nhalos < 1 || st.nhalos > kFarMaxHalos || st.nruns > kFarMaxRuns) return FarShape::Direct;
     const double dx = std::fabs(g.dx), dy = std::fabs(g.dy);
-    if (!(dx > 0.) || !(dy > 0.) || !std::isfinite(dx) || !std::isfinite(dy)) return FarShape::Direct;
+    // (the far tests square lengths in FP32)
+    if (!(std::fmin(dx, dy) > 0.) || !(std::fmax(dx, dy) >= 1e-15) || !(std::fmax(dx, dy) <= 1e15)) return FarShape::Direct;
     // pixel coordinates must resolve the squares: |coordinate| <= 2^30 steps
     const double cx = std::fabs(g.xmin) + (std::fabs((double)g.istart) + g.nx) * dx;
     const double cy = std::fabs(g.ymin) + (std::fabs((double)g.jstart) + g.ny) * dy;

@@ -153,3 +153,30 @@ def test_kappa_is_half_the_trace(hip, precision):
         hip.sync()
         np.testing.assert_array_equal(out.download(), 0.5 * (a[0] + c[0]))
         m.close()
+
+
+@pytest.mark.parametrize("power", [70, -70])
+def test_units(hip, power):
+    """A lens and its grid in units of 2^-70 and 2^70 arcseconds: the same Hessian (whose halo terms scale exactly),
+    within the rounding between forms (1e-12 of its scale). Maps this far from 1 stay direct: the far tests of the
+    expansions square lengths in FP32."""
+    lens = _pair()[0]
+    print_case(f"units of 2^{-power} arcseconds", lens, GRID)
+    m = hip.Model(lens, hip.MAP_HESSIAN)
+    want = [p[0] for p in _maps(hip, m, hip.MAP_HESSIAN, 4, 1, 0)]
+    m.close()
+    unit = 2.0 ** power
+    scaled = lens.subset(np.arange(lens.n))
+    for f in ("x", "y", "b0", "rcore", "rcut"):
+        getattr(scaled, f)[:] *= unit
+    scaled.refresh()
+    grid = M.Grid(M.grid_param(-110 * unit, 110 * unit, -110 * unit, 110 * unit), GRID.nx, GRID.ny)
+    m = hip.Model(scaled, hip.MAP_HESSIAN)
+    outs = [hip.DeviceArray(grid.npix) for _ in range(4)]
+    m.map(hip.MAP_HESSIAN, 0, [o.ptr for o in outs], grid)
+    hip.sync()
+    assert m.form(hip.MAP_HESSIAN, grid) == "pixels"
+    m.close()
+    scale = sum(np.abs(p) for p in want) + 1.0
+    for o, w in zip(outs, want):
+        assert (np.abs(o.download() - w) <= 1e-12 * scale).all()
