@@ -594,7 +594,7 @@ double halo_density(const HaloRec* recs, const std::vector<Run>& runs)
             y0 = std::min(y0, h.yh);
             y1 = std::max(y1, h.yh);
             // ellipse X^2 + Y^2 < bound, X and Y the scaled frame
-            sum += M_PI * kFarBound2 * h.kx / std::fabs(h.csx * h.csy + h.snx * h.sny);
+            sum += M_PI * kFarBound2 * h.kx * (h.cs * h.cs + h.sn * h.sn) / std::fabs(h.csx * h.csy + h.snx * h.sny);
             ++n;
         }
     }
@@ -613,12 +613,14 @@ void far_records(const HaloRec* recs, int nhalos, FarRec* out)
         r.yh = h.yh;
         r.f = 3.0e38f;       // type 14, a constant: far from everything
         if (!(h.kx > 0.)) continue;
-        const double s = 1. / std::sqrt(h.kx);  // W^2 / a^2, in units of b^2 h^2 after W = cx1 w, cx1 b = a
+        // W^2 / a^2, in units of b^2 h^2 after W = cx1 w, cx1 b = a. (The halo frame is the caller's cos and sin: where
+        // they are not of norm 1 it is as much larger than the lab frame, and so is the square in it.)
+        const double n2 = h.cs * h.cs + h.sn * h.sn, s = 1. / std::sqrt(h.kx * n2);
         r.a = (float)(s * h.csx);
         r.b = (float)(s * h.snx);
         r.c = (float)(s * h.csy);
         r.d = (float)(s * h.sny);
-        r.f = (float)std::fmin(h.far0 / h.kx, 1.0e38);
+        r.f = (float)std::fmin(h.far0 / (h.kx * n2), 1.0e38);
     }
 }
 

@@ -180,3 +180,31 @@ def test_units(hip, power):
     scale = sum(np.abs(p) for p in want) + 1.0
     for o, w in zip(outs, want):
         assert (np.abs(o.download() - w) <= 1e-12 * scale).all()
+
+
+@pytest.mark.parametrize("norm", [2.5, 0.4])
+def test_angles_of_another_norm(hip, norm):
+    """cos and sin of the angles are the caller's: of norm 2.5 and 0.4 a halo's frame is larger or smaller than the lab's
+    by that factor. The expanded Hessian at 100 x 60 pixels equals the direct one of that part of the map (1e-12)."""
+    lens = _pair()[0]
+    lens.cos *= norm
+    lens.sin *= norm
+    lens._soa = None
+    print_case(f"angles of norm {norm}", lens, GRID)
+    m = hip.Model(lens, hip.MAP_HESSIAN)
+    assert m.form(hip.MAP_HESSIAN, GRID).startswith("tiles")
+    whole = [p[0].reshape(GRID.ny, GRID.nx) for p in _maps(hip, m, hip.MAP_HESSIAN, 4, 1, 0)]
+    part = M.Grid(GRID.frame, 100, 60, step=(GRID.dx, GRID.dy))
+    worst = 0.0
+    for i0, j0 in ((0, 0), (290, 260), (573, 517), (100, 400)):
+        assert m.form(hip.MAP_HESSIAN, part, istart=i0, jstart=j0) in ("pixels", "parts")
+        outs = [hip.DeviceArray(part.npix) for _ in range(4)]
+        m.map(hip.MAP_HESSIAN, 0, [o.ptr for o in outs], part, istart=i0, jstart=j0)
+        hip.sync()
+        got = [o.download().reshape(part.ny, part.nx) for o in outs]
+        scale = sum(np.abs(g) for g in got) + 1.0
+        for g, w in zip(got, whole):
+            worst = max(worst, float((np.abs(w[j0:j0 + 60, i0:i0 + 100] - g) / scale).max()))
+    m.close()
+    print(f"norm {norm}: {worst:.2e}", flush=True)
+    assert worst <= 1e-12
