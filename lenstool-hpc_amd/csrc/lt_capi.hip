@@ -314,8 +314,7 @@ int host_map(int kind, int mode, Use use, double* const host_out[5], const lt_gr
     const size_t run_bytes = runs.size() * sizeof(Run);
     const size_t far_bytes = recs.size() * sizeof(FarRec);
     const size_t off_runs = ((rec_bytes + rec32_bytes + far_bytes + 63) / 64) * 64, halo_need = off_runs + run_bytes;
-    if ((st = host_ensure(&S.halos, &S.halos_bytes, std::max<size_t>(halo_need, 1)))) return st;
-    if ((st = host_ensure(&S.planes, &S.planes_bytes, n * np * sizeof(double)))) return st;
+    if ((st = host_room(S, std::max<size_t>(halo_need, 1), n * np * sizeof(double)))) return st;
 
     // one image of the model, in the pinned area where it fits, and one copy of it
     std::vector<char> large(halo_need <= kHostPinned ? 0 : halo_need);
@@ -996,7 +995,7 @@ int lt_autotune(lt_model m, int kind, int mode, const lt_grid_desc* grid, int pr
     const int np = planes_for_kind(kind);
     const size_t plane = (size_t)grid->nx * grid->ny * m->nsamples;
     double* buf = nullptr;
-    if (hipMalloc(&buf, plane * np * sizeof(double)) != hipSuccess) {
+    if (device_alloc((void**)&buf, plane * np * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
         return fail(LT_ERR_NOMEM, "autotune scratch planes");
     }

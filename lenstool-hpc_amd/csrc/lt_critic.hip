@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "lenstool_hip/lt_capi.h"
+#include "lt_hostio.h"
 #include "lt_internal.h"
 
 namespace lt {
@@ -365,7 +366,7 @@ int lt_critic_device(const double* det, const double* kappa, const lt_grid_desc*
     int dev;
     if ((st = current_device(&dev))) return st;
     void* buf = nullptr;
-    LT_HIP_TRY(hipMalloc(&buf, critic_scratch_bytes(grid->ny - 1)));
+    LT_HIP_TRY(device_alloc(&buf, critic_scratch_bytes(grid->ny - 1)));
     st = critic_run(det, kappa, grid, segs, kinds, max_segments, nsegments, (hipStream_t)stream, buf);
     (void)hipFree(buf);
     return st;

@@ -35,22 +35,6 @@ int host_ready(HostState& h)
     return LT_OK;
 }
 
-int host_ensure(void** buf, size_t* have, size_t need)
-{
-    if (need <= *have) return LT_OK;
-    if (*buf) LT_HIP_TRY(hipFree(*buf));
-    *buf = nullptr;
-    *have = 0;
-    size_t n = need + need / 4;
-    if (hipMalloc(buf, n) != hipSuccess) {
-        *buf = nullptr;
-        (void)hipGetLastError();
-        return set_error(LT_ERR_NOMEM, "device allocation of " + std::to_string(n) + " bytes failed");
-    }
-    *have = n;
-    return LT_OK;
-}
-
 static void give_back(HostState& h)
 {
     if (h.stream) (void)hipStreamSynchronize(h.stream);
@@ -59,6 +43,36 @@ static void give_back(HostState& h)
         *p = nullptr;
     }
     h.halos_bytes = h.planes_bytes = h.scratch_bytes = 0;
+}
+
+// a kept buffer of at least `need` bytes; what it held is lost
+static hipError_t grow(void** buf, size_t* have, size_t need, size_t slack)
+{
+    if (need <= *have) return hipSuccess;
+    hipError_t e = *buf ? hipFree(*buf) : hipSuccess;
+    *buf = nullptr;
+    *have = 0;
+    if (e == hipSuccess) e = hipMalloc(buf, need + slack);
+    if (e == hipSuccess) *have = need + slack;
+    else *buf = nullptr;
+    return e;
+}
+
+static int no_memory(size_t bytes)
+{
+    (void)hipGetLastError();
+    return set_error(LT_ERR_NOMEM, "device allocation of " + std::to_string(bytes) + " bytes failed");
+}
+
+int host_room(HostState& h, size_t halos, size_t planes)
+{
+    for (int again = 0; again < 2; ++again) {
+        if (again) give_back(h);
+        if (grow(&h.halos, &h.halos_bytes, halos, again ? 0 : halos / 4) == hipSuccess &&
+            grow(&h.planes, &h.planes_bytes, planes, again ? 0 : planes / 4) == hipSuccess)
+            return LT_OK;
+    }
+    return no_memory(halos + planes);
 }
 
 hipError_t device_alloc(void** p, size_t bytes)
@@ -76,23 +90,18 @@ hipError_t device_alloc(void** p, size_t bytes)
 
 int HostScratch::take(HostState& h, size_t bytes)
 {
-    if (bytes <= kHostKept * 4 / 5) {
-        const int st = host_ensure(&h.scratch, &h.scratch_bytes, bytes);
-        p = (char*)h.scratch;
-        return st;
+    own = bytes > kHostKept * 4 / 5;
+    for (int again = 0; again < 2; ++again) {
+        if (again) give_back(h);
+        if (own ? hipMalloc((void**)&p, bytes) == hipSuccess
+                : grow(&h.scratch, &h.scratch_bytes, bytes, again ? 0 : bytes / 4) == hipSuccess) {
+            if (!own) p = (char*)h.scratch;
+            return LT_OK;
+        }
     }
-    hipError_t e = hipMalloc((void**)&p, bytes);
-    if (e != hipSuccess) {
-        give_back(h);
-        e = hipMalloc((void**)&p, bytes);
-    }
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        p = nullptr;
-        return set_error(LT_ERR_NOMEM, "device allocation of " + std::to_string(bytes) + " bytes failed");
-    }
-    own = true;
-    return LT_OK;
+    p = nullptr;
+    own = false;
+    return no_memory(bytes);
 }
 
 HostScratch::~HostScratch()

@@ -33,8 +33,8 @@ constexpr int kMaxDevices = 64;
 HostState& host_state(int dev);
 // the stream and the pinned area of the current device's state, made on the first call
 int host_ready(HostState& h);
-// grow-only device buffer
-int host_ensure(void** buf, size_t* have, size_t need);
+// the map calls' buffers, of at least these sizes; what they held is lost. Gives back everything kept rather than fail.
+int host_room(HostState& h, size_t halos, size_t planes);
 
 // hipMalloc that gives back the kept buffers of the device, if no call is using them, rather than fail.
 hipError_t device_alloc(void** p, size_t bytes);

@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "lenstool_hip/lt_capi.h"
+#include "lt_hostio.h"
 #include "lt_internal.h"
 #include "lt_server_policy.h"
 
@@ -385,7 +386,7 @@ int lt_server_create(lt_server* out, int nslots, long long hbm_budget_bytes)
         s->slots.push_back(sl);
     }
     void* arena = nullptr;
-    if (hipMalloc(&arena, (size_t)hbm_budget_bytes) != hipSuccess) {
+    if (device_alloc(&arena, (size_t)hbm_budget_bytes) != hipSuccess) {
         (void)hipGetLastError();
         drop_slots();
         return set_error(LT_ERR_NOMEM, "could not reserve the HBM budget (" + std::to_string(hbm_budget_bytes) +
