@@ -317,8 +317,8 @@ int host_map(int kind, int mode, Use use, double* const host_out[5], const lt_gr
     if ((st = host_room(S, std::max<size_t>(halo_need, 1), n * np * sizeof(double)))) return st;
 
     // one image of the model, in the pinned area where it fits, and one copy of it
-    std::vector<char> large(halo_need <= kHostPinned ? 0 : halo_need);
-    char* const image = large.empty() ? S.pinned : large.data();
+    std::vector<char> large;
+    char* const image = host_image(S, halo_need, large);
     DevModel m;
     if (rec_bytes) {
         std::memcpy(image, recs.data(), rec_bytes);

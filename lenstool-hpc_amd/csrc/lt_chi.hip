@@ -422,8 +422,7 @@ int lt_chi_barycentersource(double* chi, int* error, int nbgridcells, int nsets,
         if (!st) st = room.take(S, bytes);
         if (!st) {
             batch_layout(&b, room.p);
-            if (host_bytes > kHostPinned) large.resize(host_bytes);
-            b.staging = large.empty() ? S.pinned : large.data();
+            b.staging = host_image(S, host_bytes, large);
             stage_families(&b, b.staging, nimages, images);
             st = batch_run(&b, lens, chi, &found, &sst, S.stream);
             if (st) (void)hipStreamSynchronize(S.stream);  // the upload reads the staging area
@@ -496,7 +495,7 @@ int lt_point_gradients(double* gx, double* gy, const double* px, const double* p
     HostScratch room;
     if ((st = room.take(S, need))) return st;
     char* const p = room.p;
-    if (input <= kHostPinned) {
+    if (S.pinned && input <= kHostPinned) {
         // the model and the points in one copy from the pinned area
         if (!runs.empty()) std::memcpy(S.pinned + o_u, runs.data(), runs.size() * sizeof(Run));
         if (!recs.empty()) std::memcpy(S.pinned + o_r, recs.data(), recs.size() * sizeof(HaloRec));

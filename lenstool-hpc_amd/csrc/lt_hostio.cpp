@@ -30,9 +30,15 @@ int host_ready(HostState& h)
     if (!h.pinned && hipHostMalloc((void**)&h.pinned, kHostPinned, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         h.pinned = nullptr;
-        return set_error(LT_ERR_NOMEM, "pinned host allocation of " + std::to_string(kHostPinned) + " bytes failed");
     }
     return LT_OK;
+}
+
+char* host_image(HostState& h, size_t bytes, std::vector<char>& own)
+{
+    if (h.pinned && bytes <= kHostPinned) return h.pinned;
+    own.resize(bytes);
+    return own.data();
 }
 
 static void give_back(HostState& h)
@@ -147,6 +153,12 @@ int host_download(HostState& h, const HostCopy* copies, int n)
 {
     size_t total = 0;
     for (int i = 0; i < n; ++i) total += copies[i].bytes;
+    if (!h.pinned) {
+        for (int i = 0; i < n; ++i)
+            if (copies[i].bytes) LT_HIP_TRY(hipMemcpyAsync(copies[i].host, copies[i].dev, copies[i].bytes, hipMemcpyDeviceToHost, h.stream));
+        LT_HIP_TRY(hipStreamSynchronize(h.stream));
+        return LT_OK;
+    }
     if (total <= kHostPiece) {
         // through the start of the pinned area, neighbours on the device in one copy
         size_t at = 0;

@@ -6,6 +6,7 @@
 
 #include <cstddef>
 #include <mutex>
+#include <vector>
 
 namespace lt {
 
@@ -18,7 +19,7 @@ constexpr size_t kHostKept = 64 << 20;             // device bytes that a call's
 struct HostState {
     std::mutex mu;
     hipStream_t stream = nullptr;
-    char* pinned = nullptr;         // kHostPinned bytes
+    char* pinned = nullptr;         // kHostPinned bytes, or NULL where they cannot be had
     void* halos = nullptr;          // grow-only buffers of the map calls
     size_t halos_bytes = 0;
     void* planes = nullptr;
@@ -31,8 +32,11 @@ struct HostState {
 
 constexpr int kMaxDevices = 64;
 HostState& host_state(int dev);
-// the stream and the pinned area of the current device's state, made on the first call
+// the stream and the pinned area of the current device's state, made on the first call; without the area the calls
+// copy from and to pageable memory
 int host_ready(HostState& h);
+// where a call forms the image of its inputs: the pinned area, or `own` where that is too small or missing
+char* host_image(HostState& h, size_t bytes, std::vector<char>& own);
 // the map calls' buffers, of at least these sizes; what they held is lost. Gives back everything kept rather than fail.
 int host_room(HostState& h, size_t halos, size_t planes);
 

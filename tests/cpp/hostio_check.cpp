@@ -1,5 +1,5 @@
 // hostio_check.cpp -- the kept buffers and copies of the host-array calls (lt_hostio.cpp) under conditions that a GPU box does
-// not bring about at will, on the stand-in runtime of fake_hip: device memory that runs out.
+// not bring about at will, on the stand-in runtime of fake_hip: device memory that runs out, pinned memory that is refused.
 #include <cstdio>
 #include <string>
 #include <vector>
@@ -57,10 +57,43 @@ static void check_room()
     expect(host_room(h, mb, 30 * mb) == LT_OK, "and fits later");
 }
 
+// Planes on the device copied to host arrays as a map call does; true when they arrive whole.
+static bool download(HostState& h, const std::vector<size_t>& sizes)
+{
+    std::vector<std::vector<char>> from, to;
+    std::vector<HostCopy> copies;
+    for (size_t n : sizes) {
+        from.emplace_back(n);
+        for (size_t i = 0; i < n; ++i) from.back()[i] = (char)(i * 31 + i / 4097 + sizes.size());
+        to.emplace_back(n, (char)0x55);
+    }
+    for (size_t k = 0; k < sizes.size(); ++k) copies.push_back({to[k].data(), from[k].data(), sizes[k]});
+    return host_download(h, copies.data(), (int)copies.size()) == LT_OK && from == to && fake::pending() == 0;
+}
+
+// Without the pinned area the calls go on.
+static void check_pinned()
+{
+    HostState& h = host_state(0);
+    fake::state().no_pinned = true;
+    expect(host_ready(h) == LT_OK && !h.pinned, "no pinned area, and no error");
+    std::vector<char> own;
+    char* const image = host_image(h, 5000, own);
+    expect(image && own.size() == 5000 && image == own.data(), "the image is the call's own");
+    expect(download(h, {1000, 24, 3 * kHostPiece + 17}), "planes arrive without it");
+    fake::state().no_pinned = false;
+    expect(host_ready(h) == LT_OK && h.pinned, "it is asked for again by the next call");
+    std::vector<char> none;
+    expect(host_image(h, 5000, none) == h.pinned && none.empty(), "the image lies in it");
+    expect(host_image(h, kHostPinned + 1, none) == none.data() && none.size() == kHostPinned + 1, "unless it is too large");
+    expect(download(h, {1000, 24}) && download(h, {0, 3 * kHostPiece + 17, 9 * kHostPiece, 5}), "planes arrive through it");
+}
+
 int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "room") check_room();
+    else if (what == "pinned") check_pinned();
     else return 2;
     std::puts(failures ? "FAILED" : "OK");
     return failures != 0;
