@@ -12,7 +12,6 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -149,42 +148,58 @@ static void copy_share(HostState& h, int dev, int w, const std::vector<HostCopy>
     }
 }
 
+// The copies queued on h.stream, all of them or up to the first that fails.
+static hipError_t queue_small(HostState& h, const HostCopy* copies, int n)
+{
+    if (!h.pinned) {
+        for (int i = 0; i < n; ++i)
+            if (copies[i].bytes) {
+                const hipError_t e = hipMemcpyAsync(copies[i].host, copies[i].dev, copies[i].bytes, hipMemcpyDeviceToHost, h.stream);
+                if (e != hipSuccess) return e;
+            }
+        return hipSuccess;
+    }
+    // through the start of the pinned area, neighbours on the device in one copy
+    size_t at = 0;
+    for (int i = 0; i < n;) {
+        size_t bytes = copies[i].bytes;
+        int k = i + 1;
+        for (; k < n && (const char*)copies[k].dev == (const char*)copies[i].dev + bytes; ++k) bytes += copies[k].bytes;
+        if (bytes) {
+            const hipError_t e = hipMemcpyAsync(h.pinned + at, copies[i].dev, bytes, hipMemcpyDeviceToHost, h.stream);
+            if (e != hipSuccess) return e;
+        }
+        at += bytes;
+        i = k;
+    }
+    return hipSuccess;
+}
+
 int host_download(HostState& h, const HostCopy* copies, int n)
 {
     size_t total = 0;
     for (int i = 0; i < n; ++i) total += copies[i].bytes;
-    if (!h.pinned) {
-        for (int i = 0; i < n; ++i)
-            if (copies[i].bytes) LT_HIP_TRY(hipMemcpyAsync(copies[i].host, copies[i].dev, copies[i].bytes, hipMemcpyDeviceToHost, h.stream));
-        LT_HIP_TRY(hipStreamSynchronize(h.stream));
-        return LT_OK;
-    }
-    if (total <= kHostPiece) {
-        // through the start of the pinned area, neighbours on the device in one copy
+    if (!h.pinned || total <= kHostPiece) {
+        const hipError_t e = queue_small(h, copies, n);
+        // also after an error: the call's upload may still read the pinned area, the copies still write it
+        const hipError_t es = hipStreamSynchronize(h.stream);
+        if (e != hipSuccess || es != hipSuccess) return hip_error(e != hipSuccess ? e : es, "copy to the host");
+        if (!h.pinned) return LT_OK;
         size_t at = 0;
-        for (int i = 0; i < n;) {
-            size_t bytes = copies[i].bytes;
-            int k = i + 1;
-            for (; k < n && (const char*)copies[k].dev == (const char*)copies[i].dev + bytes; ++k) bytes += copies[k].bytes;
-            if (bytes) LT_HIP_TRY(hipMemcpyAsync(h.pinned + at, copies[i].dev, bytes, hipMemcpyDeviceToHost, h.stream));
-            at += bytes;
-            i = k;
-        }
-        LT_HIP_TRY(hipStreamSynchronize(h.stream));
-        at = 0;
         for (int i = 0; i < n; ++i) {
             if (copies[i].bytes) std::memcpy(copies[i].host, h.pinned + at, copies[i].bytes);
             at += copies[i].bytes;
         }
         return LT_OK;
     }
+    // (the upload too is done before the pinned area is written, and before anything below may throw)
+    LT_HIP_TRY(hipStreamSynchronize(h.stream));
     std::vector<HostCopy> pieces;
     for (int i = 0; i < n; ++i)
         for (size_t o = 0; o < copies[i].bytes; o += kHostPiece)
             pieces.push_back({(char*)copies[i].host + o, (const char*)copies[i].dev + o, std::min(kHostPiece, copies[i].bytes - o)});
     int dev = 0;
     LT_HIP_TRY(hipGetDevice(&dev));
-    LT_HIP_TRY(hipStreamSynchronize(h.stream));
     std::atomic<size_t> next{0};
     std::atomic<int> error{0};
     std::vector<std::thread> others;
@@ -192,7 +207,7 @@ int host_download(HostState& h, const HostCopy* copies, int n)
     try {
         for (int w = 1; w < std::min<int>(kHostThreads, (int)pieces.size()); ++w)
             others.emplace_back([&, w] { copy_share(h, dev, w, pieces, next, error); });
-    } catch (const std::system_error&) {  // no more threads: those there are take all
+    } catch (...) {  // no more threads, or no memory for one: those there are take all
     }
     copy_share(h, dev, 0, pieces, next, error);
     for (std::thread& t : others) t.join();

@@ -1,6 +1,9 @@
 // hostio_check.cpp -- the kept buffers and copies of the host-array calls (lt_hostio.cpp) under conditions that a GPU box does
-// not bring about at will, on the stand-in runtime of fake_hip: device memory that runs out, pinned memory that is refused.
+// not bring about at will, on the stand-in runtime of fake_hip: device memory that runs out, pinned memory that is refused, copies and
+// allocations that fail under way.
 #include <cstdio>
+#include <cstdlib>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -18,6 +21,18 @@ int hip_error(hipError_t, const char* where) { return set_error(LT_ERR_HIP, wher
 }  // namespace lt
 
 using namespace lt;
+
+// the allocation of this thread that fails, counted from now (< 0: none)
+static thread_local int g_fail_new = -1;
+
+void* operator new(size_t n)
+{
+    if (g_fail_new >= 0 && g_fail_new-- == 0) throw std::bad_alloc();
+    if (void* p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 static int failures = 0;
 static void expect(bool ok, const char* what)
@@ -89,11 +104,54 @@ static void check_pinned()
     expect(download(h, {1000, 24}) && download(h, {0, 3 * kHostPiece + 17, 9 * kHostPiece, 5}), "planes arrive through it");
 }
 
+// After a failure nothing is queued that would still read or write the pinned area or the caller's arrays.
+static void check_errors()
+{
+    HostState& h = host_state(0);
+    expect(host_ready(h) == LT_OK, "stream and pinned area");
+    std::vector<char> in(1000, 1), dev(1000), a(5 * kHostPiece + 3), b(100), out(a.size()), out2(b.size());
+    const HostCopy small[3] = {{out2.data(), b.data(), 40}, {out2.data() + 50, b.data() + 50, 40}, {out.data(), a.data(), 1000}};
+    const HostCopy large[2] = {{out.data(), a.data(), a.size()}, {out2.data(), b.data(), b.size()}};
+    bool quiet = true;
+    int failed = 0;
+    for (int pinned = 1; pinned >= 0; --pinned) {
+        char* const area = h.pinned;
+        if (!pinned) h.pinned = nullptr;
+        for (int k = 0; k < 8; ++k)
+            for (int which = 0; which < 2; ++which) {
+                quiet &= hipMemcpyAsync(dev.data(), in.data(), in.size(), hipMemcpyHostToDevice, h.stream) == hipSuccess;  // the call's upload
+                fake::state().copies_until_failure = k;
+                failed += host_download(h, which ? large : small, which ? 2 : 3) != LT_OK;
+                fake::state().copies_until_failure = -1;
+                quiet &= fake::pending() == 0;
+            }
+        h.pinned = area;
+    }
+    expect(failed == 3 + 7 + 3 + 2, "a failing copy is reported");
+    expect(quiet, "and nothing is left queued");
+    expect(download(h, {9 * kHostPiece, 5}), "the next copy is whole");
+    int thrown = 0, whole = 0;
+    for (int k = 0; k < 40; ++k) {  // out of host memory: at the list of pieces, or at a thread's start
+        g_fail_new = k;
+        bool ok = false;
+        try {
+            ok = host_download(h, large, 2) == LT_OK;
+        } catch (const std::bad_alloc&) {
+            ++thrown;
+        }
+        g_fail_new = -1;
+        whole += ok && out == a;
+        quiet &= fake::pending() == 0;
+    }
+    expect(thrown >= 1 && thrown + whole == 40 && quiet, "out of memory the threads that did start take all");
+}
+
 int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "room") check_room();
     else if (what == "pinned") check_pinned();
+    else if (what == "errors") check_errors();
     else return 2;
     std::puts(failures ? "FAILED" : "OK");
     return failures != 0;

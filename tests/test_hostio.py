@@ -1,5 +1,5 @@
 """The kept buffers and copies of the host-array calls (lenstool-hpc_amd/csrc/lt_hostio.cpp) where memory runs out or is
-refused, on the CPU with a stand-in for the HIP runtime (tests/cpp/fake_hip)."""
+refused and where copies fail, on the CPU with a stand-in for the HIP runtime (tests/cpp/fake_hip)."""
 import os
 import subprocess
 
@@ -19,7 +19,7 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["room", "pinned"])
+@pytest.mark.parametrize("what", ["room", "pinned", "errors"])
 def test_hostio(check, what):
     r = subprocess.run([check, what], capture_output=True, text=True, timeout=60)
     print(r.stdout, r.stderr)
