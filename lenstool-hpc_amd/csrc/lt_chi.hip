@@ -495,21 +495,27 @@ int lt_point_gradients(double* gx, double* gy, const double* px, const double* p
     HostScratch room;
     if ((st = room.take(S, need))) return st;
     char* const p = room.p;
+    hipError_t e = hipSuccess;
+    // every copy on the stream of the kernel that reads it
+    const auto up = [&](size_t to, const void* from, size_t n) {
+        if (e == hipSuccess && n) e = hipMemcpyAsync(p + to, from, n, hipMemcpyHostToDevice, S.stream);
+    };
     if (S.pinned && input <= kHostPinned) {
         // the model and the points in one copy from the pinned area
         if (!runs.empty()) std::memcpy(S.pinned + o_u, runs.data(), runs.size() * sizeof(Run));
         if (!recs.empty()) std::memcpy(S.pinned + o_r, recs.data(), recs.size() * sizeof(HaloRec));
         std::memcpy(S.pinned + o_x, px, bytes);
         std::memcpy(S.pinned + o_y, py, bytes);
-        LT_HIP_TRY(hipMemcpyAsync(p, S.pinned, input, hipMemcpyHostToDevice, S.stream));
+        up(0, S.pinned, input);
     } else {
-        if (!runs.empty()) LT_HIP_TRY(hipMemcpy(p + o_u, runs.data(), runs.size() * sizeof(Run), hipMemcpyHostToDevice));
-        if (!recs.empty()) LT_HIP_TRY(hipMemcpy(p + o_r, recs.data(), recs.size() * sizeof(HaloRec), hipMemcpyHostToDevice));
-        LT_HIP_TRY(hipMemcpy(p + o_x, px, bytes, hipMemcpyHostToDevice));
-        LT_HIP_TRY(hipMemcpy(p + o_y, py, bytes, hipMemcpyHostToDevice));
+        up(o_u, runs.data(), runs.size() * sizeof(Run));
+        up(o_r, recs.data(), recs.size() * sizeof(HaloRec));
+        up(o_x, px, bytes);
+        up(o_y, py, bytes);
     }
-    hipError_t e = launch_points_gradient64((HaloRec*)(p + o_r), (Run*)(p + o_u), (int)runs.size(), (double*)(p + o_x),
-                                            (double*)(p + o_y), npts, 1, 0, (double*)(p + o_gx), (double*)(p + o_gy), S.stream);
+    if (e == hipSuccess)
+        e = launch_points_gradient64((HaloRec*)(p + o_r), (Run*)(p + o_u), (int)runs.size(), (double*)(p + o_x),
+                                     (double*)(p + o_y), npts, 1, 0, (double*)(p + o_gx), (double*)(p + o_gy), S.stream);
     if (e != hipSuccess) {
         (void)hipStreamSynchronize(S.stream);
         return hip_error(e, "point gradients");
