@@ -157,7 +157,8 @@ int lt_map_factors(int kind, int mode, const lt_cosmo_param* cosmo, double z_len
  * LT_MAP_HESSIAN (out0..out3 = a, b, c, d), LT_MAP_GRADIENT (out0, out1 = x, y) and LT_MAP_FIELDS
  * (out0..out4 = kappa, gamma1, gamma2, det A, mu). r = D_ls/D_s used by the map formulas, mult = the
  * mass / potential multiplier of the mode. px = launch shape: 1, 2 or 4 pixels per thread (results
- * identical bit for bit), 0 = the tuned default, or LT_PX_HALO_LANES (FP32C Hessian-derived maps
+ * identical bit for bit), 0 = the tuned default; maps in another form than LT_FORM_PIXELS (lt_map_form)
+ * have no such shape, and px does not change them. Or px = LT_PX_HALO_LANES (FP32C Hessian-derived maps
  * only): lanes over halos, a wavefront per 16-pixel row segment; its FP32 terms are summed in
  * another order and its near-core test is another region, so its results differ from the other
  * shapes' within the FP32C error; it is never the tuned default (measured slower than px 2 on a
@@ -187,7 +188,8 @@ int lt_map_form(lt_model model, int sample, int kind, const lt_grid_desc* grid, 
 /* Time the map with 1, 2 and 4 pixels per thread (one warm-up and two timed launches each, into
  * scratch planes) and make the fastest the default (px = 0) for maps of this family, precision,
  * halo-count octave and pixel-count octave in this process. ms[3] (optional) gets the per-launch
- * times. Results do not depend on these shapes: only speed does. */
+ * times. Results do not depend on these shapes: only speed does. A map in another form than
+ * LT_FORM_PIXELS is timed once: ms holds that time three times, *best_px the default, which stays. */
 int lt_autotune(lt_model model, int kind, int mode, const lt_grid_desc* grid, int precision, void* stream,
                 int* best_px, float* ms);
 

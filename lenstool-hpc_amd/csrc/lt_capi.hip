@@ -1006,9 +1006,18 @@ int lt_autotune(lt_model m, int kind, int mode, const lt_grid_desc* grid, int pr
     // the shapes whose results are bit-identical to each other (the halo-lane shape sums the FP32 terms
     // in another order: it is used when asked for explicitly)
     const int cand[3] = {1, 2, 4};
-    const int ncand = 3;
+    // a map in another form than every halo at every pixel has no pixels per thread to choose: one timing, and the
+    // default stays
+    const auto stats = std::atomic_load(&m->stats);
+    const GridDesc gd = grid_desc(m, &g);
+    bool tuned = false;
+    for (double density : stats->density) {
+        const Form f = map_form(stats->far, density, kind, precision, gd, 0);
+        tuned |= f.shape == FarShape::Direct && !f.split;
+    }
+    const int ncand = tuned ? 3 : 1;
     float best = 1e30f;
-    int bpx = 2;
+    int bpx = tuned ? 2 : default_px(kind, precision, m->nhalos, (long long)grid->nx * grid->ny);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hipError_t he = hipEventCreate(&e0);
     if (he == hipSuccess) he = hipEventCreate(&e1);
@@ -1024,8 +1033,8 @@ int lt_autotune(lt_model m, int kind, int mode, const lt_grid_desc* grid, int pr
         if (st == LT_OK && he == hipSuccess) he = hipEventSynchronize(e1);
         float t = 0.f;
         if (st == LT_OK && he == hipSuccess) he = hipEventElapsedTime(&t, e0, e1);
-        if (ms) ms[i] = t / 2.f;
-        if (st == LT_OK && he == hipSuccess && t < best) {
+        for (int k = i; ms && k < (tuned ? i + 1 : 3); ++k) ms[k] = t / 2.f;
+        if (tuned && st == LT_OK && he == hipSuccess && t < best) {
             best = t;
             bpx = px;
         }
@@ -1035,7 +1044,7 @@ int lt_autotune(lt_model m, int kind, int mode, const lt_grid_desc* grid, int pr
     (void)hipFree(buf);
     if (st) return st;
     if (he != hipSuccess) return hip_fail(he, "autotune timing");
-    {
+    if (tuned) {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         g_tuned[tune_key(kind, precision, m->nhalos, (long long)grid->nx * grid->ny)] = bpx;
     }

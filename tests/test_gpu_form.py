@@ -208,3 +208,23 @@ def test_angles_of_another_norm(hip, norm):
     m.close()
     print(f"norm {norm}: {worst:.2e}", flush=True)
     assert worst <= 1e-12
+
+
+def test_autotune(hip):
+    """A map in tiles or in parts has no pixels per thread to tune: one time, given three times, and the default stays
+    what a direct map of the same octaves of halos and pixels had it tuned to."""
+    spread, crowded = _pair()
+    small = M.Grid(GRID.frame, 97, 83)
+    print_case("autotune", spread, GRID)
+    m = hip.Model(crowded, hip.MAP_HESSIAN)
+    assert m.form(hip.MAP_FIELDS, GRID) == "pixels"
+    px, ms = m.autotune(hip.MAP_FIELDS, 0, GRID)
+    assert px in (1, 2, 4) and len(set(ms)) > 1
+    m.close()
+    m = hip.Model(spread, hip.MAP_HESSIAN)
+    for grid, form in ((GRID, "tiles_64_halves"), (small, "parts")):
+        assert m.form(hip.MAP_FIELDS, grid) == form
+        best, ms = m.autotune(hip.MAP_FIELDS, 0, grid)
+        assert ms[0] == ms[1] == ms[2] > 0
+        assert best == (px if grid is GRID else 2)
+    m.close()
