@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 namespace lt {
 
@@ -257,20 +258,21 @@ __device__ __forceinline__ double log_lt(double x)
     return __builtin_fma(de, kLn2Hi, __builtin_fma(de, kLn2Lo, lm));
 }
 
-// -2.5 log10(x) for x in [2^-1000, 2^1000], within 0.6 units in the last place: the logarithm of log_lt with what its
+// -2.5 log10(x) for x in [2^-1000, 2^1000], within 0.6 units in the last place: the steps of log_lt with what their
 // roundings leave carried along. s = f / (m + 1) is taken as sv + sl (the residuals of the sum and of the quotient are
-// exact or one FMA), ln x as a leading sum t and its remainder tl, and the factor as two doubles, so that the last
-// addition alone rounds at the result's own size. 15 instructions more than log_lt, half of the library's log10.
+// exact or one FMA), -2.5 log10 x = C e + K s + K s (s^2 R(s^2)) with the leading products C e (exact) and K sv summed
+// apart from their remainders, so that the last addition alone rounds at the result's own size. Eight instructions more
+// than log_lt.
 __device__ __forceinline__ double magnitudes_lt(double x)
 {
-    constexpr double kLn2Hi = 0x1.62e42fee00000p-1, kLn2Lo = 0x1.a39ef35793c76p-33;
-    constexpr double kSqrtHalf = 0.70710678118654757274;
-    constexpr double kHi = -0x1.15f2ced384f29p+0, kLo = 0x1.02bea6b55233cp-55;  // -2.5 / ln 10
-    int e;
-    double m = __builtin_frexp(x, &e);
-    const bool lo = m < kSqrtHalf;
-    m = lo ? m + m : m;
-    e = lo ? e - 1 : e;
+#pragma clang fp contract(off)
+    constexpr double kHi = -0x1.15f2ced384f29p+1, kLo = 0x1.02bea6b55233cp-54;      // K = -5 / ln 10
+    constexpr double kExpHi = -0x1.8151824c75800p-1, kExpLo = -0x1.fabf59b5d80b8p-47;  // C = -2.5 log10 2
+    // x = m 2^e with m in [sqrt(1/2), sqrt 2): e is the exponent field of x / sqrt(1/2), formed on the upper word
+    constexpr uint32_t kSqrtHalfHi = 0x3fe6a09e, kOneHi = 0x3ff00000;
+    const uint32_t hx = (uint32_t)__double2hiint(x) + (kOneHi - kSqrtHalfHi);
+    const int e = (int)(hx >> 20) - 1023;
+    const double m = __hiloint2double((int)((hx & 0xfffff) + kSqrtHalfHi), __double2loint(x));
     const double f = m - 1., d = m + 1.;
     const double rc = rcp64(d);
     const double sv = f * rc;
@@ -279,13 +281,12 @@ __device__ __forceinline__ double magnitudes_lt(double x)
     double p = kLogR[6];
 #pragma unroll
     for (int k = 5; k >= 0; --k) p = horner_step(p, w, kLogR[k]);
-    const double s2 = sv + sv, de = (double)e;
-    const double a = de * kLn2Hi;  // exact
-    const double t0 = a + s2;      // |a| > |s2|, or a = 0
-    const double rest = (s2 - (t0 - a)) + __builtin_fma(de, kLn2Lo, __builtin_fma(s2 * w, p, sl + sl));
-    const double t = t0 + rest;
-    const double tl = rest - (t - t0);
-    return __builtin_fma(kHi, t, __builtin_fma(kHi, tl, kLo * t));
+    const double de = (double)e, a = de * kExpHi, h = kHi * sv;
+    const double t = a + h;  // |a| > |h|, or a = 0
+    double rest = __builtin_fma(kLo, sv, __builtin_fma(kHi, sv, -h));
+    rest = __builtin_fma(de, kExpLo, __builtin_fma(kHi, sl, rest));
+    rest = __builtin_fma(h * w, p, rest);
+    return t + ((h - (t - a)) + rest);
 }
 
 // ln(1 + a) in FP64 for finite a > -1, within a few units in the last place also for small |a|:

@@ -323,17 +323,17 @@ __device__ __forceinline__ void grad_sis_circ(const HaloRec& h, double px, doubl
 // At the halo centre itself the reference's potential is 0/0 (NaN); this form gives its limit 0 there,
 // so the kernels track the smallest rem^2 of a pixel over its PIEMD halos and return NaN when it is 0.
 struct PotRad {
-    double w, d, R, lq;  // w, w - r, Re Q, ln(|Q|^2 / (c r)^2)
+    double q, iw, d, R, lq;  // w^2, 1 / w, w - r, Re Q, ln(|Q|^2 / (c r)^2)
 };
 
 template <bool FULL>
 __device__ __forceinline__ PotRad pot_rad(const HaloRec& h, double rem2, double I2, double r, double r2, double cr,
                                           double icr2)
 {
-    const double q = r2 + rem2;
     PotRad o;
-    o.w = q * rsq_c<FULL>(q);
-    o.d = rem2 * rcp_c<FULL>(o.w + r);
+    o.q = r2 + rem2;
+    o.iw = rsq_c<FULL>(o.q);
+    o.d = rem2 * rcp_c<FULL>(__builtin_fma(o.q, o.iw, r));
     const double cd = h.cx1 * o.d;
     o.R = cd + cr;
     o.lq = log1p_lt(__builtin_fma(cd, __builtin_fma(2., cr, cd), I2) * icr2);
@@ -357,7 +357,7 @@ __device__ __forceinline__ double pot_piemd(const HaloRec& h, const PixelFrame& 
         return __builtin_fma(f.x, arg, __builtin_fma(f.y, ay, -(h.psra * a.lq)));
     }
     const PotRad b = pot_rad<FULL>(h, rem2, I2, h.rcut, h.rb2, h.pcrb, h.picrb2);
-    const double sig = (a.d + b.d) * rcp_c<FULL>(a.w + b.w);
+    const double sig = (a.d + b.d) * rcp_c<FULL>(__builtin_fma(a.q, a.iw, b.q * b.iw));
     const double dR = h.pdr * __builtin_fma(-h.cx1, sig, h.pc);
     const double arg = atan2p_lt(I * dR, __builtin_fma(a.R, b.R, I2));
     const double Q2a = __builtin_fma(a.R, a.R, I2);
@@ -398,7 +398,8 @@ __device__ __forceinline__ void eigen(double A, double B, double C, double& lam,
 // -2.5 log10(x), x >= 0: the library's log10 for zero, infinity, NaN and the largest and smallest numbers
 __device__ __forceinline__ double magnitudes(double x)
 {
-    if (x >= 0x1p-1000 && x <= 0x1p1000) return magnitudes_lt(x);
+    // 2^-1000 <= x < 2^1000 by the upper word
+    if ((uint32_t)__double2hiint(x) - 0x01700000u < 0x7d000000u) return magnitudes_lt(x);
     return -2.5 * log10(x);
 }
 
@@ -414,7 +415,7 @@ __device__ __forceinline__ void hess_epilogue(const OutDesc& o, int64_t idx, dou
         if (o.p3) o.p3[idx] = b;
     } else if constexpr (KIND == LT_MAP_FIELDS) {
         double kappa = 0.5 * T * r, g1 = 0.5 * D * r, g2 = B * r;
-        double omk = __builtin_fma(-0.5 * T, r, 1.);
+        double omk = 1. - kappa;
         double det = __builtin_fma(omk, omk, -__builtin_fma(g1, g1, g2 * g2));
         if (o.p0) o.p0[idx] = kappa;
         if (o.p1) o.p1[idx] = g1;
@@ -428,7 +429,7 @@ __device__ __forceinline__ void hess_epilogue(const OutDesc& o, int64_t idx, dou
         double v;
         if (o.mode <= 3) {
             // det A, the product of the eigenvalues of 1 - r H, without their square root
-            const double omk = __builtin_fma(-0.5 * T, r, 1.), g1 = 0.5 * D * r, g2 = B * r;
+            const double omk = 1. - 0.5 * T * r, g1 = 0.5 * D * r, g2 = B * r;
             const double det = __builtin_fma(omk, omk, -__builtin_fma(g1, g1, g2 * g2));
             if (o.mode == 1) v = 1. / det;
             else if (o.mode == 2) v = 1. / fabs(det);
