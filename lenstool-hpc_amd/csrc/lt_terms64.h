@@ -336,7 +336,7 @@ __device__ __forceinline__ PotRad pot_rad(const HaloRec& h, double rem2, double 
     o.d = rem2 * rcp_c<FULL>(__builtin_fma(o.q, o.iw, r));
     const double cd = h.cx1 * o.d;
     o.R = cd + cr;
-    o.lq = log1p_lt(__builtin_fma(cd, __builtin_fma(2., cr, cd), I2) * icr2);
+    o.lq = log1p_mul_lt(__builtin_fma(cd, __builtin_fma(2., cr, cd), I2), icr2);
     return o;
 }
 
@@ -348,10 +348,9 @@ __device__ __forceinline__ double pot_piemd(const HaloRec& h, const PixelFrame& 
     mn = min64(mn, rem2);
     const double I = h.gki * f.x;
     const double I2 = I * I;
-    const double v = h.gkv * f.y;
     const PotRad a = pot_rad<FULL>(h, rem2, I2, h.rc, h.ra2, h.pcra, h.picra2);
     if (!CUT) {
-        const double ls = log1p_lt((a.d + v) * h.picra);
+        const double ls = log1p_mul_lt(__builtin_fma(h.gkv, f.y, a.d), h.picra);
         const double arg = atan2p_lt(I, a.R);
         const double ay = __builtin_fma(-0.5, a.lq, ls);
         return __builtin_fma(f.x, arg, __builtin_fma(f.y, ay, -(h.psra * a.lq)));
@@ -361,12 +360,13 @@ __device__ __forceinline__ double pot_piemd(const HaloRec& h, const PixelFrame& 
     const double dR = h.pdr * __builtin_fma(-h.cx1, sig, h.pc);
     const double arg = atan2p_lt(I * dR, __builtin_fma(a.R, b.R, I2));
     const double Q2a = __builtin_fma(a.R, a.R, I2);
+    const double v = h.gkv * f.y;
     const double Sa = (h.pcra + a.d) + v, Sb = (h.pcrb + b.d) + v;
     const double ga = __builtin_fma(h.pomc, a.d, v);
     const double Pa = __builtin_fma(ga, Sa + a.R, -I2);
     const double dP = __builtin_fma(Sb + b.R, h.pomcdr * sig, -(ga * (h.pcdr * (2. - sig))));
     const double N = __builtin_fma(Pa, dR * (a.R + b.R), Q2a * dP);
-    const double ay = 0.5 * log1p_lt(N * rcp_c<FULL>((Sb * Sb) * Q2a));
+    const double ay = 0.5 * log1p_mul_lt(N, rcp_c<FULL>((Sb * Sb) * Q2a));
     const double L = __builtin_fma(h.psra, a.lq, -(h.psrb * b.lq));
     return __builtin_fma(f.x, arg, __builtin_fma(f.y, ay, -L));
 }
