@@ -17,7 +17,7 @@
  *
  * precision: LT_PREC_FP64 or LT_PREC_FP32C (lt_status.h). FP32C (FP32 halo terms with FP64 offsets
  * and FP64 chunk sums; FP64 terms next to the cores for the Hessian, gradient and displacement) applies
- * to every map kind.
+ * to every map kind that is summed at its pixels; maps summed in tiles (LT_FORM_TILES_*) are FP64 in both.
  */
 #ifndef LENSTOOL_HIP_LT_CAPI_H
 #define LENSTOOL_HIP_LT_CAPI_H
@@ -170,10 +170,12 @@ int lt_map_device(lt_model model, int kind, int mode, double* out0, double* out1
 
 /* The form in which lt_map_device sums the map of `sample` of the model: from its types, halo count and run
  * structure, the sample's own parameters and the grid, by estimated time. Maps of one lens in one form
- * are equal bit for bit, in a batch or alone, updated or new; forms differ by rounding. The LT_FORM_TILES forms
- * sum halos far from a tile of pixels at nodes of the tile, in FP64 also where FP32C is asked for; models of more than
- * 2048 halos or 16 runs (of equal type, and dlsds for LT_MAP_MASS) do not take them. A captured launch
- * sequence keeps the form of its capture: its replays with parameters staged later are maps of that form. */
+ * are equal bit for bit, in a batch or alone, updated or new; forms differ by rounding (FP32C maps, of which only
+ * the tiles are FP64 sums, by the FP32C error), as may a part of a map that is asked for as a grid of its own. The
+ * LT_FORM_TILES forms sum halos far from a tile of pixels at nodes of the tile, in FP64 also where FP32C is asked
+ * for; models of more than 2048 halos or 16 runs (of equal type, and dlsds for LT_MAP_MASS) do not take them, nor
+ * maps whose larger pixel step lies outside [1e-15, 1e15]. A captured launch sequence keeps the form of its
+ * capture: its replays with parameters staged later are maps of that form. */
 #define LT_FORM_PIXELS            0 /* every halo at every pixel                                           */
 #define LT_FORM_PARTS             1 /* the same in eight parts of the halos (small maps)                   */
 #define LT_FORM_TILES_64          2 /* tiles of 64 pixels, four waves                                      */

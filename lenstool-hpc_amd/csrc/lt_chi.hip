@@ -261,8 +261,8 @@ int batch_run(lt_chi_batch_s* b, const lt_potential_soa* lenses, double* chi, in
         o.p0 = b->gx + (size_t)c0 * g.plane_stride;
         o.p1 = b->gy + (size_t)c0 * g.plane_stride;
         // 4 pixels per thread: with few halos per sample each halo record's scalar load is shared by
-        // more pixels (1024 samples of 11 halos on 512^2: 9.9 ms per batch step against 10.4 at 2; the
-        // planes are bit-identical for every pixels-per-thread)
+        // more pixels (1024 samples of 11 halos on 512^2: 5.75 ms a step, 5.98 at 2; one sample 81 us, 83 at 2,
+        // within its noise; the planes are bit-identical for every pixels-per-thread)
         LT_HIP_TRY(launch_gradient64(b->recs + (size_t)c0 * b->H, b->druns, (int)b->runs.size(), g, o, 4, s));
     }
     LT_HIP_TRY(launch_points_gradient64(b->recs, b->druns, (int)b->runs.size(), b->d.img_x, b->d.img_y, b->nimg,

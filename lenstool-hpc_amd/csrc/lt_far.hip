@@ -324,9 +324,10 @@ __device__ __forceinline__ void store4(double* p, int lane, const d4& v)
 
 // Bound by the FP64 pipes: VALU issue (70 % of the cycles on the 503-halo 4096^2 fields, 88 % on the 2048^2 potential) and,
 // for light models, matrix instructions beside it (38 % and 26 % on 256 maps of 11 halos). Work-groups of 4 waves are held to
-// three waves a SIMD (168 registers): 256 maps of 2048^2 in 7.1 ms, 8.7 with two, 8.8 with four, which spills. The
-// logarithm's and arctangent's coefficients stay in scalar registers, 36 vector registers less: the potential
-// 2048^2, 503 halos, 825 -> 800 us, displacement 701 x 643, 160 mixed halos, 152 -> 146.
+// three waves a SIMD (168 registers): 256 magnitude maps of 2048^2 in 7.1 ms, 8.7 with two, 8.8 with four, which spills
+// (7.3 with the logarithm that carries its remainders). The logarithm's and arctangent's coefficients stay in scalar
+// registers, 36 vector registers less: the potential 2048^2, 503 halos, roots of 128, 825 -> 800 us (770 with the
+// logarithm's product unrounded), displacement 701 x 643, 160 mixed halos, 152 -> 146.
 // PARTS 2 and 4: the halves or the subs of a root go to a work-group each, all of which sum its nodes: a map of fewer than
 // 128 roots would leave the other CUs idle (displacement 701 x 643, 160 mixed halos, 121 roots: 147 us, halved 87).
 template <int FAM, int KIND, int LV, int UNIT, int PARTS>
@@ -629,16 +630,17 @@ static unsigned tiles_over(int start, int n, int side);
 // Tile expansions cost, per pixel, the halos near its 32-pixel square, 256 nodes over the area of a square for each
 // halo first expanded there, and the expansion itself (72 matrix instructions per 1024 pixels and three fields,
 // in VALU issue slots). From that count and the number of work-groups follows a time in cycles of a CU (four
-// instructions a cycle and 64 lanes), with the efficiencies and fixed shares that were measured: a root of 64 pixels takes 1.15 times its
-// count and about 100 000 cycles beside it (its barriers and the longest wave), a half or a quarter of one 1.25 and 1.5 times
-// its share, the root's nodes included, and about half as much. Over 176 maps (20 to 1000 halos, four kinds, 240^2 to 2100^2)
+// instructions a cycle and 64 lanes), with the efficiencies and fixed shares that were measured: a root of 64 pixels
+// takes 1.15 times its count and about 100 000 cycles beside it (its barriers and the longest wave), a half or a
+// quarter of one 1.25 and 1.5 times its share, the root's nodes included, and about half as much. Over 176 maps (20 to 1000 halos, four kinds, 240^2 to 2100^2)
 // the shape taken is 2 % behind the best of the six in the mean. Some of them, us (direct, 4 waves, 16, halves, quarters):
 //   dpl 672 x 635, 160 mixed halos: 233, 174, 158, 100; fields 450 x 413, 258 dPIE: 129, 214, 174, 110;
 //   potential 450 x 413, 1000 dPIE: 1638, 2409, 2262, 1300; fields 900 x 863, 258: 498, 118, 101, 121.
 //   light models (1 dPIE + 10 SIS): 256 maps of 2048^2 in 7.1 ms with 4 waves, 17.6 with 16.
 //   503 halos, 4096^2: root 128 565 us, root 64 1145; 2000 on 8192^2: root 256 2.6 ms, root 128 5.3.
-// Where roots of 128 pixels halve the count of 64 with these shares added (fine pixels, many halos), the shape depends on the steps and the model alone,
-// so that a part of a map takes the same form as the whole; roots of 256 again have to halve the count of 128: their
+// Where roots of 128 pixels halve the count of 64 with these shares added (fine pixels, many halos), the shape depends on
+// the steps and the lens alone, so that a part of a map takes the same form as the whole; roots of 256 again have to halve
+// the count of 128: their
 // work-groups are few and uneven (a 300 x 200 part of the 4096^2 map: 271 us, 111 with 128, 183 directly).
 // Elsewhere the quickest shape is taken, or the direct sum.
 FarShape far_shape(const FarStats& st, double density, int kind, int precision, const GridDesc& g, double* cost)

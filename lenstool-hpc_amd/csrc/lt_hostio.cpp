@@ -4,8 +4,9 @@
 // of 90 MB of such planes took 6.6 ms, 37 times the kernel before it. Here the device writes pieces into a pinned area
 // and four threads move them on, page faults included, while the next pieces arrive (2.3 ms); up to one piece a single
 // thread does the same without starting others. With one image of the inputs in pinned memory, one copy of the results
-// and buffers that stay, a likelihood evaluation on 512 x 512 pixels takes 87 us (335 with its own allocations and nine
-// copies), 20000 point gradients of 503 halos 146 (192). What stays is bounded (64 MB of scratch, 16 MB pinned, the
+// and buffers that stay, a likelihood evaluation on 512 x 512 pixels takes 80-89 us (335 with its own allocations and
+// nine copies), 20000 point gradients of 503 halos 145-148 (192). Where the area cannot be had the calls copy from and to
+// pageable memory. What stays is bounded (64 MB of scratch, 16 MB pinned, the
 // planes of the largest map call) and given back when an allocation would fail.
 #include "lt_hostio.h"
 

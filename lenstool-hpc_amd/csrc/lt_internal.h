@@ -23,7 +23,8 @@ int critic_noalloc_setup(int dev, void** ptr);
 // lt_map_device of `grid`, a part of the map `whole`, by the kernel that the whole map takes
 int map_device_rows(lt_model m, int kind, int mode, double* const outs[5], double r, double mult,
                     const lt_grid_desc* grid, const lt_grid_desc* whole, int precision, int px, void* stream);
-// estimated instructions per pixel of that map, and whether it is computed in tiles of 64 or 128 rows
+// estimated instructions per pixel of that map, and whether it is computed by tile expansions (tiles of 64,
+// 128 or 256 rows)
 double map_rows_cost(lt_model m, int kind, int precision, const lt_grid_desc* whole, bool* tiled);
 
 }  // namespace lt
