@@ -280,8 +280,8 @@ __device__ __forceinline__ void run32(const HaloRec* __restrict__ h64, const Hal
     }
 }
 
-// The FP64 Hessian sums of one pixel over every run, exactly as the FP64 kernel forms them (same
-// terms, same order): the fallback for pixels where det A would amplify the FP32 rounding.
+// The FP64 Hessian sums of one pixel over every run, exactly as the FP64 kernel forms them for LT_FORM_PIXELS
+// (same terms, same order; maps summed in parts differ from it by rounding): the fallback for pixels where det A would amplify the FP32 rounding.
 __device__ __forceinline__ void hessian_fp64_pixel(const HaloRec* __restrict__ h64, const Run* __restrict__ runs,
                                                 int nruns, double px, double py, double& tT, double& tD, double& tB)
 {
