@@ -175,7 +175,8 @@ int lt_map_device(lt_model model, int kind, int mode, double* out0, double* out1
  * LT_FORM_TILES forms sum halos far from a tile of pixels at nodes of the tile, in FP64 also where FP32C is asked
  * for; models of more than 2048 halos or 16 runs (of equal type, and dlsds for LT_MAP_MASS) do not take them, nor
  * maps whose larger pixel step lies outside [1e-15, 1e15]. A captured launch sequence keeps the form of its
- * capture: its replays with parameters staged later are maps of that form. */
+ * capture: its replays with parameters staged later are maps of that form; other maps go by the samples on the
+ * device, which a launch of a sequence that holds the model's upload replaces by those staged last. */
 #define LT_FORM_PIXELS            0 /* every halo at every pixel                                           */
 #define LT_FORM_PARTS             1 /* the same in eight parts of the halos (small maps)                   */
 #define LT_FORM_TILES_64          2 /* tiles of 64 pixels, four waves                                      */

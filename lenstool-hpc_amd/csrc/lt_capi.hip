@@ -633,6 +633,50 @@ int lt_map_fields(double* kappa, double* gamma1, double* gamma2, double* det_a, 
 // ---- resident models ------------------------------------------------------------------------------
 }  // extern "C"
 
+// What the forms of a model's maps go by, in parts that maps, uploads and launches of captured sequences exchange as a whole
+// (std::atomic_load, atomic_store), whatever another thread stages or uploads meanwhile: for the samples on the device, for
+// those in `staging`, and for maps captured after a captured upload, which come after it in each replay.
+struct ModelForms {
+    struct Captured {
+        unsigned long long id;  // of the capture
+        std::shared_ptr<const LensStats> stats;
+    };
+    std::shared_ptr<const LensStats> device, staged;
+    std::shared_ptr<const Captured> captured;
+};
+
+// The sequences being captured (lt_graph_begin to lt_graph_end) and the models whose uploads they hold. A replay puts on
+// the device what is staged then. (A capture begun by the caller's own means is not known here: its
+// upload counts from the call on.)
+struct Capture {
+    hipStream_t stream;
+    unsigned long long id;
+    std::vector<std::shared_ptr<ModelForms>> uploads;
+};
+static std::mutex g_captures_mu;
+static std::vector<Capture> g_captures;
+
+// whether s is being captured, and the capture's number
+static bool capture_of(hipStream_t s, unsigned long long* id)
+{
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return s && hipStreamGetCaptureInfo(s, &cs, id) == hipSuccess && cs == hipStreamCaptureStatusActive;
+}
+
+// the sequence that s is being captured for, taken off the list
+static Capture take_capture(hipStream_t s)
+{
+    std::lock_guard<std::mutex> lock(g_captures_mu);
+    Capture c{s, 0, {}};
+    for (size_t i = 0; i < g_captures.size(); ++i)
+        if (g_captures[i].stream == s) {
+            c = std::move(g_captures[i]);
+            g_captures.erase(g_captures.begin() + i);
+            break;
+        }
+    return c;
+}
+
 struct lt_model_s {
     int device = 0;
     Use use = Use::Hessian;
@@ -641,9 +685,7 @@ struct lt_model_s {
     std::vector<Run> runs_host;
     std::vector<int> types;
     DevModel dm;
-    // of the samples on the device, and of those in `staging`; a map takes `stats` as it finds it, whatever another
-    // thread stages or uploads meanwhile
-    std::shared_ptr<const LensStats> stats, staged_stats;
+    const std::shared_ptr<ModelForms> forms = std::make_shared<ModelForms>();
     size_t bytes = 0;
     size_t rec_bytes = 0, rec32_bytes = 0;  // all samples
     void* base = nullptr;                   // device: records [S*H], fp32 records [S*H], far records [S*H], runs
@@ -712,7 +754,7 @@ static int stage_samples(lt_model_s* m, const lt_potential_soa* lenses, int nsam
         stats->density[s] = halo_density(recs.data(), runs);
     }
     stats->far = far_stats(H, batch_runs);
-    m->staged_stats = stats;
+    std::atomic_store(&m->forms->staged, std::shared_ptr<const LensStats>(std::move(stats)));
     if (!batch_runs.empty()) std::memcpy(st + m->off_runs, batch_runs.data(), batch_runs.size() * sizeof(Run));
     return LT_OK;
 }
@@ -723,9 +765,20 @@ static int upload_staged(lt_model_s* m, hipStream_t s)
     const size_t n = m->off_runs + m->runs_host.size() * sizeof(Run);
     if (!n) return LT_OK;
     HIP_TRY(hipMemcpyAsync(m->base, m->staging, n, hipMemcpyHostToDevice, s));
-    std::atomic_store(&m->stats, m->staged_stats);
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing(s, &cs));
+    const auto staged = std::atomic_load(&m->forms->staged);
+    unsigned long long id = 0;
+    if (cs != hipStreamCaptureStatusNone && capture_of(s, &id)) {
+        std::lock_guard<std::mutex> lock(g_captures_mu);
+        for (Capture& c : g_captures)
+            if (c.id == id) {
+                c.uploads.push_back(m->forms);
+                std::atomic_store(&m->forms->captured, std::make_shared<const ModelForms::Captured>(ModelForms::Captured{id, staged}));
+                return LT_OK;
+            }
+    }
+    std::atomic_store(&m->forms->device, staged);
     if (cs == hipStreamCaptureStatusNone) {
         HIP_TRY(hipEventRecord(m->staged, s));
         m->staged_pending = true;
@@ -792,7 +845,7 @@ int lt_model_create_batch(lt_model* out, const lt_potential_soa* lenses, int nsa
         free_model(m);
         return st;
     }
-    m->stats = m->staged_stats;
+    m->forms->device = m->forms->staged;
     e = hipMemcpy(m->base, m->staging, off_runs + runs.size() * sizeof(Run), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         free_model(m);
@@ -874,10 +927,19 @@ static GridDesc grid_desc(const lt_model_s* m, const lt_grid_desc* grid)
     return g;
 }
 
+// what the form of a map launched on s goes by
+static std::shared_ptr<const LensStats> map_stats(const lt_model_s* m, hipStream_t s)
+{
+    unsigned long long id = 0;
+    const auto c = std::atomic_load(&m->forms->captured);
+    if (c && capture_of(s, &id) && c->id == id) return c->stats;
+    return std::atomic_load(&m->forms->device);
+}
+
 double lt::map_rows_cost(lt_model m, int kind, int precision, const lt_grid_desc* whole, bool* tiled)
 {
     double cost = 0;
-    const auto stats = std::atomic_load(&m->stats);
+    const auto stats = std::atomic_load(&m->forms->device);
     *tiled = far_shape(stats->far, stats->density[0], kind, precision, grid_desc(m, whole), &cost) != FarShape::Direct;
     return cost;
 }
@@ -905,8 +967,8 @@ int lt::map_device_rows(lt_model m, int kind, int mode, double* const outs[5], d
         return fail(LT_ERR_INVALID, "gradient output needs two planes");
     if (kind != LT_MAP_HESSIAN && kind != LT_MAP_FIELDS && !outs[0]) return fail(LT_ERR_INVALID, "out0 is NULL");
     HIP_TRY(hipSetDevice(m->device));
-    return launch_map(m->dm, *std::atomic_load(&m->stats), kind, mode, outs, r, mult, grid_desc(m, grid), grid_desc(m, whole), precision, px,
-                      (hipStream_t)stream, m->nhalos);
+    return launch_map(m->dm, *map_stats(m, (hipStream_t)stream), kind, mode, outs, r, mult, grid_desc(m, grid),
+                      grid_desc(m, whole), precision, px, (hipStream_t)stream, m->nhalos);
 }
 
 extern "C" {
@@ -927,7 +989,7 @@ int lt_map_form(lt_model m, int sample, int kind, const lt_grid_desc* grid, int 
     int st;
     if ((st = check_use(m, kind)) || (st = check_launch(kind, precision, px))) return st;
     if (grid->nx <= 0 || grid->ny <= 0 || grid->pitch < grid->nx) return fail(LT_ERR_INVALID, "bad grid");
-    const auto stats = std::atomic_load(&m->stats);
+    const auto stats = std::atomic_load(&m->forms->device);
     const Form f = map_form(stats->far, stats->density[sample], kind, precision, grid_desc(m, grid), px);
     switch (f.shape) {
     case FarShape::Root64: *form = LT_FORM_TILES_64; break;
@@ -1008,7 +1070,7 @@ int lt_autotune(lt_model m, int kind, int mode, const lt_grid_desc* grid, int pr
     const int cand[3] = {1, 2, 4};
     // a map in another form than every halo at every pixel has no pixels per thread to choose: one timing, and the
     // default stays
-    const auto stats = std::atomic_load(&m->stats);
+    const auto stats = std::atomic_load(&m->forms->device);
     const GridDesc gd = grid_desc(m, &g);
     bool tuned = false;
     for (double density : stats->density) {
@@ -1057,12 +1119,19 @@ struct lt_graph_s {
     int device = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
+    std::vector<std::shared_ptr<ModelForms>> uploads;  // of the models whose upload it holds
 };
 
 int lt_graph_begin(void* stream)
 {
     if (!stream) return fail(LT_ERR_INVALID, "capture needs a caller stream (not the NULL stream)");
     HIP_TRY(hipStreamBeginCapture((hipStream_t)stream, hipStreamCaptureModeThreadLocal));
+    (void)take_capture((hipStream_t)stream);  // of a capture that the caller ended otherwise
+    Capture c{(hipStream_t)stream, 0, {}};
+    if (capture_of(c.stream, &c.id)) {
+        std::lock_guard<std::mutex> lock(g_captures_mu);
+        g_captures.push_back(std::move(c));
+    }
     return LT_OK;
 }
 
@@ -1074,6 +1143,11 @@ int lt_graph_end(void* stream, lt_graph* out)
     int dev, st;
     if ((st = current_device(&dev))) return st;
     hipGraph_t g = nullptr;
+    Capture c = take_capture((hipStream_t)stream);
+    for (const auto& f : c.uploads) {
+        const auto captured = std::atomic_load(&f->captured);
+        if (captured && captured->id == c.id) std::atomic_store(&f->captured, std::shared_ptr<const ModelForms::Captured>());
+    }
     HIP_TRY(hipStreamEndCapture((hipStream_t)stream, &g));
     hipGraphExec_t x = nullptr;
     hipError_t e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
@@ -1085,6 +1159,7 @@ int lt_graph_end(void* stream, lt_graph* out)
     r->device = dev;
     r->graph = g;
     r->exec = x;
+    r->uploads = std::move(c.uploads);
     *out = r;
     return LT_OK;
 }
@@ -1094,6 +1169,7 @@ int lt_graph_launch(lt_graph g, void* stream)
     if (!g) return fail(LT_ERR_NOT_FOUND, "graph is NULL");
     HIP_TRY(hipSetDevice(g->device));
     HIP_TRY(hipGraphLaunch(g->exec, (hipStream_t)stream));
+    for (const auto& f : g->uploads) std::atomic_store(&f->device, std::atomic_load(&f->staged));
     return LT_OK;
 }
 
