@@ -158,7 +158,7 @@ __device__ __forceinline__ Q32 q_term(const HaloRec32& h, const QShared& s, floa
     const float W2 = s.wq0 + r2c;
     const float iW = rsq32(W2);
     const float W = W2 * iW;
-    const float Qr = W + r;
+    const float Qr = __builtin_fmaf(W2, iW, r);
     const float U = __builtin_fmaf(s.Y, iW, h.k5);
     Q32 o;
     o.dd = -__builtin_fmaf(s.A, iW, U * __builtin_fmaf(h.k3, W, -s.ky4));
@@ -198,7 +198,7 @@ __device__ __forceinline__ void hess_sis32(const HaloRec32& h, const Frame32& f,
     const float x2 = f.x * f.x, y2 = f.y * f.y;
     const float iR = rsq32(__builtin_fmaf(h.sa, x2, h.sb * y2));
     const float g = iR * iR * iR;
-    acc_lab(h, g * (x2 + y2), g * (y2 - x2), -(g * f.x * f.y), fT, fD, fB);
+    acc_lab(h, g * __builtin_fmaf(f.x, f.x, y2), g * __builtin_fmaf(-f.x, f.x, y2), -(g * f.x * f.y), fT, fD, fB);
 }
 
 // circular SIS (a run of them): the lab-frame offsets tx, ty give the Hessian directly (hT = b0)
@@ -526,7 +526,7 @@ __device__ __forceinline__ void add_term32(const HaloRec32& h, const Seg32& s, f
         const float x2 = X * X, y2 = Y * Y;
         const float iR = rsq32(__builtin_fmaf(h.sa, x2, h.sb * y2));
         const float g = far ? iR * iR * iR : 0.f;
-        acc_lab(h, g * (x2 + y2), g * (y2 - x2), -(g * X * Y), aT, aD, aB);
+        acc_lab(h, g * __builtin_fmaf(X, X, y2), g * __builtin_fmaf(-X, X, y2), -(g * X * Y), aT, aD, aB);
     } else {
         const QShared q = q_shared(h, X, Y);
         const Q32 a = q_term(h, q, h.ra, h.ra2c);

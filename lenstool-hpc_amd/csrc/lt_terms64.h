@@ -109,7 +109,7 @@ __device__ __forceinline__ PiemdQ piemd_q_term(const HaloRec& h, const PiemdShar
     const double W2 = s.wq0 + r2c;
     const double iW = rsq_c<FULL>(W2);
     const double W = W2 * iW;
-    const double Qr = W + r;
+    const double Qr = __builtin_fma(W2, iW, r);
     const double U = __builtin_fma(s.Y, iW, h.k5);
     PiemdQ o;
     o.dd = -__builtin_fma(s.A, iW, U * __builtin_fma(h.k3, W, -s.ky4));
@@ -163,9 +163,9 @@ __device__ __forceinline__ void hess_sis_at(const HaloRec& h, double tx, double 
     double R2 = __builtin_fma(h.sa, f.x2, h.sb * f.y2);
     double iR = rsq_c<FULL>(R2);
     double g = iR * iR * iR;
-    double dyx = f.y2 - f.x2;
+    double dyx = __builtin_fma(-f.x, f.x, f.y2);
     double xy = f.x * f.y;
-    aT = __builtin_fma(g * h.amph, f.x2 + f.y2, aT);
+    aT = __builtin_fma(g * h.amph, __builtin_fma(f.x, f.x, f.y2), aT);
     aD = __builtin_fma(g, __builtin_fma(h.hc2, dyx, 2.0 * h.hs2 * xy), aD);
     aB = __builtin_fma(g, __builtin_fma(0.5 * h.hs2, dyx, -(h.hc2 * xy)), aB);
 }
@@ -177,23 +177,29 @@ __device__ __forceinline__ void hess_sis(const HaloRec& h, double px, double py,
 }
 
 // Circular SIS (e = 0): the Hessian b0/r^3 (y^2, -xy, x^2) holds in any frame, so it is formed from
-// the lab-frame offsets, with no rotation to the halo frame and back (T = b0 / r).
+// the lab-frame offsets, with no rotation to the halo frame and back (T = b0 / r). The square that is formed is that of the
+// offset which a lane's pixels share: the row's ty here, the column's tx in `_at` (lt_far.hip).
 template <bool FULL>
 __device__ __forceinline__ void hess_sis_circ_at(const HaloRec& h, double tx, double ty, double& aT, double& aD,
                                                  double& aB)
 {
-    const double y2 = ty * ty;
-    const double iR = rsq_c<FULL>(__builtin_fma(tx, tx, y2));
+    const double x2 = tx * tx;
+    const double iR = rsq_c<FULL>(__builtin_fma(ty, ty, x2));
     const double ga = h.amph * (iR * iR * iR);
     aT = __builtin_fma(h.amph, iR, aT);
-    aD = __builtin_fma(ga, __builtin_fma(-tx, tx, y2), aD);
+    aD = __builtin_fma(ga, __builtin_fma(ty, ty, -x2), aD);
     aB = __builtin_fma(-ga, tx * ty, aB);
 }
 
 __device__ __forceinline__ void hess_sis_circ(const HaloRec& h, double px, double py, double& aT, double& aD,
                                               double& aB)
 {
-    hess_sis_circ_at<false>(h, px - h.xh, py - h.yh, aT, aD, aB);
+    const double tx = px - h.xh, ty = py - h.yh, y2 = ty * ty;
+    const double iR = rsq64_n2(__builtin_fma(tx, tx, y2));
+    const double ga = h.amph * (iR * iR * iR);
+    aT = __builtin_fma(h.amph, iR, aT);
+    aD = __builtin_fma(ga, __builtin_fma(-tx, tx, y2), aD);
+    aB = __builtin_fma(-ga, tx * ty, aB);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -218,11 +224,11 @@ __device__ __forceinline__ QS64 qs64(const HaloRec& h, double rem2, double I2, d
                                      double rcx)
 {
     const double q = r2 + rem2;
-    const double w = q * rsq_c<FULL>(q);
+    const double iw = rsq_c<FULL>(q);
     QS64 o;
-    o.R = __builtin_fma(h.cx1, w, r);
+    o.R = __builtin_fma(h.cx1, q * iw, r);
     o.Q2 = __builtin_fma(o.R, o.R, I2);
-    o.S = __builtin_fma(h.gkv, y, w + rcx);
+    o.S = __builtin_fma(h.gkv, y, __builtin_fma(q, iw, rcx));
     return o;
 }
 
@@ -279,14 +285,17 @@ __device__ __forceinline__ void grad_sis(const HaloRec& h, double px, double py,
 // Circular SIS: b0 (x, y) / r in any frame, formed from the lab-frame offsets.
 __device__ __forceinline__ void grad_sis_circ_at(const HaloRec& h, double tx, double ty, double& gx, double& gy)
 {
-    const double s = h.ampg * rsq64(__builtin_fma(tx, tx, ty * ty));
+    const double s = h.ampg * rsq64(__builtin_fma(ty, ty, tx * tx));
     gx = __builtin_fma(s, tx, gx);
     gy = __builtin_fma(s, ty, gy);
 }
 
 __device__ __forceinline__ void grad_sis_circ(const HaloRec& h, double px, double py, double& gx, double& gy)
 {
-    grad_sis_circ_at(h, px - h.xh, py - h.yh, gx, gy);
+    const double tx = px - h.xh, ty = py - h.yh;
+    const double s = h.ampg * rsq64(__builtin_fma(tx, tx, ty * ty));
+    gx = __builtin_fma(s, tx, gx);
+    gy = __builtin_fma(s, ty, gy);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -335,7 +344,7 @@ __device__ __forceinline__ PotRad pot_rad(const HaloRec& h, double rem2, double 
     o.iw = rsq_c<FULL>(o.q);
     o.d = rem2 * rcp_c<FULL>(__builtin_fma(o.q, o.iw, r));
     const double cd = h.cx1 * o.d;
-    o.R = cd + cr;
+    o.R = __builtin_fma(h.cx1, o.d, cr);
     o.lq = log1p_mul_lt(__builtin_fma(cd, __builtin_fma(2., cr, cd), I2), icr2);
     return o;
 }
@@ -361,7 +370,7 @@ __device__ __forceinline__ double pot_piemd(const HaloRec& h, const PixelFrame& 
     const double arg = atan2p_lt(I * dR, __builtin_fma(a.R, b.R, I2));
     const double Q2a = __builtin_fma(a.R, a.R, I2);
     const double v = h.gkv * f.y;
-    const double Sa = (h.pcra + a.d) + v, Sb = (h.pcrb + b.d) + v;
+    const double Sa = __builtin_fma(h.gkv, f.y, h.pcra + a.d), Sb = __builtin_fma(h.gkv, f.y, h.pcrb + b.d);
     const double ga = __builtin_fma(h.pomc, a.d, v);
     const double Pa = __builtin_fma(ga, Sa + a.R, -I2);
     const double dP = __builtin_fma(Sb + b.R, h.pomcdr * sig, -(ga * (h.pcdr * (2. - sig))));
