@@ -326,8 +326,8 @@ __device__ __forceinline__ void store4(double* p, int lane, const d4& v)
 // for light models, matrix instructions beside it (38 % and 26 % on 256 maps of 11 halos). Work-groups of 4 waves are held to
 // three waves a SIMD (168 registers): 256 magnitude maps of 2048^2 in 7.1 ms, 8.7 with two, 8.8 with four, which spills
 // (7.3 with the logarithm that carries its remainders). The logarithm's and arctangent's coefficients stay in scalar
-// registers, 36 vector registers less: the potential 2048^2, 503 halos, roots of 128, 825 -> 800 us (770 with the
-// logarithm's product unrounded), displacement 701 x 643, 160 mixed halos, 152 -> 146.
+// registers, 36 vector registers less: the potential 2048^2, 503 halos, roots of 128, 825 -> 800 us, displacement
+// 701 x 643, 160 mixed halos, 152 -> 146.
 // PARTS 2 and 4: the halves or the subs of a root go to a work-group each, all of which sum its nodes: a map of fewer than
 // 128 roots would leave the other CUs idle (displacement 701 x 643, 160 mixed halos, 121 roots: 147 us, halved 87).
 template <int FAM, int KIND, int LV, int UNIT, int PARTS>
